@@ -33,9 +33,9 @@ METRIC = "Mrays/s + LBVH Mtri/s; s/frame to relMSE≤0.01: learned vs plain, 1 G
 HBM_PEAK_GBS = 8000.0
 
 # Algorithmic bytes of the walk (one ray): the ray in (32), the hit out (8),
-# the root node (32), both children at every inner step (2 x 32), one
+# the root node (32), four boxes and their words at every visit (7 x 16), one
 # triangle record per test (48: three corners in 16-byte rows).
-RAY_BYTES, HIT_BYTES, ROOT_BYTES, STEP_BYTES, TEST_BYTES = 32, 8, 32, 64, 48
+RAY_BYTES, HIT_BYTES, ROOT_BYTES, STEP_BYTES, TEST_BYTES = 32, 8, 32, 112, 48
 PATH_BUILDS = ("nested", "regen", "wavefront", "split")  # the tracer's path_regen modes 0-3
 
 

@@ -37,8 +37,9 @@ constexpr uint32_t PHR_INST = 1u << 30;  // a top-tree leaf's range is instance 
 
 struct SceneDev {
     const float4* nodes;
-    const float4* recs;    // one tree's walk records (4 float4 a node index); a forest walks `nodes`
-    const float4* kids;    // the records' second level (8 float4 a node index), after the first
+    const float4* wide;    // one tree's wide records (WIDE_ROWS float4 a node index); a forest walks `nodes`
+    const float4* recs;    // binary records (4 float4 a node index) of the ordered any-hit walk
+    const float4* kids;    // their second level (8 float4 a node index), after the first
     const float4* tris;    // 3 float4 per slot: (a.xyz, b.x) (b.yz, c.xy) (c.z, -, -, -)
     const uint4* faces;    // slot order: 3 vertex ids + material
     const float4* verts;   // 2 float4 per vertex: (pos, 1) (oct.xy, u, v)
@@ -118,28 +119,224 @@ __device__ __forceinline__ float box_t(float4 lo, float4 hi, V3 o, V3 inv, float
     return (tmax >= e && tmin < best) ? e : PHR_INF;
 }
 
-// trace_blas for one identity instance, root at node `root`, over the tree's
-// walk records: record x (node x an inner node) holds x's two children side
-// by side as 32-byte nodes, an inner child's words replaced by (its own node
-// index, 0) and a leaf child's kept (first | LEAF, end). A step reads one
-// aligned 64-byte record and tests both boxes; the stack holds the far
-// child's first word, so a pop needs no load of its own. A leaf taken from
-// the stack learns its end from the cache row of its first triangle (row 2,
-// word 1). The visits, and so the hits and counts, are those of the node
-// walk: both children tested, the nearer entered first (a tie to the left),
-// the farther pushed. `stk` is this thread's LDS stack column (stride =
-// threads per block).
+// ---- the wide walk ---------------------------------------------------------
+// A closest hit is the least t over the triangles the ray meets, and of equal
+// t's the first in the binary walk's order; a shadow ray only asks whether
+// anything blocks it. Neither depends on the order the walk takes, so one
+// tree is walked four boxes at a time: each inner node x has a record of up
+// to four descendants (x's children, the widest inner one opened, then the
+// widest of those), as rows of one coordinate of all four, and a child word
+// each: an inner child's node index, a leaf's first | LEAF (its end sits in
+// row 2 .y of its first triangle's cache row), PHR_NONE for no child (its box
+// is NaN and never met). On the 1.31M-triangle spheres scene a ray takes 11.7
+// such visits where the binary records took 14.5 two-level ones, and a visit
+// is shorter: near and far planes are picked by address from the ray's signs
+// (no min / max a plane) and only the nearest child is sorted out (the others
+// pushed as they lie: 1% more visits than a full sort).
+//
+// Every box's test is box_t's, product for product, so a leaf is met exactly
+// where the binary walk would meet it (a box inside another is met only where
+// the other is, since rounding keeps the order of the planes); a box the ray
+// enters at the very t of the hit in hand is still entered, for a tie.
+constexpr uint32_t WIDE_ROWS = 8;  // lo.x hi.x lo.y hi.y lo.z hi.z words, one row unused: 128 B, one cache line
+
+typedef float vec4 __attribute__((ext_vector_type(4)));
+// The visit of inner node `cur`: the nearest child met is entered (cur), the
+// others are pushed. False when none is met. The caller keeps three free
+// entries on the stack.
+__device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float best_t, uint32_t& cur, uint32_t* stk, uint32_t stride,
+                                       uint32_t& sp) {
+    // A ray's near x, y and z rows: lo where it goes up the axis, else hi.
+    const uint32_t nx = (__float_as_uint(inv.x) >> 27) & 16u, ny = (__float_as_uint(inv.y) >> 27) & 16u,
+                   nz = (__float_as_uint(inv.z) >> 27) & 16u;
+    const char* r = (const char*)s.wide + (uint64_t)cur * (16u * WIDE_ROWS);
+    auto row = [&](uint32_t off, uint32_t at) { return *(const vec4*)(r + off + at); };
+    const vec4 ax = row(nx, 0u), bx = row(nx ^ 16u, 0u), ay = row(ny, 32u), by = row(ny ^ 16u, 32u), az = row(nz, 64u),
+               bz = row(nz ^ 16u, 64u), wd = row(96u, 0u);
+    auto child = [&](float x0, float x1, float y0, float y1, float z0, float z1) {  // where the ray enters, PHR_INF on a miss
+        const float tn = fmaxf(fmaxf(fmaxf((x0 - o.x) * inv.x, (y0 - o.y) * inv.y), (z0 - o.z) * inv.z), 0.f);
+        const float tf = fminf(fminf((x1 - o.x) * inv.x, (y1 - o.y) * inv.y), (z1 - o.z) * inv.z);
+        return (tn <= tf && tn <= best_t) ? tn : PHR_INF;
+    };
+    float k0 = child(ax.x, bx.x, ay.x, by.x, az.x, bz.x), k1 = child(ax.y, bx.y, ay.y, by.y, az.y, bz.y);
+    float k2 = child(ax.z, bx.z, ay.z, by.z, az.z, bz.z), k3 = child(ax.w, bx.w, ay.w, by.w, az.w, bz.w);
+    float w0 = wd.x, w1 = wd.y, w2 = wd.z, w3 = wd.w;
+    auto nearer_first = [](float& ka, float& wa, float& kb, float& wb) {
+        const bool sw = kb < ka;
+        const float k = sw ? kb : ka, w = sw ? wb : wa;
+        kb = sw ? ka : kb;
+        wb = sw ? wa : wb;
+        ka = k;
+        wa = w;
+    };
+    nearer_first(k0, w0, k1, w1);
+    nearer_first(k2, w2, k3, w3);
+    nearer_first(k0, w0, k2, w2);
+    // Stored whether met or not; the count moves on only past a met one.
+    stk[sp * stride] = __float_as_uint(w3);
+    sp += k3 < PHR_INF ? 1u : 0u;
+    stk[sp * stride] = __float_as_uint(w2);
+    sp += k2 < PHR_INF ? 1u : 0u;
+    stk[sp * stride] = __float_as_uint(w1);
+    sp += k1 < PHR_INF ? 1u : 0u;
+    cur = __float_as_uint(w0);
+    return k0 < PHR_INF;
+}
+// A visit pushes up to three and stores one past what it pushes.
+constexpr uint32_t WIDE_ROOM = PHR_STACK - 3u;
+
+// Of two triangles (slots a and b) the ray meets at the same t, whether a
+// comes first in the binary walk: at the node where their ways part, the
+// nearer child does (a tie to the left); within a leaf, the lower slot.
+__device__ __forceinline__ bool first_of(const SceneDev& s, V3 o, V3 inv, uint32_t a, uint32_t b) {
+    uint32_t x = s.root;
+    for (;;) {
+        const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
+        const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
+        if (l & PHR_LEAF) return a < b;
+        uint32_t y = r;  // the right child's first slot: its leftmost leaf's
+        uint32_t w = __float_as_uint(s.nodes[2 * (size_t)y].w);
+        while (!(w & PHR_LEAF)) {
+            y = w;
+            w = __float_as_uint(s.nodes[2 * (size_t)y].w);
+        }
+        const uint32_t split = w & ~PHR_LEAF;
+        const bool a_left = a < split, b_left = b < split;
+        if (a_left == b_left) {
+            x = a_left ? l : r;
+            continue;
+        }
+        const float tl = box_t(s.nodes[2 * (size_t)l], s.nodes[2 * (size_t)l + 1], o, inv, PHR_INF);
+        const float tr = box_t(s.nodes[2 * (size_t)r], s.nodes[2 * (size_t)r + 1], o, inv, PHR_INF);
+        return (tl <= tr) == a_left;
+    }
+}
+// Whether a triangle met at t replaces the hit (best_t, best): the nearer one
+// does, and of two at one t the binary walk's first.
+__device__ __forceinline__ bool takes(const SceneDev& s, V3 o, V3 inv, float t, uint32_t id, float best_t, uint32_t best) {
+    if (t < best_t) return true;
+    return t == best_t && best != PHR_NONE && id != best && first_of(s, o, inv, id, best);
+}
+__device__ __forceinline__ bool blocks(const SceneDev& s, uint32_t id) {  // bvh.wgsl:158-160: glass and cut-outs pass
+    const float* m = s.mats + MAT_WORDS * (size_t)s.faces[id].w;
+    return !(m[6] > 0.5f || m[3] < 0.5f);
+}
+
+// The rest of a walk whose stack has no room left (far deeper than any tree
+// measured: 13 of 32 entries at most on the benchmark scenes): the whole tree
+// again by the binary walk over the nodes, which holds one pending node a
+// level and so always fits, with the hit found so far.
+__device__ __forceinline__ void walk_nodes(const SceneDev& s, V3 o, V3 inv, const RaySpace& rs, bool any, PhrHit& best, uint32_t* stk,
+                                           uint32_t stride, uint32_t& tests) {
+    uint32_t sp = 0, x = s.root;
+    for (;;) {
+        const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
+        const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
+        if (l & PHR_LEAF) {
+            for (uint32_t id = l & ~PHR_LEAF; id < r; ++id) {
+                ++tests;
+                float u, v;
+                const float t = tri_t(s.tris[3 * (size_t)id], s.tris[3 * (size_t)id + 1], s.tris[3 * (size_t)id + 2], o, rs, u, v);
+                if (any) {
+                    if (t < best.t && blocks(s, id)) {
+                        best.tri = id;
+                        return;
+                    }
+                } else if (takes(s, o, inv, t, id, best.t, best.tri)) {
+                    best = PhrHit{t, id, u, v, 0u};
+                }
+            }
+        } else {
+            // One step past a hit: an equal t further on may come first.
+            const float far = best.tri != PHR_NONE && !any ? __uint_as_float(__float_as_uint(best.t) + 1u) : best.t;
+            const float tl = box_t(s.nodes[2 * (size_t)l], s.nodes[2 * (size_t)l + 1], o, inv, far);
+            const float tr = box_t(s.nodes[2 * (size_t)r], s.nodes[2 * (size_t)r + 1], o, inv, far);
+            const bool hl = tl < PHR_INF, hr = tr < PHR_INF;
+            if (hl || hr) {
+                const bool left = hl && (!hr || tl <= tr);
+                if (hl && hr) stk[sp++ * stride] = left ? r : l;
+                x = left ? l : r;
+                continue;
+            }
+        }
+        if (sp == 0) return;
+        x = stk[--sp * stride];
+    }
+}
+
+// Where a walk starts: the root's index, or its leaf word where the root is
+// a leaf, whose end (no record holds it) is then `end` (else PHR_NONE).
+__device__ __forceinline__ uint32_t wide_root(const SceneDev& s, uint32_t& end) {
+    const uint32_t w = __float_as_uint(s.nodes[2 * (size_t)s.root].w);
+    end = (w & PHR_LEAF) ? __float_as_uint(s.nodes[2 * (size_t)s.root + 1].w) : PHR_NONE;
+    return (w & PHR_LEAF) ? w : s.root;
+}
+
+// The walk to the closest hit, or (ANY) to whether something blocks the ray
+// before tmax (then the hit's triangle is some blocking one). `steps` and
+// `tests` count visits and triangle tests, the units the walk's memory
+// traffic is priced in.
+template <bool ANY>
+__device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* stk, uint32_t stride, uint32_t& steps,
+                                       uint32_t& tests) {
+    PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
+    const V3 inv = safe_inv(d);
+    const RaySpace rs = ray_space(d);
+    uint32_t sp = 0, only, cur = wide_root(s, only);
+    for (;;) {
+        if (cur & PHR_LEAF) {
+            uint32_t id = cur & ~PHR_LEAF;
+            float4 t0 = s.tris[3 * (size_t)id], t1 = s.tris[3 * (size_t)id + 1], t2 = s.tris[3 * (size_t)id + 2];
+            const uint32_t end = only != PHR_NONE ? only : __float_as_uint(t2.y);
+            for (;;) {
+                ++tests;
+                // The leaf's next triangle is loaded while this one is tested.
+                const bool more = id + 1u < end;
+                float4 n0 = t0, n1 = t1, n2 = t2;
+                if (more) {
+                    n0 = s.tris[3 * (size_t)(id + 1u)];
+                    n1 = s.tris[3 * (size_t)(id + 1u) + 1];
+                    n2 = s.tris[3 * (size_t)(id + 1u) + 2];
+                }
+                float u, v;
+                const float t = tri_t(t0, t1, t2, o, rs, u, v);
+                if constexpr (ANY) {
+                    if (t < best.t && blocks(s, id)) return PhrHit{t, id, u, v, 0u};
+                } else {
+                    if (takes(s, o, inv, t, id, best.t, best.tri)) best = PhrHit{t, id, u, v, 0u};
+                }
+                if (!more) break;
+                ++id;
+                t0 = n0;
+                t1 = n1;
+                t2 = n2;
+            }
+        } else if (sp > WIDE_ROOM) {
+            walk_nodes(s, o, inv, rs, ANY, best, stk, stride, tests);
+            break;
+        } else {
+            ++steps;
+            if (visit4(s, o, inv, best.t, cur, stk, stride, sp)) continue;
+        }
+        if (sp == 0) break;
+        cur = stk[--sp * stride];
+    }
+    return best;
+}
+
+// ---- the ordered any-hit walk -------------------------------------------------
+// A caller's any-hit ray (Tracer raycast) gets the first triangle the binary
+// walk meets, so this one keeps that walk's order: trace_blas for one
+// identity instance, root at node `root`, over binary records.
 // Any-hit rays skip triangles of glass or cut-out materials (trans > 0.5 or
 // alpha < 0.5, bvh.wgsl:158-160): `faces` and `mats` give the material.
-// `steps` and `tests` count inner-node visits and triangle tests, the units
-// the walk's memory traffic is priced in.
-// Walk records, for each node index x of an inner node a walk reaches: its
-// children A and B as two Nodes (4 float4 at recs[4x], dense, what the
-// binary step reads), and, for each child that is inner, that child's two
-// children (8 float4 at kids[8x]: A's, then B's). An inner child's words
-// are (its node index, 0); a leaf child keeps (first | LEAF, end). Both
-// live in one array of REC_ROWS float4 a node: recs for every node, then
-// kids for every node.
+// The records, for each node index x of an inner node a walk reaches: its
+// children A and B as two Nodes (4 float4 at recs[4x]) and, for each child
+// that is inner, that child's two children (8 float4 at kids[8x]: A's, then
+// B's). An inner child's words are (its node index, 0); a leaf child keeps
+// (first | LEAF, end). Both live in one array of REC_ROWS float4 a node: recs
+// for every node, then kids for every node. The stack holds the far child's
+// first word, so a pop needs no load of its own.
 constexpr uint32_t REC_ROWS = 12;
 
 // The walk's visit of inner node `cur` from its record: the binary step at
@@ -149,31 +346,6 @@ constexpr uint32_t REC_ROWS = 12;
 // walk's decisions and pushes; the record's three 64-B lines are read at
 // once (r = recs + 4 cur, k = kids + 8 cur). False when nothing is entered
 // (the caller pops).
-// visit1 is the binary step alone (the record's first line), for kernels
-// whose registers have no room for the other two lines.
-__device__ __forceinline__ bool visit1(const float4* __restrict__ r, V3 o, V3 inv, float best_t, uint32_t& cur, uint32_t& end,
-                                       uint32_t* stk, uint32_t stride, uint32_t& sp, uint32_t& steps) {
-    const float4 llo = r[0], lhi = r[1], qlo = r[2], qhi = r[3];
-    ++steps;
-    const float tl = box_t(llo, lhi, o, inv, best_t);
-    const float tr = box_t(qlo, qhi, o, inv, best_t);
-    if (tl < PHR_INF && tr < PHR_INF) {
-        if (tl <= tr) {
-            stk[sp * stride] = __float_as_uint(qlo.w);
-            cur = __float_as_uint(llo.w);
-            end = __float_as_uint(lhi.w);
-        } else {
-            stk[sp * stride] = __float_as_uint(llo.w);
-            cur = __float_as_uint(qlo.w);
-            end = __float_as_uint(qhi.w);
-        }
-        ++sp;
-        return true;
-    }
-    if (tl < PHR_INF) { cur = __float_as_uint(llo.w); end = __float_as_uint(lhi.w); return true; }
-    if (tr < PHR_INF) { cur = __float_as_uint(qlo.w); end = __float_as_uint(qhi.w); return true; }
-    return false;
-}
 // visit2_rows: the visit from rows already loaded (the record's four, then
 // its eight kids rows); visit2 loads them from the record.
 __device__ __forceinline__ bool visit2_rows(float4 alo, float4 ahi, float4 blo, float4 bhi, float4 a0lo, float4 a0hi, float4 a1lo,
@@ -229,27 +401,22 @@ __device__ __forceinline__ bool visit2(const float4* __restrict__ r, const float
                        steps);
 }
 
-// TWO: a visit takes two levels from the record (visit2), else one (visit1);
-// the same decisions either way.
-template <bool ANY, bool TWO = false>
-__device__ __forceinline__ PhrHit walk(const float4* __restrict__ nodes, const float4* __restrict__ recs, const float4* __restrict__ kids,
-                                       uint32_t root,
-                                       const float4* __restrict__ tris, const uint4* __restrict__ faces, const float* __restrict__ mats,
-                                       V3 o, V3 d, float tmax, uint32_t* stk, uint32_t stride, uint32_t& steps, uint32_t& tests) {
-    PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
-    V3 inv = safe_inv(d);
-    const float4 rlo = nodes[2 * root], rhi = nodes[2 * root + 1];
-    if (box_t(rlo, rhi, o, inv, best.t) >= PHR_INF) return best;
-    RaySpace rs = ray_space(d);
+__device__ __forceinline__ PhrHit walk_first(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* stk, uint32_t stride, uint32_t& steps,
+                                             uint32_t& tests) {
+    const PhrHit none{tmax, PHR_NONE, 0.f, 0.f, 0u};
+    const V3 inv = safe_inv(d);
+    const float4 rlo = s.nodes[2 * (size_t)s.root], rhi = s.nodes[2 * (size_t)s.root + 1];
+    if (box_t(rlo, rhi, o, inv, tmax) >= PHR_INF) return none;
+    const RaySpace rs = ray_space(d);
     uint32_t sp = 0;
     // The entry in hand: an inner node's index (its record), or a leaf's
     // first | LEAF with its end (PHR_NONE when it came off the stack).
     uint32_t cur = __float_as_uint(rlo.w), end = __float_as_uint(rhi.w);
-    if (!(cur & PHR_LEAF)) cur = root;
+    if (!(cur & PHR_LEAF)) cur = s.root;
     for (;;) {
         if (cur & PHR_LEAF) {
             uint32_t id = cur & ~PHR_LEAF;
-            float4 t0 = tris[3 * id], t1 = tris[3 * id + 1], t2 = tris[3 * id + 2];
+            float4 t0 = s.tris[3 * (size_t)id], t1 = s.tris[3 * (size_t)id + 1], t2 = s.tris[3 * (size_t)id + 2];
             if (end == PHR_NONE) end = __float_as_uint(t2.y);
             for (;;) {
                 ++tests;
@@ -257,45 +424,32 @@ __device__ __forceinline__ PhrHit walk(const float4* __restrict__ nodes, const f
                 const bool more = id + 1u < end;
                 float4 n0 = t0, n1 = t1, n2 = t2;
                 if (more) {
-                    n0 = tris[3 * (id + 1u)];
-                    n1 = tris[3 * (id + 1u) + 1];
-                    n2 = tris[3 * (id + 1u) + 2];
+                    n0 = s.tris[3 * (size_t)(id + 1u)];
+                    n1 = s.tris[3 * (size_t)(id + 1u) + 1];
+                    n2 = s.tris[3 * (size_t)(id + 1u) + 2];
                 }
                 float u, v;
-                float t = tri_t(t0, t1, t2, o, rs, u, v);
-                if (t < best.t) {
-                    if (ANY) {
-                        const float* m = mats + MAT_WORDS * (size_t)faces[id].w;
-                        if (!(m[6] > 0.5f || m[3] < 0.5f)) return PhrHit{t, id, u, v, 0u};
-                    } else {
-                        best = PhrHit{t, id, u, v, 0u};
-                    }
-                }
+                const float t = tri_t(t0, t1, t2, o, rs, u, v);
+                if (t < tmax && blocks(s, id)) return PhrHit{t, id, u, v, 0u};
                 if (!more) break;
                 ++id;
                 t0 = n0;
                 t1 = n1;
                 t2 = n2;
             }
-        } else if (TWO ? visit2(recs + 4 * (size_t)cur, kids + 8 * (size_t)cur, o, inv, best.t, cur, end, stk, stride, sp, steps)
-                       : visit1(recs + 4 * (size_t)cur, o, inv, best.t, cur, end, stk, stride, sp, steps)) {
+        } else if (visit2(s.recs + 4 * (size_t)cur, s.kids + 8 * (size_t)cur, o, inv, tmax, cur, end, stk, stride, sp, steps)) {
             continue;
         }
-        if (sp == 0) break;
-        --sp;
-        cur = stk[sp * stride];
+        if (sp == 0) return none;
+        cur = stk[--sp * stride];
         end = PHR_NONE;
     }
-    return best;
 }
 
 // A walk that can stop after any unit and go on later (the split build):
-// the ray, its best hit, where it is (cur, end) and its stack (sp entries of
-// the thread's column). A unit is an inner node's record (both boxes, the
-// nearer child entered and the farther pushed) or one triangle, so a walk
-// makes walk<ANY>'s visits, decisions and pushes in walk<ANY>'s order and
-// ends with its hit. `any`: a shadow ray's walk, which ends at the first
-// triangle that blocks it.
+// the ray, its best hit, the entry in hand (cur) and its stack (sp entries of
+// the thread's column). A unit is an inner node's visit or one triangle.
+// `any`: a shadow ray's walk, which ends at the first triangle that blocks it.
 struct Walker {
     V3 o, inv;
     RaySpace rs;
@@ -312,96 +466,52 @@ __device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, V3 o,
     w.tri = PHR_NONE;
     w.sp = 0;
     w.any = any;
-    const float4 rlo = s.nodes[2 * s.root], rhi = s.nodes[2 * s.root + 1];
-    w.on = box_t(rlo, rhi, o, w.inv, tmax) < PHR_INF;
-    w.cur = __float_as_uint(rlo.w);
-    w.end = __float_as_uint(rhi.w);
-    if (!(w.cur & PHR_LEAF)) w.cur = s.root;
+    w.on = true;
+    w.cur = wide_root(s, w.end);
 }
-// TWO: an inner node's unit is visit2's (two levels from the record and its
-// kids rows), else the binary step.
-template <bool TWO = false>
 __device__ __forceinline__ void walker_step(Walker& w, const SceneDev& s, uint32_t* stk, uint32_t stride, uint32_t& steps,
                                             uint32_t& tests) {
-    const bool leaf = (w.cur & PHR_LEAF) != 0u;
-    const float4* q = leaf ? s.tris + 3 * (size_t)(w.cur & ~PHR_LEAF) : s.recs + 4 * (size_t)w.cur;
-    const float4 a = q[0], b = q[1], c = q[2];
-    float4 d = a, k0 = a, k1 = a, k2 = a, k3 = a, k4 = a, k5 = a, k6 = a, k7 = a;
-    if (!leaf) {
-        d = q[3];
-        if constexpr (TWO) {
-            const float4* kk = s.kids + 8 * (size_t)w.cur;
-            k0 = kk[0];
-            k1 = kk[1];
-            k2 = kk[2];
-            k3 = kk[3];
-            k4 = kk[4];
-            k5 = kk[5];
-            k6 = kk[6];
-            k7 = kk[7];
-        }
-    }
-    if constexpr (TWO) {
-        if (!leaf) {
-            if (visit2_rows(a, b, c, d, k0, k1, k2, k3, k4, k5, k6, k7, w.o, w.inv, w.t, w.cur, w.end, stk, stride, w.sp, steps)) return;
-            if (w.sp == 0) {
-                w.on = false;
-                return;
-            }
-            --w.sp;
-            w.cur = stk[w.sp * stride];
-            w.end = PHR_NONE;
-            return;
-        }
-    }
-    if (leaf) {
+    if (w.cur & PHR_LEAF) {
         const uint32_t id = w.cur & ~PHR_LEAF;
+        const float4 a = s.tris[3 * (size_t)id], b = s.tris[3 * (size_t)id + 1], c = s.tris[3 * (size_t)id + 2];
         ++tests;
         if (w.end == PHR_NONE) w.end = __float_as_uint(c.y);
         float u, v;
         const float t = tri_t(a, b, c, w.o, w.rs, u, v);
-        if (t < w.t) {
-            if (w.any) {
-                const float* m = s.mats + MAT_WORDS * (size_t)s.faces[id].w;
-                if (!(m[6] > 0.5f || m[3] < 0.5f)) {
-                    w.tri = id;
-                    w.on = false;
-                    return;
-                }
-            } else {
-                w.t = t;
+        if (w.any) {
+            if (t < w.t && blocks(s, id)) {
                 w.tri = id;
-                w.u = u;
-                w.v = v;
+                w.on = false;
+                return;
             }
+        } else if (takes(s, w.o, w.inv, t, id, w.t, w.tri)) {
+            w.t = t;
+            w.tri = id;
+            w.u = u;
+            w.v = v;
         }
         if (id + 1u < w.end) {
             w.cur = (id + 1u) | PHR_LEAF;
             return;
         }
+        w.end = PHR_NONE;
+    } else if (w.sp > WIDE_ROOM) {
+        PhrHit best{w.t, w.tri, w.u, w.v, 0u};
+        walk_nodes(s, w.o, w.inv, w.rs, w.any, best, stk, stride, tests);
+        w.t = best.t;
+        w.tri = best.tri;
+        w.u = best.u;
+        w.v = best.v;
+        w.sp = 0;
     } else {
         ++steps;
-        const float tl = box_t(a, b, w.o, w.inv, w.t);
-        const float tr = box_t(c, d, w.o, w.inv, w.t);
-        const bool hl = tl < PHR_INF, hr = tr < PHR_INF;
-        if (hl || hr) {
-            const bool left = hl && (!hr || tl <= tr);
-            if (hl && hr) {
-                stk[w.sp * stride] = __float_as_uint(left ? c.w : a.w);
-                ++w.sp;
-            }
-            w.cur = __float_as_uint(left ? a.w : c.w);
-            w.end = __float_as_uint(left ? b.w : d.w);
-            return;
-        }
+        if (visit4(s, w.o, w.inv, w.t, w.cur, stk, stride, w.sp)) return;
     }
     if (w.sp == 0) {
         w.on = false;
         return;
     }
-    --w.sp;
-    w.cur = stk[w.sp * stride];
-    w.end = PHR_NONE;
+    w.cur = stk[--w.sp * stride];
 }
 
 // The walk records of a tree's nodes (one entry per node index; only inner
@@ -438,6 +548,62 @@ __global__ __launch_bounds__(256) void k_walk_records(const float4* __restrict__
         rec_child(nodes, g0, k + 4 * c, tris);
         rec_child(nodes, g1, k + 4 * c + 2, tris);
     }
+}
+
+// The wide records of a tree's inner nodes (as `inner` marks them).
+struct WideKid {
+    float4 lo, hi;  // words: an inner child's (its own left, right), a leaf's
+    uint32_t at;
+};
+__device__ __forceinline__ WideKid wide_kid(const float4* __restrict__ nodes, uint32_t y) {
+    return WideKid{nodes[2 * (size_t)y], nodes[2 * (size_t)y + 1], y};
+}
+__device__ __forceinline__ float wide_area(const WideKid& k) {  // -1: a leaf is not opened
+    const float x = k.hi.x - k.lo.x, y = k.hi.y - k.lo.y, z = k.hi.z - k.lo.z;
+    return (__float_as_uint(k.lo.w) & PHR_LEAF) ? -1.0f : x * y + y * z + z * x;
+}
+__global__ __launch_bounds__(256) void k_wide_records(const float4* __restrict__ nodes, const uint8_t* __restrict__ inner, uint32_t count,
+                                                      float4* __restrict__ wide, float4* __restrict__ tris) {
+    const uint32_t x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= count || !inner[x]) return;
+    const float nan = __uint_as_float(0x7fc00000u);
+    const WideKid none{make_float4(nan, nan, nan, __uint_as_float(PHR_NONE)), make_float4(nan, nan, nan, 0.f), PHR_NONE};
+    WideKid k[4] = {wide_kid(nodes, __float_as_uint(nodes[2 * (size_t)x].w)), wide_kid(nodes, __float_as_uint(nodes[2 * (size_t)x + 1].w)),
+                    none, none};
+    for (int c = 0; c < 2; ++c)  // a leaf's end, in its first triangle's cache row
+        if (__float_as_uint(k[c].lo.w) & PHR_LEAF) tris[3 * (size_t)(__float_as_uint(k[c].lo.w) & ~PHR_LEAF) + 2].y = k[c].hi.w;
+#pragma unroll
+    for (int c = 2; c < 4; ++c) {
+        int at = -1;
+        float most = -1.0f;
+#pragma unroll
+        for (int e = 0; e < c; ++e) {
+            const float a = k[e].at == PHR_NONE ? -1.0f : wide_area(k[e]);
+            if (a > most) most = a, at = e;
+        }
+        const uint32_t l = __float_as_uint(at == 0 ? k[0].lo.w : (at == 1 ? k[1].lo.w : k[2].lo.w));
+        const uint32_t r = __float_as_uint(at == 0 ? k[0].hi.w : (at == 1 ? k[1].hi.w : k[2].hi.w));
+        if (at < 0) continue;
+        const WideKid kl = wide_kid(nodes, l);
+        k[c] = wide_kid(nodes, r);
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (e == at) k[e] = kl;
+    }
+    float4* o = wide + WIDE_ROWS * (size_t)x;
+    o[0] = make_float4(k[0].lo.x, k[1].lo.x, k[2].lo.x, k[3].lo.x);
+    o[1] = make_float4(k[0].hi.x, k[1].hi.x, k[2].hi.x, k[3].hi.x);
+    o[2] = make_float4(k[0].lo.y, k[1].lo.y, k[2].lo.y, k[3].lo.y);
+    o[3] = make_float4(k[0].hi.y, k[1].hi.y, k[2].hi.y, k[3].hi.y);
+    o[4] = make_float4(k[0].lo.z, k[1].lo.z, k[2].lo.z, k[3].lo.z);
+    o[5] = make_float4(k[0].hi.z, k[1].hi.z, k[2].hi.z, k[3].hi.z);
+    float w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t a = __float_as_uint(k[e].lo.w);
+        w[e] = __uint_as_float((a & PHR_LEAF) ? a : k[e].at);  // PHR_NONE has the leaf bit
+    }
+    o[6] = make_float4(w[0], w[1], w[2], w[3]);
 }
 
 // An instance's row times (x, y, z, w), summed in trace_blas's order.
@@ -754,8 +920,8 @@ __global__ __launch_bounds__(TRACE_THREADS) void k_raycast(SceneDev sc, const Ph
             h = any ? walk_forest<true>(sc, o, d, a.w, s_tstack + threadIdx.x, stk, TRACE_THREADS, steps, tests)
                     : walk_forest<false>(sc, o, d, a.w, s_tstack + threadIdx.x, stk, TRACE_THREADS, steps, tests);
         else
-            h = any ? walk<true, true>(sc.nodes, sc.recs, sc.kids, sc.root, sc.tris, sc.faces, sc.mats, o, d, a.w, stk, TRACE_THREADS, steps, tests)
-                    : walk<false, true>(sc.nodes, sc.recs, sc.kids, sc.root, sc.tris, sc.faces, sc.mats, o, d, a.w, stk, TRACE_THREADS, steps, tests);
+            h = any ? walk_first(sc, o, d, a.w, stk, TRACE_THREADS, steps, tests)
+                    : walk<false>(sc, o, d, a.w, stk, TRACE_THREADS, steps, tests);
         hits[i] = h;
     }
     if (counters) {
@@ -828,13 +994,11 @@ __device__ __forceinline__ PhrHit trace(Ctx& c, V3 o, V3 d, float tmax, bool fir
     if (first) {
         c.shadow++;
         if constexpr (F) return walk_forest<true>(c.s, o, d, tmax, c.tstk, c.stk, TRACE_THREADS, c.steps, c.tests);
-        return walk<true>(c.s.nodes, c.s.recs, c.s.kids, c.s.root, c.s.tris, c.s.faces, c.s.mats, o, d, tmax, c.stk, TRACE_THREADS, c.steps,
-                          c.tests);
+        return walk<true>(c.s, o, d, tmax, c.stk, TRACE_THREADS, c.steps, c.tests);
     }
     c.closest++;
     if constexpr (F) return walk_forest<false>(c.s, o, d, tmax, c.tstk, c.stk, TRACE_THREADS, c.steps, c.tests);
-    return walk<false>(c.s.nodes, c.s.recs, c.s.kids, c.s.root, c.s.tris, c.s.faces, c.s.mats, o, d, tmax, c.stk, TRACE_THREADS, c.steps,
-                       c.tests);
+    return walk<false>(c.s, o, d, tmax, c.stk, TRACE_THREADS, c.steps, c.tests);
 }
 template <bool F>
 __device__ __forceinline__ float visible(Ctx& c, V3 org, V3 l, float dist) {
@@ -1777,7 +1941,7 @@ struct SplitWalk {
     Walker w;
     __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, s, o, d, tmax, any); }
     __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t*, uint32_t& steps, uint32_t& tests) {
-        walker_step<true>(w, s, stk, TRACE_THREADS, steps, tests);
+        walker_step(w, s, stk, TRACE_THREADS, steps, tests);
     }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, 0u}; }
 };
@@ -2137,11 +2301,12 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
     PhrHit best{PHR_INF, PHR_NONE, 0.f, 0.f, 0u};
     V3 o = v3(0, 0, 0), inv = o;
     RaySpace rs{};
-    uint32_t cur = 0, end = 0, sp = 0, slot = 0;
+    uint32_t cur = 0, sp = 0, slot = 0;
     uint32_t steps = 0, tests = 0, nrays = 0;
     bool live = false, drained = count == 0u;
     uint32_t cbase = 0, cend = 0;  // the wave's chunk of the queue
-    const float4 rlo = sc.nodes[2 * sc.root], rhi = sc.nodes[2 * sc.root + 1];
+    uint32_t only;
+    const uint32_t root = wide_root(sc, only);
     // A finished walk's result: the hit for the shading, or the shadow ray's
     // visibility taken into the field its turn left.
     // A finished walk only stores: the hit for the shading, or the shadow
@@ -2188,16 +2353,10 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                 ++nrays;
                 best = PhrHit{tmax, PHR_NONE, 0.f, 0.f, 0u};
                 inv = safe_inv(d);
-                if (box_t(rlo, rhi, o, inv, best.t) >= PHR_INF) {
-                    finish();
-                } else {
-                    rs = ray_space(d);
-                    sp = 0;
-                    cur = __float_as_uint(rlo.w);
-                    end = __float_as_uint(rhi.w);
-                    if (!(cur & PHR_LEAF)) cur = sc.root;
-                    live = true;
-                }
+                rs = ray_space(d);
+                sp = 0;
+                cur = root;
+                live = true;
             }
         }
         if (__ballot(live) == 0ull) {
@@ -2209,34 +2368,35 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
         // pop if nothing was entered.
         bool more = true, popped = true;
         if (cur & PHR_LEAF) {
-            uint32_t id = cur & ~PHR_LEAF;
+            uint32_t id = cur & ~PHR_LEAF, end = only;
             do {
                 ++tests;
-                const float4 t0 = sc.tris[3 * id], t1 = sc.tris[3 * id + 1], t2 = sc.tris[3 * id + 2];
+                const float4 t0 = sc.tris[3 * (size_t)id], t1 = sc.tris[3 * (size_t)id + 1], t2 = sc.tris[3 * (size_t)id + 2];
                 if (end == PHR_NONE) end = __float_as_uint(t2.y);
                 float u, v;
                 const float t = tri_t(t0, t1, t2, o, rs, u, v);
-                if (t < best.t) {
-                    if (ANY) {
-                        const float* m = sc.mats + MAT_WORDS * (size_t)sc.faces[id].w;
-                        if (m[6] > 0.5f || m[3] < 0.5f) continue;
+                if constexpr (ANY) {
+                    if (t < best.t && blocks(sc, id)) {
                         best = PhrHit{t, id, u, v, 0u};
                         more = false;
                         break;
                     }
+                } else if (takes(sc, o, inv, t, id, best.t, best.tri)) {
                     best = PhrHit{t, id, u, v, 0u};
                 }
             } while (++id < end);
+        } else if (sp > WIDE_ROOM) {
+            walk_nodes(sc, o, inv, rs, ANY, best, stk, WF_THREADS, tests);
+            more = false;
         } else {
-            popped = !visit2(sc.recs + 4 * (size_t)cur, sc.kids + 8 * (size_t)cur, o, inv, best.t, cur, end, stk, WF_THREADS, sp, steps);
+            ++steps;
+            popped = !visit4(sc, o, inv, best.t, cur, stk, WF_THREADS, sp);
         }
         if (more && popped) {
             if (sp == 0) {
                 more = false;
             } else {
-                --sp;
-                cur = stk[sp * WF_THREADS];
-                end = PHR_NONE;
+                cur = stk[--sp * WF_THREADS];
             }
         }
         if (!more) {
@@ -2718,10 +2878,20 @@ phr_array* phr_bvh_internal_order(phr_bvh* b);
 const uint8_t* phr_bvh_internal_inner(phr_bvh* b);
 
 // The walk records of a built tree (after its gather wrote the triangle
-// cache), into `recs`, allocated on first use.
-static int enqueue_walk_records(phr_gpu* g, phr_bvh* bvh, phr_array** recs, phr_array* tris) {
+// cache): the wide ones into `wide` and, where `recs` is given, the ordered
+// any-hit walk's into it; each allocated on first use.
+static int enqueue_walk_records(phr_gpu* g, phr_bvh* bvh, phr_array** wide, phr_array** recs, phr_array* tris) {
     phr_array* nodes = phr_bvh_internal_nodes(bvh);
     const uint64_t count = nodes->len;
+    if (!*wide) {
+        int rc = phr_array_alloc(g, 16 * WIDE_ROWS, std::max<uint64_t>(count, 1), wide);
+        if (rc != PHR_OK) return rc;
+    }
+    if (count)
+        hipLaunchKernelGGL(k_wide_records, dim3((uint32_t)((count + 255) / 256)), dim3(256), 0, g->stream, (const float4*)nodes->ptr,
+                           phr_bvh_internal_inner(bvh), (uint32_t)count, (float4*)(*wide)->ptr, (float4*)tris->ptr);
+    PHR_HIP(hipGetLastError());
+    if (!recs) return PHR_OK;
     if (!*recs) {
         int rc = phr_array_alloc(g, 16 * REC_ROWS, std::max<uint64_t>(count, 1), recs);
         if (rc != PHR_OK) return rc;
@@ -2750,7 +2920,8 @@ struct phr_tracer {
     phr_array* prims = nullptr;     // Aabb per input face
     phr_array* faces = nullptr;     // uint4 per slot
     phr_array* tris = nullptr;      // 3 float4 per slot
-    phr_array* recs = nullptr;      // one tree's walk records: 64 B a node index
+    phr_array* wide = nullptr;      // one tree's wide walk records: 128 B a node index
+    phr_array* recs = nullptr;      // its binary records for ordered any-hit rays: 192 B a node index
     phr_array* lights = nullptr;    // [count, ids, insts, cdf]
     phr_array* px = nullptr;        // PX_LEN * w * h + 1 words
     unsigned long long* rays = nullptr;  // closest, shadow
@@ -2886,7 +3057,7 @@ void tracer_release(phr_tracer* t) {
     if (!t) return;
     if (t->bvh) phr_bvh_free(t->bvh);
     if (t->tlas) phr_bvh_free(t->tlas);
-    for (phr_array* a : {t->in_faces, t->verts, t->mats, t->prims, t->faces, t->tris, t->recs, t->lights, t->px, t->nodes, t->wboxes,
+    for (phr_array* a : {t->in_faces, t->verts, t->mats, t->prims, t->faces, t->tris, t->wide, t->recs, t->lights, t->px, t->nodes, t->wboxes,
                          t->insts, t->placed_dev, t->worlds_dev, t->inst_mesh, t->lcand, t->lpow, t->wf_state, t->wf_queue,
                          t->wf_shadow})
         phr_array_release(a);
@@ -2961,6 +3132,7 @@ int build_lights(phr_tracer* t, const std::vector<uint32_t>& in_faces, const std
 SceneDev scene_dev(phr_tracer* t) {
     SceneDev s;
     s.nodes = (const float4*)(t->forest ? t->nodes : phr_bvh_internal_nodes(t->bvh))->ptr;
+    s.wide = t->forest ? nullptr : (const float4*)t->wide->ptr;
     s.recs = t->forest ? nullptr : (const float4*)t->recs->ptr;
     s.kids = t->forest ? nullptr : s.recs + 4 * t->recs->len;  // recs holds len nodes' records
     s.insts = t->forest ? (const uint32_t*)t->insts->ptr : nullptr;
@@ -3433,7 +3605,7 @@ int phr_tracer_new(phr_gpu* g, const void* tris_v, uint32_t n, uint32_t leaf, ph
     phr_array* order = phr_bvh_internal_order(t->bvh);
     hipLaunchKernelGGL(k_gather, dim3((n + 255) / 256), dim3(256), 0, s, (const uint4*)t->in_faces->ptr,
                        (const float4*)t->verts->ptr, (const uint32_t*)order->ptr, n, (uint4*)t->faces->ptr, (float4*)t->tris->ptr);
-    if ((rc = enqueue_walk_records(g, t->bvh, &t->recs, t->tris)) != PHR_OK) return fail(rc);
+    if ((rc = enqueue_walk_records(g, t->bvh, &t->wide, &t->recs, t->tris)) != PHR_OK) return fail(rc);
     t->order.resize(n);
     if (hipMemcpyAsync(t->order.data(), order->ptr, 4ull * n, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
@@ -4612,7 +4784,7 @@ struct phr_batch {
     std::vector<uint32_t> seg_lo, node_base, light_at, glow;
     std::vector<float> extent;
     phr_array *in_faces = nullptr, *verts = nullptr, *mats = nullptr, *prims = nullptr, *faces = nullptr, *tris = nullptr,
-              *lights = nullptr, *px = nullptr, *recs = nullptr;
+              *lights = nullptr, *px = nullptr, *wide = nullptr;
     phr_bvh* bvh = nullptr;
     SceneDev* table = nullptr;    // one SceneDev a scene
     PhrCamera* cams = nullptr;    // one stamped camera a scene (device)
@@ -4639,7 +4811,7 @@ void batch_release(phr_batch* b) {
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     if (b->bvh) phr_bvh_free(b->bvh);
-    for (phr_array* a : {b->in_faces, b->verts, b->mats, b->prims, b->faces, b->tris, b->lights, b->px, b->recs}) phr_array_release(a);
+    for (phr_array* a : {b->in_faces, b->verts, b->mats, b->prims, b->faces, b->tris, b->lights, b->px, b->wide}) phr_array_release(a);
     if (b->table) (void)hipFree(b->table);
     if (b->cams) (void)hipFree(b->cams);
     if (b->gcams) (void)hipFree(b->gcams);
@@ -4661,7 +4833,7 @@ int batch_enqueue_build(phr_batch* b) {
     hipLaunchKernelGGL(k_gather, dim3((n + 255) / 256), dim3(256), 0, s, (const uint4*)b->in_faces->ptr, (const float4*)b->verts->ptr,
                        (const uint32_t*)phr_bvh_internal_order(b->bvh)->ptr, n, (uint4*)b->faces->ptr, (float4*)b->tris->ptr);
     PHR_HIP(hipGetLastError());
-    return enqueue_walk_records(b->gpu, b->bvh, &b->recs, b->tris);
+    return enqueue_walk_records(b->gpu, b->bvh, &b->wide, nullptr, b->tris);
 }
 
 // Each scene's camera as a tracer of that scene alone stamps it.
@@ -4827,7 +4999,7 @@ int phr_batch_new(phr_gpu* g, const void* tris_v, const uint32_t* seg_lo, uint32
         return fail(rc);
     hipLaunchKernelGGL(k_gather, dim3((n + 255) / 256), dim3(256), 0, s, (const uint4*)b->in_faces->ptr, (const float4*)b->verts->ptr,
                        (const uint32_t*)phr_bvh_internal_order(b->bvh)->ptr, n, (uint4*)b->faces->ptr, (float4*)b->tris->ptr);
-    if ((rc = enqueue_walk_records(g, b->bvh, &b->recs, b->tris)) != PHR_OK) return fail(rc);
+    if ((rc = enqueue_walk_records(g, b->bvh, &b->wide, nullptr, b->tris)) != PHR_OK) return fail(rc);
     std::vector<uint32_t> order(n);
     if (hipMemcpyAsync(order.data(), phr_bvh_internal_order(b->bvh)->ptr, 4ull * n, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
@@ -4849,8 +5021,8 @@ int phr_batch_new(phr_gpu* g, const void* tris_v, const uint32_t* seg_lo, uint32
         SceneDev& d = table[k];
         std::memset(&d, 0, sizeof d);
         d.nodes = (const float4*)phr_bvh_internal_nodes(b->bvh)->ptr;
-        d.recs = (const float4*)b->recs->ptr;
-        d.kids = d.recs + 4 * b->recs->len;
+        d.wide = (const float4*)b->wide->ptr;
+        d.recs = d.kids = nullptr;
         d.tris = (const float4*)b->tris->ptr;
         d.faces = (const uint4*)b->faces->ptr;
         d.verts = (const float4*)b->verts->ptr;
