@@ -447,17 +447,31 @@ __device__ __forceinline__ PhrHit walk_first(const SceneDev& s, V3 o, V3 d, floa
 }
 
 // A walk that can stop after any unit and go on later (the split build):
-// the ray, its best hit, the entry in hand (cur) and its stack (sp entries of
-// the thread's column). A unit is an inner node's visit or one triangle.
+// the ray, its best hit, the entry in hand (cur), a leaf put by (leaf) and its
+// stack (sp entries of the thread's column). A unit is an inner node's visit
+// or a leaf's triangles. A leaf reached is put by and the walk goes on from
+// the stack, until a second leaf is reached or nothing else is left.
 // `any`: a shadow ray's walk, which ends at the first triangle that blocks it.
 struct Walker {
     V3 o, inv;
     RaySpace rs;
     float t, u, v;  // closest: the nearest hit so far; shadow: t is the ray's length
-    uint32_t tri, cur, end, sp;
+    uint32_t tri, cur, leaf, sp;  // cur, leaf: PHR_NONE when there is none
     bool on, any;
 };
-__device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, V3 o, V3 d, float tmax, bool any) {
+__device__ __forceinline__ void walker_pop(Walker& w, const uint32_t* stk, uint32_t stride) {
+    w.cur = PHR_NONE;
+    if (w.sp != 0u) w.cur = stk[--w.sp * stride];
+}
+// A leaf in hand is put by if none is yet; a walk with nothing left ends.
+__device__ __forceinline__ void walker_settle(Walker& w, const uint32_t* stk, uint32_t stride) {
+    if (w.leaf == PHR_NONE && (w.cur & PHR_LEAF)) {
+        w.leaf = w.cur;
+        w.on = w.cur != PHR_NONE;
+        if (w.on) walker_pop(w, stk, stride);
+    }
+}
+__device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, uint32_t root, V3 o, V3 d, float tmax, bool any) {
     w.o = o;
     w.inv = safe_inv(d);
     w.rs = ray_space(d);
@@ -467,17 +481,45 @@ __device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, V3 o,
     w.sp = 0;
     w.any = any;
     w.on = true;
-    w.cur = wide_root(s, w.end);
+    const bool leaf = (root & PHR_LEAF) != 0u;
+    w.cur = leaf ? PHR_NONE : root;
+    w.leaf = leaf ? root : PHR_NONE;
 }
-__device__ __forceinline__ void walker_step(Walker& w, const SceneDev& s, uint32_t* stk, uint32_t stride, uint32_t& steps,
+__device__ __forceinline__ void walker_visit(Walker& w, const SceneDev& s, uint32_t* stk, uint32_t stride, uint32_t& steps,
+                                             uint32_t& tests) {
+    if (w.sp > WIDE_ROOM) {
+        PhrHit best{w.t, w.tri, w.u, w.v, 0u};
+        walk_nodes(s, w.o, w.inv, w.rs, w.any, best, stk, stride, tests);
+        w.t = best.t;
+        w.tri = best.tri;
+        w.u = best.u;
+        w.v = best.v;
+        w.on = false;
+        return;
+    }
+    ++steps;
+    if (!visit4(s, w.o, w.inv, w.t, w.cur, stk, stride, w.sp)) walker_pop(w, stk, stride);
+    walker_settle(w, stk, stride);
+}
+// The triangles of the leaf put by; `only`: the root's end where it is a leaf.
+__device__ __forceinline__ void walker_leaf(Walker& w, const SceneDev& s, uint32_t only, const uint32_t* stk, uint32_t stride,
                                             uint32_t& tests) {
-    if (w.cur & PHR_LEAF) {
-        const uint32_t id = w.cur & ~PHR_LEAF;
-        const float4 a = s.tris[3 * (size_t)id], b = s.tris[3 * (size_t)id + 1], c = s.tris[3 * (size_t)id + 2];
+    uint32_t id = w.leaf & ~PHR_LEAF;
+    float4 t0 = s.tris[3 * (size_t)id], t1 = s.tris[3 * (size_t)id + 1], t2 = s.tris[3 * (size_t)id + 2];
+    const uint32_t end = only != PHR_NONE ? only : __float_as_uint(t2.y);
+    w.leaf = PHR_NONE;
+    for (;;) {
         ++tests;
-        if (w.end == PHR_NONE) w.end = __float_as_uint(c.y);
+        // The leaf's next triangle is loaded while this one is tested.
+        const bool more = id + 1u < end;
+        float4 n0 = t0, n1 = t1, n2 = t2;
+        if (more) {
+            n0 = s.tris[3 * (size_t)(id + 1u)];
+            n1 = s.tris[3 * (size_t)(id + 1u) + 1];
+            n2 = s.tris[3 * (size_t)(id + 1u) + 2];
+        }
         float u, v;
-        const float t = tri_t(a, b, c, w.o, w.rs, u, v);
+        const float t = tri_t(t0, t1, t2, w.o, w.rs, u, v);
         if (w.any) {
             if (t < w.t && blocks(s, id)) {
                 w.tri = id;
@@ -490,28 +532,13 @@ __device__ __forceinline__ void walker_step(Walker& w, const SceneDev& s, uint32
             w.u = u;
             w.v = v;
         }
-        if (id + 1u < w.end) {
-            w.cur = (id + 1u) | PHR_LEAF;
-            return;
-        }
-        w.end = PHR_NONE;
-    } else if (w.sp > WIDE_ROOM) {
-        PhrHit best{w.t, w.tri, w.u, w.v, 0u};
-        walk_nodes(s, w.o, w.inv, w.rs, w.any, best, stk, stride, tests);
-        w.t = best.t;
-        w.tri = best.tri;
-        w.u = best.u;
-        w.v = best.v;
-        w.sp = 0;
-    } else {
-        ++steps;
-        if (visit4(s, w.o, w.inv, w.t, w.cur, stk, stride, w.sp)) return;
+        if (!more) break;
+        ++id;
+        t0 = n0;
+        t1 = n1;
+        t2 = n2;
     }
-    if (w.sp == 0) {
-        w.on = false;
-        return;
-    }
-    w.cur = stk[--w.sp * stride];
+    walker_settle(w, stk, stride);
 }
 
 // The walk records of a tree's nodes (one entry per node index; only inner
@@ -1935,22 +1962,38 @@ __global__ __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(W
 // before the walk: a sample that ended waits with its radiance both ways; a
 // sample that goes on is advanced as lit and, if the ray was blocked, gets
 // back the two sums that differ (the camera hit's light, the bounces' sum).
+// Leaves are tested once this many eighths of a wave's walks wait on one (of
+// 2 to 6, 3 was the fastest on the spheres frame, a tie with 4, and on the
+// cloud frame and the batch).
+constexpr uint32_t LEAF8 = 3u;
 // The split build's walk of one tree, or of a forest (F).
 template <bool F>
 struct SplitWalk {
     Walker w;
-    __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, s, o, d, tmax, any); }
+    uint32_t root, only;
+    __device__ __forceinline__ void scene(const SceneDev& s) { root = wide_root(s, only); }
+    __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, s, root, o, d, tmax, any); }
+    // The wave's next unit: the lanes at an inner node visit it while they are
+    // enough; once LEAF8 eighths of the walks have a leaf put by and nothing
+    // to visit, every lane with a leaf put by tests its triangles.
     __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t*, uint32_t& steps, uint32_t& tests) {
-        walker_step(w, s, stk, TRACE_THREADS, steps, tests);
+        const uint32_t on = (uint32_t)__popcll(__ballot(w.on));
+        const uint32_t stuck = (uint32_t)__popcll(__ballot(w.on && (w.cur & PHR_LEAF)));
+        if (8u * stuck >= LEAF8 * on) {
+            if (w.on && w.leaf != PHR_NONE) walker_leaf(w, s, only, stk, TRACE_THREADS, tests);
+        } else if (w.on && !(w.cur & PHR_LEAF)) {
+            walker_visit(w, s, stk, TRACE_THREADS, steps, tests);
+        }
     }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, 0u}; }
 };
 template <>
 struct SplitWalk<true> {
     ForestWalker w;
+    __device__ __forceinline__ void scene(const SceneDev&) {}
     __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { forest_begin(w, s, o, d, tmax, any); }
     __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t* tstk, uint32_t& steps, uint32_t& tests) {
-        forest_step(w, s, tstk, stk, TRACE_THREADS, steps, tests);
+        if (w.on) forest_step(w, s, tstk, stk, TRACE_THREADS, steps, tests);
     }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, w.hinst}; }
 };
@@ -1993,6 +2036,7 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
     st.min_pdf = 3.0e38f;
     RgGuide g0;  // what rg_start clears of a sample's guide (the first segment's rg_hit sets it anew)
     SplitWalk<F> sw;
+    sw.scene(sc);
     auto& w = sw.w;
     w.on = w.any = false;
     bool done = !inside || spp == 0u, pfinal = false;
@@ -2008,7 +2052,7 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
             const uint32_t waiting = (uint32_t)__popcll(__ballot(!done && !w.on));
             const uint32_t working = (uint32_t)__popcll(__ballot(!done));
             if (waiting == working || 8u * waiting >= shade8 * working) break;
-            if (w.on) sw.step(sc, stk, tstk, steps, tests);
+            sw.step(sc, stk, tstk, steps, tests);
         }
         if (done || w.on) continue;
         bool next = false;
