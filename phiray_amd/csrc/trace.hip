@@ -182,9 +182,16 @@ __device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float be
     cur = __float_as_uint(w0);
     return k0 < PHR_INF;
 }
-// A visit pushes up to three and stores one past what it pushes.
-constexpr uint32_t WIDE_ROOM = PHR_STACK - 3u;
+// The most entries a stack of `entries` may hold before a visit, which stores
+// at up to two past them.
+constexpr uint32_t wide_room(uint32_t entries) { return entries - 3u; }
 
+// The first slot of the tree under node x: its leftmost leaf's.
+__device__ __forceinline__ uint32_t first_slot(const SceneDev& s, uint32_t x) {
+    uint32_t w = __float_as_uint(s.nodes[2 * (size_t)x].w);
+    while (!(w & PHR_LEAF)) w = __float_as_uint(s.nodes[2 * (size_t)w].w);
+    return w & ~PHR_LEAF;
+}
 // Of two triangles (slots a and b) the ray meets at the same t, whether a
 // comes first in the binary walk: at the node where their ways part, the
 // nearer child does (a tie to the left); within a leaf, the lower slot.
@@ -194,13 +201,7 @@ __device__ __forceinline__ bool first_of(const SceneDev& s, V3 o, V3 inv, uint32
         const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
         const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
         if (l & PHR_LEAF) return a < b;
-        uint32_t y = r;  // the right child's first slot: its leftmost leaf's
-        uint32_t w = __float_as_uint(s.nodes[2 * (size_t)y].w);
-        while (!(w & PHR_LEAF)) {
-            y = w;
-            w = __float_as_uint(s.nodes[2 * (size_t)y].w);
-        }
-        const uint32_t split = w & ~PHR_LEAF;
+        const uint32_t split = first_slot(s, r);
         const bool a_left = a < split, b_left = b < split;
         if (a_left == b_left) {
             x = a_left ? l : r;
@@ -222,17 +223,30 @@ __device__ __forceinline__ bool blocks(const SceneDev& s, uint32_t id) {  // bvh
     return !(m[6] > 0.5f || m[3] < 0.5f);
 }
 
-// The rest of a walk whose stack has no room left (far deeper than any tree
-// measured: 13 of 32 entries at most on the benchmark scenes): the whole tree
-// again by the binary walk over the nodes, which holds one pending node a
-// level and so always fits, with the hit found so far.
-__device__ __forceinline__ void walk_nodes(const SceneDev& s, V3 o, V3 inv, const RaySpace& rs, bool any, PhrHit& best, uint32_t* stk,
-                                           uint32_t stride, uint32_t& tests) {
-    uint32_t sp = 0, x = s.root;
-    for (;;) {
-        const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
-        const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
-        if (l & PHR_LEAF) {
+// The rest of a walk whose stack has no room left (13 entries at most on the
+// benchmark scenes): the whole tree again by its nodes and without a stack,
+// leaf after leaf in slot order, each found from the root (a box the ray
+// misses skips its leaves), with the hit found so far.
+__device__ __forceinline__ uint32_t end_slot(const SceneDev& s, uint32_t x) {
+    while (!(__float_as_uint(s.nodes[2 * (size_t)x].w) & PHR_LEAF)) x = __float_as_uint(s.nodes[2 * (size_t)x + 1].w);
+    return __float_as_uint(s.nodes[2 * (size_t)x + 1].w);
+}
+__device__ __forceinline__ void walk_nodes(const SceneDev& s, V3 o, V3 inv, const RaySpace& rs, bool any, PhrHit& best, uint32_t& tests) {
+    const uint32_t last = end_slot(s, s.root);
+    for (uint32_t slot = first_slot(s, s.root); slot < last;) {
+        for (uint32_t x = s.root;;) {
+            const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
+            // One step past a hit: an equal t further on may come first.
+            const float far = best.tri != PHR_NONE && !any ? __uint_as_float(__float_as_uint(best.t) + 1u) : best.t;
+            if (box_t(lo, hi, o, inv, far) >= PHR_INF) {
+                slot = end_slot(s, x);
+                break;
+            }
+            const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
+            if (!(l & PHR_LEAF)) {
+                x = slot < first_slot(s, r) ? l : r;
+                continue;
+            }
             for (uint32_t id = l & ~PHR_LEAF; id < r; ++id) {
                 ++tests;
                 float u, v;
@@ -246,21 +260,9 @@ __device__ __forceinline__ void walk_nodes(const SceneDev& s, V3 o, V3 inv, cons
                     best = PhrHit{t, id, u, v, 0u};
                 }
             }
-        } else {
-            // One step past a hit: an equal t further on may come first.
-            const float far = best.tri != PHR_NONE && !any ? __uint_as_float(__float_as_uint(best.t) + 1u) : best.t;
-            const float tl = box_t(s.nodes[2 * (size_t)l], s.nodes[2 * (size_t)l + 1], o, inv, far);
-            const float tr = box_t(s.nodes[2 * (size_t)r], s.nodes[2 * (size_t)r + 1], o, inv, far);
-            const bool hl = tl < PHR_INF, hr = tr < PHR_INF;
-            if (hl || hr) {
-                const bool left = hl && (!hr || tl <= tr);
-                if (hl && hr) stk[sp++ * stride] = left ? r : l;
-                x = left ? l : r;
-                continue;
-            }
+            slot = r;
+            break;
         }
-        if (sp == 0) return;
-        x = stk[--sp * stride];
     }
 }
 
@@ -311,8 +313,8 @@ __device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax
                 t1 = n1;
                 t2 = n2;
             }
-        } else if (sp > WIDE_ROOM) {
-            walk_nodes(s, o, inv, rs, ANY, best, stk, stride, tests);
+        } else if (sp > wide_room(PHR_STACK)) {
+            walk_nodes(s, o, inv, rs, ANY, best, tests);
             break;
         } else {
             ++steps;
@@ -485,11 +487,11 @@ __device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, uint3
     w.cur = leaf ? PHR_NONE : root;
     w.leaf = leaf ? root : PHR_NONE;
 }
-__device__ __forceinline__ void walker_visit(Walker& w, const SceneDev& s, uint32_t* stk, uint32_t stride, uint32_t& steps,
-                                             uint32_t& tests) {
-    if (w.sp > WIDE_ROOM) {
+__device__ __forceinline__ void walker_visit(Walker& w, const SceneDev& s, uint32_t* stk, uint32_t stride, uint32_t entries,
+                                             uint32_t& steps, uint32_t& tests) {
+    if (w.sp > wide_room(entries)) {
         PhrHit best{w.t, w.tri, w.u, w.v, 0u};
-        walk_nodes(s, w.o, w.inv, w.rs, w.any, best, stk, stride, tests);
+        walk_nodes(s, w.o, w.inv, w.rs, w.any, best, tests);
         w.t = best.t;
         w.tri = best.tri;
         w.u = best.u;
@@ -926,6 +928,9 @@ constexpr uint32_t TRACE_THREADS = 256;
 // waves) and nearly all of a 1024 x 1024 raycast.
 constexpr uint32_t COUNT_SLOTS = 256, COUNT_WORDS = 8;
 constexpr size_t COUNT_BYTES = 8ull * COUNT_SLOTS * COUNT_WORDS;
+// After them the split build's queues: pixels handed out (a word a scene of a
+// batch) and waves done.
+constexpr size_t COUNT_ALLOC = COUNT_BYTES + 64;
 __device__ __forceinline__ void add_counts(unsigned long long* __restrict__ rays, unsigned long long closest, unsigned long long shadow,
                                            unsigned long long steps, unsigned long long tests) {
     unsigned long long* c = rays + COUNT_WORDS * (blockIdx.x % COUNT_SLOTS);
@@ -1986,6 +1991,46 @@ __global__ __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(W
 // 2 to 6, 3 was the fastest on the spheres frame, a tie with 4, and on the
 // cloud frame and the batch).
 constexpr uint32_t LEAF8 = 3u;
+// A block of the split build is one wave: it leaves as soon as it is done.
+constexpr uint32_t SPLIT_THREADS = 64;
+// A pixel's sums while its samples run. One tree: in the lane's LDS column (13
+// of the 40 words a lane has at 4 waves a SIMD; the walk's stack has the rest),
+// so that no register holds them through the walks. A forest's two stacks
+// leave no room: registers.
+constexpr uint32_t SUM_WORDS = 13;
+template <int WPE>
+constexpr uint32_t split_stack() { return WPE >= 5 ? 32u - SUM_WORDS : 40u - SUM_WORDS; }
+template <bool F>
+struct PixelSums {
+    float* c;
+    __device__ __forceinline__ V3 at3(uint32_t k) const { return v3(c[k * SPLIT_THREADS], c[(k + 1) * SPLIT_THREADS], c[(k + 2) * SPLIT_THREADS]); }
+    __device__ __forceinline__ void put3(uint32_t k, V3 v) { c[k * SPLIT_THREADS] = v.x; c[(k + 1) * SPLIT_THREADS] = v.y; c[(k + 2) * SPLIT_THREADS] = v.z; }
+    __device__ __forceinline__ float at(uint32_t k) const { return c[k * SPLIT_THREADS]; }
+    __device__ __forceinline__ void put(uint32_t k, float v) { c[k * SPLIT_THREADS] = v; }
+};
+template <>
+struct PixelSums<true> {
+    float r[SUM_WORDS];
+    __device__ __forceinline__ V3 at3(uint32_t k) const { return v3(r[k], r[k + 1], r[k + 2]); }
+    __device__ __forceinline__ void put3(uint32_t k, V3 v) { r[k] = v.x; r[k + 1] = v.y; r[k + 2] = v.z; }
+    __device__ __forceinline__ float at(uint32_t k) const { return r[k]; }
+    __device__ __forceinline__ void put(uint32_t k, float v) { r[k] = v; }
+};
+enum : uint32_t { SUM_L = 0, SUM_ALB = 3, SUM_NRM = 6, SUM_DEP = 9, SUM_COV = 10, SUM_MISS = 11, SUM_OUTLINE = 12 };
+
+// The pixels a wave works on, by id (256 to a 16 x 16 tile, 64 to an 8 x 8
+// block of it): `given` from `first`, then, up to `hi`, the 64s that `next`
+// hands out from `base` on (an add a pixel block: fewer would leave the last
+// waves longer, more would wait on one another at 12 ns an add).
+struct PathWork {
+    uint32_t first, given, base, hi;
+    uint32_t* next;
+};
+// A wave takes new pixels once this many of its lanes have none (1080p 16-spp
+// spheres frame, ms: 4 lanes 23.7, 6 23.7, 8 24.0, 12 24.4, 16 24.7, 32 26.5; a
+// 32-scene batch: 22.6, 22.7, 22.2, 22.2; 720p 1-spp: 8 the least).
+constexpr uint32_t REFILL = 8u;
+
 // The split build's walk of one tree, or of a forest (F).
 template <bool F>
 struct SplitWalk {
@@ -1996,13 +2041,14 @@ struct SplitWalk {
     // The wave's next unit: the lanes at an inner node visit it while they are
     // enough; once LEAF8 eighths of the walks have a leaf put by and nothing
     // to visit, every lane with a leaf put by tests its triangles.
+    template <uint32_t STK>
     __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t*, uint32_t& steps, uint32_t& tests) {
         const uint32_t on = (uint32_t)__popcll(__ballot(w.on));
         const uint32_t stuck = (uint32_t)__popcll(__ballot(w.on && (w.cur & PHR_LEAF)));
         if (8u * stuck >= LEAF8 * on) {
-            if (w.on && w.leaf != PHR_NONE) walker_leaf(w, s, only, stk, TRACE_THREADS, tests);
+            if (w.on && w.leaf != PHR_NONE) walker_leaf(w, s, only, stk, SPLIT_THREADS, tests);
         } else if (w.on && !(w.cur & PHR_LEAF)) {
-            walker_visit(w, s, stk, TRACE_THREADS, steps, tests);
+            walker_visit(w, s, stk, SPLIT_THREADS, STK, steps, tests);
         }
     }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, 0u}; }
@@ -2012,40 +2058,33 @@ struct SplitWalk<true> {
     ForestWalker w;
     __device__ __forceinline__ void scene(const SceneDev&) {}
     __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { forest_begin(w, s, o, d, tmax, any); }
+    template <uint32_t STK>
     __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t* tstk, uint32_t& steps, uint32_t& tests) {
-        if (w.on) forest_step(w, s, tstk, stk, TRACE_THREADS, steps, tests);
+        if (w.on) forest_step(w, s, tstk, stk, SPLIT_THREADS, steps, tests);
     }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, w.hinst}; }
 };
 
-// path_split: tile `blk` of one image. s_stack: the block's stack columns
-// (a forest's mesh trees'); s_tstack: a forest's top-tree columns.
-template <bool F = false>
-__device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* __restrict__ camp, uint32_t blk, uint32_t tiles_x,
+// path_split: a wave's share of one image. s_stack: the wave's stack columns
+// (a forest's mesh trees'); s_tstack: a forest's top-tree columns; s_sum: one
+// tree's sums.
+// A lane whose pixel has all its samples takes another: pixels differ in
+// length (one that sees the sky ends at once), and a wave that kept its 64 to
+// the end had 47 of its lanes at work on the 1.31M-triangle frame.
+template <bool F, uint32_t STK>
+__device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* __restrict__ camp, const PathWork& work, uint32_t tiles_x,
                                            uint32_t frame0, uint32_t spp, uint32_t* __restrict__ px,
-                                           unsigned long long* __restrict__ rays, uint32_t* s_stack, uint16_t* s_tstack,
+                                           unsigned long long* __restrict__ rays, uint32_t* s_stack, uint16_t* s_tstack, float* s_sum,
                                            uint32_t shade8) {
     const PhrCamera* p = camp;
     const size_t n = (size_t)p->w * p->h;
-    const uint32_t tx = blk % tiles_x, ty = blk / tiles_x;
-    const uint32_t pxl = tx * 16 + (threadIdx.x & 15u), pyl = ty * 16 + (threadIdx.x >> 4);
-    const bool inside = pxl < p->w && pyl < p->h;
-    const uint32_t i = pyl * p->w + pxl;
-    uint32_t* stk = s_stack + threadIdx.x;
-    uint16_t* tstk = F ? s_tstack + threadIdx.x : nullptr;
+    const uint32_t lane = threadIdx.x;
+    uint32_t* stk = s_stack + lane;
+    uint16_t* tstk = F ? s_tstack + lane : nullptr;
+    PixelSums<F> sum;
+    if constexpr (!F) sum.c = s_sum + lane;
     uint32_t closest = 0, shadow = 0, steps = 0, tests = 0;
     const bool keep = frame0 > 0u;
-    V3 l = v3(0, 0, 0), ga = l, gn = l;
-    float gd = 0.f, cov = 0.f, gone = 0.f;
-    if (inside && keep) {
-        l = v3(ldf(px, n + 3 * i), ldf(px, n + 3 * i + 1), ldf(px, n + 3 * i + 2));
-        ga = v3(ldf(px, 7 * n + 3 * i), ldf(px, 7 * n + 3 * i + 1), ldf(px, 7 * n + 3 * i + 2));
-        gn = v3(ldf(px, 10 * n + 3 * i), ldf(px, 10 * n + 3 * i + 1), ldf(px, 10 * n + 3 * i + 2));
-        gd = ldf(px, 13 * n + i);
-        cov = ldf(px, 23 * n + i);
-        gone = ldf(px, 33 * n + i);
-    }
-    uint32_t outline = 0;
     const RgConst k = rg_const(p);
     RgSample st;
     st.seed = 0;
@@ -2059,27 +2098,89 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
     sw.scene(sc);
     auto& w = sw.w;
     w.on = w.any = false;
-    bool done = !inside || spp == 0u, pfinal = false;
+    bool pfinal = false;
     V3 pa = v3(0, 0, 0), pb = pa;  // what a shadow walk's answer picks between
-    uint32_t s = 0;
-    if (!done) {
-        rg_start(st, g0, p, i, frame0);
-        sw.begin(sc, st.o, st.d, PHR_INF, false);
-        ++closest;
-    }
-    while (__ballot(!done) != 0ull) {
-        for (;;) {  // walk until shade8 / 8 of the lanes at work wait to shade, or all do
-            const uint32_t waiting = (uint32_t)__popcll(__ballot(!done && !w.on));
-            const uint32_t working = (uint32_t)__popcll(__ballot(!done));
-            if (waiting == working || 8u * waiting >= shade8 * working) break;
-            sw.step(sc, stk, tstk, steps, tests);
+    uint32_t s = 0, i = 0;
+    bool live = false, full = false;  // the lane has a pixel; its pixel has every sample and waits to be written
+    uint32_t at = work.first, end = min(at + work.given, work.hi);  // the wave's ids in hand
+    bool drained = false;  // no ids are left to take
+    for (;;) {
+        const uint64_t lv = __ballot(live);
+        const uint32_t idle = 64u - (uint32_t)__popcll(lv);
+        if (lv == 0ull || (!drained && idle >= REFILL)) {
+            if (full) {
+                full = false;
+                const V3 l = sum.at3(SUM_L), ga = sum.at3(SUM_ALB), gn = sum.at3(SUM_NRM);
+                const float cov = sum.at(SUM_COV), gone = sum.at(SUM_MISS);
+                V3 gs = keep ? v3(ldf(px, 20 * n + 3 * i), ldf(px, 20 * n + 3 * i + 1), ldf(px, 20 * n + 3 * i + 2)) : v3(0, 0, 0);
+                float film = keep ? ldf(px, 24 * n + i) : 0.f;
+                const uint32_t taken = (keep ? px[31 * n + i] : 0u) + spp;
+                for (uint32_t kk = 0; kk < spp; ++kk) {
+                    gs = gs + v3(0.f, 0.f, 0.f);
+                    film = film + 1.0f;
+                }
+                if (frame0 == 0u) { px[29 * n + i] = 0u; px[30 * n + i] = 0u; }
+                stf(px, n + 3 * i, l.x); stf(px, n + 3 * i + 1, l.y); stf(px, n + 3 * i + 2, l.z);
+                stf(px, 7 * n + 3 * i, ga.x); stf(px, 7 * n + 3 * i + 1, ga.y); stf(px, 7 * n + 3 * i + 2, ga.z);
+                stf(px, 10 * n + 3 * i, gn.x); stf(px, 10 * n + 3 * i + 1, gn.y); stf(px, 10 * n + 3 * i + 2, gn.z);
+                stf(px, 13 * n + i, sum.at(SUM_DEP));
+                stf(px, 20 * n + 3 * i, gs.x); stf(px, 20 * n + 3 * i + 1, gs.y); stf(px, 20 * n + 3 * i + 2, gs.z);
+                stf(px, 23 * n + i, cov);
+                stf(px, 24 * n + i, film);
+                px[25 * n + i] = __float_as_uint(sum.at(SUM_OUTLINE));
+                px[31 * n + i] = taken;
+                stf(px, 33 * n + i, gone);
+                put_shown(px, n, i, *p, l, gs, cov, gone, film, taken);
+            }
+            if (drained) break;  // and no lane has a pixel
+            if (at == end) {  // the queue's next 64
+                uint32_t q = 0;
+                if (lane == 0u) q = atomicAdd(work.next, SPLIT_THREADS);
+                at = min(work.base + (uint32_t)__builtin_amdgcn_readfirstlane((int)q), work.hi);
+                end = min(at + SPLIT_THREADS, work.hi);
+            }
+            const uint32_t got = min(idle, end - at);
+            const uint32_t rank = (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(~lv >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)~lv, 0u));
+            if (!live && rank < got) {
+                const uint32_t id = at + rank;
+                const uint32_t tile = id >> 8, tx = tile % tiles_x, ty = tile / tiles_x;
+                const uint32_t x = tx * 16u + ((id >> 6) & 1u) * 8u + (id & 7u), y = ty * 16u + ((id >> 7) & 1u) * 8u + ((id >> 3) & 7u);
+                live = x < p->w && y < p->h;
+                if (live) {
+                    i = y * p->w + x;
+                    s = 0;
+                    st.phase = 0u;
+                    if (keep) {
+                        sum.put3(SUM_L, v3(ldf(px, n + 3 * i), ldf(px, n + 3 * i + 1), ldf(px, n + 3 * i + 2)));
+                        sum.put3(SUM_ALB, v3(ldf(px, 7 * n + 3 * i), ldf(px, 7 * n + 3 * i + 1), ldf(px, 7 * n + 3 * i + 2)));
+                        sum.put3(SUM_NRM, v3(ldf(px, 10 * n + 3 * i), ldf(px, 10 * n + 3 * i + 1), ldf(px, 10 * n + 3 * i + 2)));
+                        sum.put(SUM_DEP, ldf(px, 13 * n + i));
+                        sum.put(SUM_COV, ldf(px, 23 * n + i));
+                        sum.put(SUM_MISS, ldf(px, 33 * n + i));
+                    } else {
+                        for (uint32_t kk = 0; kk < SUM_OUTLINE; ++kk) sum.put(kk, 0.f);
+                    }
+                    sum.put(SUM_OUTLINE, 0.f);
+                    rg_start(st, g0, p, i, frame0);
+                    sw.begin(sc, st.o, st.d, PHR_INF, false);
+                    ++closest;
+                }
+            }
+            at += got;
+            drained = at == end && end == work.hi;
+            continue;
         }
-        if (done || w.on) continue;
+        for (;;) {  // walk until shade8 / 8 of the lanes at work wait to shade, or all do
+            const uint32_t working = (uint32_t)__popcll(lv), waiting = working - (uint32_t)__popcll(__ballot(w.on));
+            if (waiting == working || 8u * waiting >= shade8 * working) break;
+            sw.template step<STK>(sc, stk, tstk, steps, tests);
+        }
+        if (!live || w.on) continue;
         bool next = false;
         if (w.any) {  // the turn's shadow ray has its answer
             const bool blocked = w.tri != PHR_NONE;
             if (pfinal) {
-                l = l + (blocked ? pb : pa);
+                sum.put3(SUM_L, sum.at3(SUM_L) + (blocked ? pb : pa));
             } else if (blocked) {
                 st.cc = pa;
                 st.acc = pb;
@@ -2095,12 +2196,12 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
             RgGuide g{v3(0, 0, 0), v3(0, 0, 0), 0.f, 0.f, 0.f, 0u};
             rg_hit<F>(st, g, q, sc, p, k, h);
             if (first) {  // shade's `out`, summed as path_block sums it
-                ga = ga + g.alb;
-                gn = gn + g.nrm;
-                gd = gd + g.dep;
-                gone = gone + g.missed;
-                cov = cov + g.cov;
-                outline = g.outline;
+                sum.put3(SUM_ALB, sum.at3(SUM_ALB) + g.alb);
+                sum.put3(SUM_NRM, sum.at3(SUM_NRM) + g.nrm);
+                sum.put(SUM_DEP, sum.at(SUM_DEP) + g.dep);
+                sum.put(SUM_MISS, sum.at(SUM_MISS) + g.missed);
+                sum.put(SUM_COV, sum.at(SUM_COV) + g.cov);
+                sum.put(SUM_OUTLINE, __uint_as_float(g.outline));
             }
             bool ended;
             if (q.qon) {
@@ -2123,7 +2224,7 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
                 ++shadow;
             } else {
                 ended = rg_post(st, q, p, 1.0f);
-                if (ended) l = l + st.col;
+                if (ended) sum.put3(SUM_L, sum.at3(SUM_L) + st.col);
                 next = true;
             }
             if (ended) {
@@ -2137,31 +2238,10 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
                 sw.begin(sc, st.o, st.d, PHR_INF, false);
                 ++closest;
             } else {
-                done = true;
+                live = false;
+                full = true;
             }
         }
-    }
-    if (inside) {
-        V3 gs = keep ? v3(ldf(px, 20 * n + 3 * i), ldf(px, 20 * n + 3 * i + 1), ldf(px, 20 * n + 3 * i + 2)) : v3(0, 0, 0);
-        float film = keep ? ldf(px, 24 * n + i) : 0.f;
-        uint32_t taken = keep ? px[31 * n + i] : 0u;
-        for (uint32_t kk = 0; kk < spp; ++kk) {
-            gs = gs + v3(0.f, 0.f, 0.f);
-            film = film + 1.0f;
-        }
-        taken = taken + spp;
-        if (frame0 == 0u) { px[29 * n + i] = 0u; px[30 * n + i] = 0u; }
-        stf(px, n + 3 * i, l.x); stf(px, n + 3 * i + 1, l.y); stf(px, n + 3 * i + 2, l.z);
-        stf(px, 7 * n + 3 * i, ga.x); stf(px, 7 * n + 3 * i + 1, ga.y); stf(px, 7 * n + 3 * i + 2, ga.z);
-        stf(px, 10 * n + 3 * i, gn.x); stf(px, 10 * n + 3 * i + 1, gn.y); stf(px, 10 * n + 3 * i + 2, gn.z);
-        stf(px, 13 * n + i, gd);
-        stf(px, 20 * n + 3 * i, gs.x); stf(px, 20 * n + 3 * i + 1, gs.y); stf(px, 20 * n + 3 * i + 2, gs.z);
-        stf(px, 23 * n + i, cov);
-        stf(px, 24 * n + i, film);
-        px[25 * n + i] = outline;
-        px[31 * n + i] = taken;
-        stf(px, 33 * n + i, gone);
-        put_shown(px, n, i, *p, l, gs, cov, gone, film, taken);
     }
     unsigned long long rc = closest, rs = shadow, st_ = steps, tt = tests;
     for (int kk = 32; kk > 0; kk >>= 1) {
@@ -2170,26 +2250,45 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
         st_ += __shfl_xor(st_, kk);
         tt += __shfl_xor(tt, kk);
     }
-    if ((threadIdx.x & 63) == 0 && (rc | rs)) {
+    if (lane == 0u && (rc | rs)) {
         add_counts(rays, rc, rs, st_, tt);
     }
 }
+// A frame's waves: `tiles` tiles from tile0, by the queue behind the counters.
+// The last wave to end clears it for the next launch.
+__device__ __forceinline__ PathWork split_work(unsigned long long* rays, uint32_t tile0, uint32_t tiles) {
+    const uint32_t lo = tile0 * 256u;
+    return PathWork{lo + blockIdx.x * SPLIT_THREADS, SPLIT_THREADS, lo + gridDim.x * SPLIT_THREADS, lo + tiles * 256u,
+                    (uint32_t*)(rays + COUNT_SLOTS * COUNT_WORDS)};
+}
+__device__ __forceinline__ void split_done(const PathWork& work) {
+    if (threadIdx.x != 0u) return;
+    if (atomicAdd(work.next + 1, 1u) + 1u == gridDim.x) {
+        atomicExch(work.next, 0u);
+        atomicExch(work.next + 1, 0u);
+    }
+}
 template <int WPE>
-__global__ __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_sw(
+__global__ __launch_bounds__(SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_sw(
     SceneDev sc, const PhrCamera* __restrict__ camp, uint32_t tiles_x, uint32_t frame0, uint32_t spp, uint32_t* __restrict__ px,
-    unsigned long long* __restrict__ rays, uint32_t tile0, uint32_t shade8) {
-    __shared__ uint32_t s_stack[PHR_STACK * TRACE_THREADS];
-    path_split(sc, camp, blockIdx.x + tile0, tiles_x, frame0, spp, px, rays, s_stack, nullptr, shade8);
+    unsigned long long* __restrict__ rays, uint32_t tile0, uint32_t tiles, uint32_t shade8) {
+    __shared__ uint32_t s_stack[split_stack<WPE>() * SPLIT_THREADS];
+    __shared__ float s_sum[SUM_WORDS * SPLIT_THREADS];
+    const PathWork work = split_work(rays, tile0, tiles);
+    path_split<false, split_stack<WPE>()>(sc, camp, work, tiles_x, frame0, spp, px, rays, s_stack, nullptr, s_sum, shade8);
+    split_done(work);
 }
 // The split build over a forest: MSTK mesh-tree entries a thread (the
 // caller checked the mesh trees' depth when it is below PHR_STACK).
 template <int WPE, uint32_t MSTK>
-__global__ __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_sw_forest(
+__global__ __launch_bounds__(SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_sw_forest(
     SceneDev sc, const PhrCamera* __restrict__ camp, uint32_t tiles_x, uint32_t frame0, uint32_t spp, uint32_t* __restrict__ px,
-    unsigned long long* __restrict__ rays, uint32_t tile0, uint32_t shade8) {
-    __shared__ uint32_t s_stack[MSTK * TRACE_THREADS];
-    __shared__ uint16_t s_tstack[PHR_STACK * TRACE_THREADS];
-    path_split<true>(sc, camp, blockIdx.x + tile0, tiles_x, frame0, spp, px, rays, s_stack, s_tstack, shade8);
+    unsigned long long* __restrict__ rays, uint32_t tile0, uint32_t tiles, uint32_t shade8) {
+    __shared__ uint32_t s_stack[MSTK * SPLIT_THREADS];
+    __shared__ uint16_t s_tstack[PHR_STACK * SPLIT_THREADS];
+    const PathWork work = split_work(rays, tile0, tiles);
+    path_split<true, MSTK>(sc, camp, work, tiles_x, frame0, spp, px, rays, s_stack, s_tstack, nullptr, shade8);
+    split_done(work);
 }
 
 // ---- the wavefront build --------------------------------------------------------
@@ -2446,8 +2545,8 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                     best = PhrHit{t, id, u, v, 0u};
                 }
             } while (++id < end);
-        } else if (sp > WIDE_ROOM) {
-            walk_nodes(sc, o, inv, rs, ANY, best, stk, WF_THREADS, tests);
+        } else if (sp > wide_room(PHR_STACK)) {
+            walk_nodes(sc, o, inv, rs, ANY, best, tests);
             more = false;
         } else {
             ++steps;
@@ -2661,23 +2760,33 @@ __global__ __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(W
     path_block<false>(sc, cams + scene, tile, tiles_x, 0u, spp, px + px_stride * scene, rays, 0u, s_stack, s_tstack);
 }
 // The same batch with the split build's samples (path_split): for cameras
-// with lamps or a lit world and no Adaptive Sampling.
+// with lamps or a lit world and no Adaptive Sampling. As many waves as the GPU
+// holds at once; each takes pixels of one scene from that scene's queue until
+// it is drained, then of the next: of its XCD's scenes in turn (`grouped`),
+// then of the other XCDs', or of all scenes from its own on.
 template <int WPE>
-__global__ __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_batch_sw(
-    const SceneDev* __restrict__ scenes, const PhrCamera* __restrict__ cams, uint32_t tiles, uint32_t tiles_x, uint32_t spp,
-    uint32_t* __restrict__ px, uint64_t px_stride, unsigned long long* __restrict__ rays, uint32_t grouped, uint32_t shade8) {
-    __shared__ uint32_t s_stack[PHR_STACK * TRACE_THREADS];
-    uint32_t scene, tile;
-    if (grouped) {
-        const uint32_t x = blockIdx.x % 8u, q = blockIdx.x / 8u;
-        scene = x + 8u * (q / tiles);
-        tile = q % tiles;
-    } else {
-        scene = blockIdx.x / tiles;
-        tile = blockIdx.x % tiles;
+__global__ __launch_bounds__(SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_batch_sw(
+    const SceneDev* __restrict__ scenes, const PhrCamera* __restrict__ cams, uint32_t nscenes, uint32_t tiles, uint32_t tiles_x,
+    uint32_t spp, uint32_t* __restrict__ px, uint64_t px_stride, unsigned long long* __restrict__ rays, uint32_t grouped,
+    uint32_t shade8) {
+    __shared__ uint32_t s_stack[split_stack<WPE>() * SPLIT_THREADS];
+    __shared__ float s_sum[SUM_WORDS * SPLIT_THREADS];
+    uint32_t* queue = (uint32_t*)(rays + COUNT_SLOTS * COUNT_WORDS);  // waves done, then a word a scene
+    const uint32_t per = grouped ? nscenes / 8u : nscenes;  // scenes a group
+    const uint32_t group = grouped ? blockIdx.x % 8u : 0u, own = (grouped ? blockIdx.x / 8u : blockIdx.x) % per;
+    for (uint32_t t = 0; t < nscenes; ++t) {
+        const uint32_t scene = grouped ? (group + t / per) % 8u + 8u * ((own + t) % per) : (own + t) % per;
+        const uint32_t taken = __hip_atomic_load(queue + 1 + scene, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane((int)(taken >= tiles * 256u))) continue;
+        const SceneDev sc = scenes[scene];
+        const PathWork work{0u, 0u, 0u, tiles * 256u, queue + 1 + scene};
+        path_split<false, split_stack<WPE>()>(sc, cams + scene, work, tiles_x, 0u, spp, px + px_stride * scene, rays, s_stack, nullptr,
+                                              s_sum, shade8);
     }
-    const SceneDev sc = scenes[scene];
-    path_split(sc, cams + scene, tile, tiles_x, 0u, spp, px + px_stride * scene, rays, s_stack, nullptr, shade8);
+    uint32_t last = 0;
+    if (threadIdx.x == 0u) last = atomicAdd(queue, 1u) + 1u == gridDim.x ? 1u : 0u;
+    if (__builtin_amdgcn_readfirstlane((int)last))  // clear the queues for the next launch
+        for (uint32_t k = threadIdx.x; k < nscenes + 1u; k += SPLIT_THREADS) atomicExch(queue + k, 0u);
 }
 
 // The builds of the path kernels the tracer and the batch choose among.
@@ -2697,28 +2806,30 @@ bool regen_allowed(const PhrCamera& cam) {
 // checks the camera).
 // short_stack: the forest's 3-wave build with FOREST_SHORT_STACK mesh-tree
 // entries (the caller checked the mesh trees' depth).
-void launch_path(uint32_t waves, bool forest, uint32_t regen, dim3 grid, hipStream_t s, const SceneDev& sc, const PhrCamera* cp,
-                 uint32_t tiles_x, uint32_t f0, uint32_t spp, uint32_t* px, unsigned long long* rays, uint32_t listed,
+void launch_path(phr_gpu* g, uint32_t waves, bool forest, uint32_t regen, dim3 grid, hipStream_t s, const SceneDev& sc,
+                 const PhrCamera* cp, uint32_t tiles_x, uint32_t f0, uint32_t spp, uint32_t* px, unsigned long long* rays, uint32_t listed,
                  uint32_t tile0, bool short_stack = false, uint32_t shade8 = 4) {
     const dim3 block(TRACE_THREADS);
-    if (regen == 3u && !forest && !listed) {
-        if (waves == 5)
-            hipLaunchKernelGGL(k_path_sw<5>, grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-        else if (waves == 4)
-            hipLaunchKernelGGL(k_path_sw<4>, grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-        else if (waves == 3)
-            hipLaunchKernelGGL(k_path_sw<3>, grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-        else
-            hipLaunchKernelGGL(k_path_sw<2>, grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-    } else if (regen == 3u && forest && !listed) {  // the caller checked the mesh trees' depth for the short stacks
-        if (waves >= 4)
-            hipLaunchKernelGGL((k_path_sw_forest<4, FOREST_SHORT_STACK>), grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-        else if (waves == 3 && short_stack)
-            hipLaunchKernelGGL((k_path_sw_forest<3, FOREST_SHORT_STACK>), grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-        else if (waves == 3)
-            hipLaunchKernelGGL((k_path_sw_forest<3, PHR_STACK>), grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
-        else
-            hipLaunchKernelGGL((k_path_sw_forest<2, PHR_STACK>), grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, shade8);
+    if (regen == 3u && !listed) {
+        // As many waves as the GPU holds at once (fewer where that many have
+        // no 64 pixels each): they share the launch's pixels out by a queue.
+        const uint32_t fit = forest ? std::min(waves, 4u) : waves;
+        const uint32_t resident = (uint32_t)std::max(g->cu_count, 1) * 4u * fit;
+        const dim3 wgrid(std::min(grid.x * (256u / SPLIT_THREADS), resident)), wblock(SPLIT_THREADS);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, wgrid, wblock, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0, grid.x, shade8);
+        };
+        if (!forest) {
+            if (waves == 5) go(k_path_sw<5>);
+            else if (waves == 4) go(k_path_sw<4>);
+            else if (waves == 3) go(k_path_sw<3>);
+            else go(k_path_sw<2>);
+        } else {  // the caller checked the mesh trees' depth for the short stacks
+            if (waves >= 4) go(k_path_sw_forest<4, FOREST_SHORT_STACK>);
+            else if (waves == 3 && short_stack) go(k_path_sw_forest<3, FOREST_SHORT_STACK>);
+            else if (waves == 3) go(k_path_sw_forest<3, PHR_STACK>);
+            else go(k_path_sw_forest<2, PHR_STACK>);
+        }
     } else if (regen && !forest && !listed) {
         if (waves == 5)
             hipLaunchKernelGGL(k_path_rg<5>, grid, block, 0, s, sc, cp, tiles_x, f0, spp, px, rays, tile0);
@@ -2748,19 +2859,20 @@ void launch_path(uint32_t waves, bool forest, uint32_t regen, dim3 grid, hipStre
 
 // split: the split build (k_path_batch_sw, shading at shade8 eighths), else
 // the nested one.
-void launch_path_batch(uint32_t waves, bool split, dim3 grid, hipStream_t s, const SceneDev* table, const PhrCamera* cams,
-                       uint32_t tiles, uint32_t tiles_x, uint32_t spp, uint32_t* px, uint64_t stride, unsigned long long* rays,
-                       uint32_t grouped, uint32_t shade8) {
-    const dim3 block(TRACE_THREADS);
+void launch_path_batch(phr_gpu* g, uint32_t waves, bool split, uint32_t scenes, hipStream_t s, const SceneDev* table,
+                       const PhrCamera* cams, uint32_t tiles, uint32_t tiles_x, uint32_t spp, uint32_t* px, uint64_t stride,
+                       unsigned long long* rays, uint32_t grouped, uint32_t shade8) {
+    const dim3 block(TRACE_THREADS), grid(tiles * scenes);
     if (split) {
-        if (waves == 5)
-            hipLaunchKernelGGL(k_path_batch_sw<5>, grid, block, 0, s, table, cams, tiles, tiles_x, spp, px, stride, rays, grouped, shade8);
-        else if (waves == 4)
-            hipLaunchKernelGGL(k_path_batch_sw<4>, grid, block, 0, s, table, cams, tiles, tiles_x, spp, px, stride, rays, grouped, shade8);
-        else if (waves == 3)
-            hipLaunchKernelGGL(k_path_batch_sw<3>, grid, block, 0, s, table, cams, tiles, tiles_x, spp, px, stride, rays, grouped, shade8);
-        else
-            hipLaunchKernelGGL(k_path_batch_sw<2>, grid, block, 0, s, table, cams, tiles, tiles_x, spp, px, stride, rays, grouped, shade8);
+        const uint32_t resident = (uint32_t)std::max(g->cu_count, 1) * 4u * waves;
+        const dim3 wgrid(std::min(tiles * scenes * (256u / SPLIT_THREADS), resident)), wblock(SPLIT_THREADS);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, wgrid, wblock, 0, s, table, cams, scenes, tiles, tiles_x, spp, px, stride, rays, grouped, shade8);
+        };
+        if (waves == 5) go(k_path_batch_sw<5>);
+        else if (waves == 4) go(k_path_batch_sw<4>);
+        else if (waves == 3) go(k_path_batch_sw<3>);
+        else go(k_path_batch_sw<2>);
     } else if (waves == 5)
         hipLaunchKernelGGL(k_path_batch<5>, grid, block, 0, s, table, cams, tiles, tiles_x, spp, px, stride, rays, grouped);
     else if (waves == 4)
@@ -2936,11 +3048,13 @@ phr_array* phr_bvh_internal_order(phr_bvh* b);
 const uint8_t* phr_bvh_internal_inner(phr_bvh* b);
 
 // The walk records of a built tree (after its gather wrote the triangle
-// cache): the wide ones into `wide` and, where `recs` is given, the ordered
-// any-hit walk's into it; each allocated on first use.
+// cache): the wide ones into `wide` and, where `recs` is given (one tree), the
+// ordered any-hit walk's into it; each allocated on first use.
 static int enqueue_walk_records(phr_gpu* g, phr_bvh* bvh, phr_array** wide, phr_array** recs, phr_array* tris) {
     phr_array* nodes = phr_bvh_internal_nodes(bvh);
-    const uint64_t count = nodes->len;
+    // The inner nodes of one tree come before its leaves; a batch's trees lie
+    // one after another.
+    const uint64_t count = recs ? (nodes->len + 1) / 2 : nodes->len;
     if (!*wide) {
         int rc = phr_array_alloc(g, 16 * WIDE_ROWS, std::max<uint64_t>(count, 1), wide);
         if (rc != PHR_OK) return rc;
@@ -3650,7 +3764,7 @@ int phr_tracer_new(phr_gpu* g, const void* tris_v, uint32_t n, uint32_t leaf, ph
     if ((rc = phr_array_alloc(g, 32, n, &t->prims)) != PHR_OK) return fail(rc);
     if ((rc = phr_array_alloc(g, 16, n, &t->faces)) != PHR_OK) return fail(rc);
     if ((rc = phr_array_alloc(g, 48, n, &t->tris)) != PHR_OK) return fail(rc);
-    if (hipMalloc(&t->rays, COUNT_BYTES) != hipSuccess || hipMemsetAsync(t->rays, 0, COUNT_BYTES, s) != hipSuccess ||
+    if (hipMalloc(&t->rays, COUNT_ALLOC) != hipSuccess || hipMemsetAsync(t->rays, 0, COUNT_ALLOC, s) != hipSuccess ||
         hipMalloc(&t->cam_dev, sizeof(PhrCamera)) != hipSuccess) {
         phr_set_error_msg("phr_tracer_new: allocation failed");
         return fail(PHR_ERR_HIP);
@@ -3940,7 +4054,7 @@ int phr_tracer_sample_in(phr_tracer* t, const void* cam_v, uint32_t w, uint32_t 
         for (uint32_t k = 0; k < slices && !abandoned; ++k) {
             const uint32_t a = (uint32_t)((uint64_t)tiles * k / slices), b = (uint32_t)((uint64_t)tiles * (k + 1) / slices);
             if (b == a) continue;
-            launch_path(path_build_waves(t), t->forest, regen, dim3(b - a), s, sc, cp, tiles_x, f0, count, pxp, t->rays, listed, a,
+            launch_path(t->gpu, path_build_waves(t), t->forest, regen, dim3(b - a), s, sc, cp, tiles_x, f0, count, pxp, t->rays, listed, a,
                         path_short_stack(t), t->split_shade);
             PHR_HIP(hipGetLastError());
             if (slices > 1) {
@@ -4274,7 +4388,7 @@ int phr_tracer_record_frame(phr_tracer* t, const void* cam_v, uint32_t w, uint32
     uint32_t* pxp = (uint32_t*)t->px->ptr;
     PHR_HIP(hipStreamSynchronize(s));
     PHR_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-    launch_path(path_build_waves(t), t->forest, regen_allowed(cam) ? t->path_regen : 0u, dim3(tiles), s, sc, cp, tiles_x, 0u, spp, pxp,
+    launch_path(t->gpu, path_build_waves(t), t->forest, regen_allowed(cam) ? t->path_regen : 0u, dim3(tiles), s, sc, cp, tiles_x, 0u, spp, pxp,
                 t->rays, 0u, 0u, path_short_stack(t), t->split_shade);
     int rc = PHR_OK;
     if (denoise == 1) rc = phr_denoise_enqueue(t->gpu, pxp, t->w, t->h, 0, t->dn_scratch, t->last.view);
@@ -4401,7 +4515,7 @@ int phr_tracer_record_pose_frame(phr_tracer* t, phr_array* verts, const float* w
     if (rc == PHR_OK) {
         hipLaunchKernelGGL(k_stamp_pose, dim3(1), dim3(64), 0, s, (const float4*)t->nodes->ptr, (const uint32_t*)t->lights->ptr, 1u,
                            cam.ao <= 0.f ? 1u : 0u, cp);
-        launch_path(path_build_waves(t), t->forest, 0u, dim3(tiles), s, sc, cp, tiles_x, 0u, spp, pxp, t->rays, 0u, 0u,
+        launch_path(t->gpu, path_build_waves(t), t->forest, 0u, dim3(tiles), s, sc, cp, tiles_x, 0u, spp, pxp, t->rays, 0u, 0u,
                     path_short_stack(t));
         if (denoise == 1) rc = phr_denoise_enqueue(t->gpu, pxp, t->w, t->h, 0, t->dn_scratch, t->last.view);
         if (denoise == 2) {
@@ -4733,7 +4847,7 @@ int phr_tracer_from_scene(phr_gpu* g, const phr_scene_desc* d, uint32_t leaf, ph
     if ((rc = phr_array_alloc(g, 4, t->ninsts, &t->inst_mesh)) != PHR_OK) return fail(rc);
     std::vector<uint32_t> mesh_of(t->ninsts);
     for (uint32_t i = 0; i < t->ninsts; ++i) mesh_of[i] = std::min(t->inst_in[i].mesh, t->nmeshes - 1);  // placed ones are valid
-    if (hipMalloc(&t->rays, COUNT_BYTES) != hipSuccess || hipMemsetAsync(t->rays, 0, COUNT_BYTES, s) != hipSuccess ||
+    if (hipMalloc(&t->rays, COUNT_ALLOC) != hipSuccess || hipMemsetAsync(t->rays, 0, COUNT_ALLOC, s) != hipSuccess ||
         hipMalloc(&t->cam_dev, sizeof(PhrCamera)) != hipSuccess || hipMalloc(&t->bases_dev, 4ull * t->nmeshes) != hipSuccess) {
         phr_set_error_msg("phr_tracer_from_scene: allocation failed");
         return fail(PHR_ERR_HIP);
@@ -4933,9 +5047,8 @@ int batch_image(phr_batch* b, uint32_t w, uint32_t h) {
 void batch_launch(phr_batch* b, const PhrCamera* cams, uint32_t spp, uint32_t waves, uint32_t grouped, uint32_t build,
                   uint32_t shade8) {
     const uint32_t tiles_x = (b->w + 15) / 16, tiles = tiles_x * ((b->h + 15) / 16);
-    const dim3 grid(tiles * b->scenes);
     const uint64_t stride = PX_LEN * (uint64_t)b->w * b->h + 1;
-    launch_path_batch(waves, build == 3u && b->split_ok, grid, b->gpu->stream, b->table, cams, tiles, tiles_x, spp, (uint32_t*)b->px->ptr,
+    launch_path_batch(b->gpu, waves, build == 3u && b->split_ok, b->scenes, b->gpu->stream, b->table, cams, tiles, tiles_x, spp, (uint32_t*)b->px->ptr,
                       stride, b->rays, grouped, shade8);
 }
 
@@ -5029,7 +5142,7 @@ int phr_batch_new(phr_gpu* g, const void* tris_v, const uint32_t* seg_lo, uint32
     if ((rc = phr_array_alloc(g, 32, n, &b->prims)) != PHR_OK) return fail(rc);
     if ((rc = phr_array_alloc(g, 16, n, &b->faces)) != PHR_OK) return fail(rc);
     if ((rc = phr_array_alloc(g, 48, n, &b->tris)) != PHR_OK) return fail(rc);
-    if (hipMalloc((void**)&b->rays, COUNT_BYTES) != hipSuccess || hipMemsetAsync(b->rays, 0, COUNT_BYTES, s) != hipSuccess ||
+    if (hipMalloc((void**)&b->rays, COUNT_ALLOC + 4ull * scenes) != hipSuccess || hipMemsetAsync(b->rays, 0, COUNT_ALLOC + 4ull * scenes, s) != hipSuccess ||
         hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess) {
         phr_set_error_msg("phr_batch_new: allocation failed");
         return fail(PHR_ERR_HIP);
