@@ -165,3 +165,23 @@ def test_gpu_denoise_matches_the_restatement(gpu, orc, keep):
     assert (np.abs(a - b) <= 1).all()
     assert (tr.pixels().reshape(-1) == got[:n].view(np.uint8)).all()
     assert (tr.display().reshape(-1) == got[4 * n:7 * n].view(np.float32)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [(1, 1), (3, 70), (65, 9), (129, 131), (481, 345), (640, 401), (1025, 801)])
+def test_gpu_denoise_at_every_row_count(gpu, orc, size):
+    """One, two and three rows a lane, with columns and rows left over, and
+    images smaller than a tap's reach, held to the restatement within 1e-5."""
+    w, h = size
+    tris, cam = scene()
+    cam["aspect"] = w / h
+    tr = P.Tracer.new(gpu, tris, 4)
+    tr.sample(cam, w, h, 2)
+    want = tr.px()
+    v = np.zeros(4, dtype=np.float32)
+    orc.lib().orc_denoise(orc.ptr(want), w, h, 0, orc.ptr(v))
+    tr.denoise(keep=False)
+    got, n = tr.px(), w * h
+    for lo, hi in [(1 * n, 4 * n), (4 * n, 7 * n), (14 * n, 20 * n)]:
+        a, b = got[lo:hi].view(np.float32), want[lo:hi].view(np.float32)
+        assert np.allclose(a, b, rtol=1e-5, atol=1e-7), f"words {lo}..{hi}: {np.abs(a - b).max()}"
