@@ -37,11 +37,11 @@
 //    beside the skip (upsampled concatenation), so the pooled and concatenated
 //    tensors exist only for training. The same kernel computes the input
 //    gradient, with the weights flipped and transposed.
-//  * wgrad: dW[tap][co][ci] = sum_p dZ[p][co] X[p + off(tap)][ci]. The pixel
-//    tiles are staged transposed in LDS, so the reduction over pixels is the
-//    MFMA K dimension. Each block writes a partial for its pixel chunk, and a
-//    second kernel sums the chunks in a fixed order, so the result is
-//    deterministic.
+//  * wgrad: dW[tap][co][ci] = sum_p dZ[p][co] X[p + off(tap)][ci]. The
+//    reduction over pixels is the MFMA K dimension: the pixel tiles are staged
+//    in LDS as they lie in memory and read transposed. Each block writes a
+//    partial for its tiles, and a second kernel sums the partials in a fixed
+//    order, so the result is deterministic.
 //  * apply: softmax over the 25 logits, the 5x5 filter, remodulation; the
 //    relMSE loss mean((y - t)^2 / (t^2 + 0.01)) and its gradient w.r.t. the
 //    logits.
@@ -85,9 +85,6 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
 __device__ __forceinline__ float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ float from_bf16s(short h) { return from_bf16((uint16_t)h); }
 
-__device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
 // gfx950's 16x16x32 form: 8 bf16 of K a lane. A and B fragments are loaded
 // with the same lane-slot to channel map, so the product does not depend on
 // the order the hardware gives the K slots.
@@ -143,7 +140,7 @@ struct ConvArgs {
 // Eight input channels [c, c + 8) of pixel (gy, gx) of image img, in the
 // input form `a` describes.
 __device__ __forceinline__ uint4 conv_input(const ConvArgs& a, uint64_t b, int gy, int gx, uint32_t c) {
-    if (a.pooled) {  // k_pool's sum order and rounding
+    if (a.pooled) {  // each 2x2 block summed row by row, rounded once
         const uint64_t W2 = 2ull * a.W;
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         for (int dy = 0; dy < 2; ++dy)
@@ -291,164 +288,166 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a, uint32_t tiles_x, uint
 }
 
 // ---- weight gradient ------------------------------------------------------------
-// Grid (chunks, 9 taps). Block b sums pixels [b * chunk, (b + 1) * chunk) for one tap.
-template <int NCO, int NCI>
-__global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dz,
-                                               uint32_t B, uint32_t H, uint32_t W, uint64_t chunk,
-                                               float* __restrict__ part, float* __restrict__ bpart) {
-    constexpr int COUT = NCO * 16, CIN = NCI * 16;
-    constexpr int TP = 64, LD = TP + 4;
-    constexpr int NFR = NCO * NCI, FW = (NFR + 3) / 4;
-    __shared__ __align__(16) uint16_t sdz[COUT * LD];
-    __shared__ __align__(16) uint16_t sx[CIN * LD];
-    const uint32_t tap = blockIdx.y;
-    const int dy = (int)tap / 3 - 1, dx = (int)tap % 3 - 1;
-    const uint64_t HW = (uint64_t)H * W, P = B * HW;
-    const uint64_t lo = (uint64_t)blockIdx.x * chunk, hi = min(P, lo + chunk);
+// dW[tap][co][ci] = sum over pixels of dz[pixel][co] x[pixel + tap][ci]: the
+// pixels are the matrix instruction's K. A block takes tiles of 4 rows x 32
+// columns one after another (grid x), for 16 of the input channels (grid y):
+// the tile's dz and its x with a one-pixel halo are staged in LDS as they lie
+// in memory, 16 B a load, and ds_read_b64_tr_b16 hands each lane four pixels
+// of one channel, so a tap is an offset into the same staged pixels. A wave
+// owns some of the taps with all output channels. The next tile is loaded into
+// registers while this one's products run. Waves in flight bound it: all of
+// d0's 80 input channels in one block read x and dz once but held 290
+// registers, one wave a SIMD, and took 430 us at 8 x 512 x 512; 48 at a time
+// 249, 32 at a time 261, 16 at a time, reading dz five times, 217 (843 when
+// each tap read both for itself).
+constexpr int WG_ROWS = 4, WG_COLS = 32, WG_PIX = WG_ROWS * WG_COLS;
+constexpr int WG_HW = WG_COLS + 2, WG_HP = WG_HW * (WG_ROWS + 2);
+constexpr int WG_TILES = 4;         // tiles a block takes at least, while the blocks still cover the CUs twice
+constexpr int WG_BLOCKS = 512;      // blocks (grid x) at most
+// Bytes a staged pixel: 64 channels apart, four pixels would share their banks.
+constexpr int wg_pitch(int ch) { return 2 * ch + (ch % 64 == 0 ? 16 : 0); }
+
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+// Eight pixels (K slots 8 g .. 8 g + 7) of channel c0 + lane % 16, of the
+// pixels at `at` (the lane's own: pixel 8 g + lane % 16 / 4 of the run, 4 (lane
+// % 4) channels on).
+__device__ __forceinline__ uint4 pixels_of(const char* at, int pitch) {
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)at);
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)(at + 4 * pitch));
+    const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+    return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+template <int NCO>
+__global__ __launch_bounds__(256) void k_wgrad(ConvArgs a, const uint16_t* __restrict__ dz, uint32_t tiles_x, uint32_t tiles_y,
+                                               uint32_t tiles, float* __restrict__ part, float* __restrict__ bpart) {
+    constexpr int COUT = NCO * 16, CIN = 16;  // CIN: the block's
+    constexpr int PX = wg_pitch(CIN), PZ = wg_pitch(COUT);
+    constexpr int PW = 3;  // taps a wave: wave, wave + 4, wave + 8
+    constexpr int XU = (WG_HP * (CIN / 8) + 255) / 256, ZU = (WG_PIX * (COUT / 8) + 255) / 256;
+    __shared__ __align__(16) char sx[WG_HP * PX];
+    __shared__ __align__(16) char sz[WG_PIX * PZ];
+    const uint32_t ci0 = blockIdx.y * CIN;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    f32x4 acc[FW];
+    const int H = (int)a.H, W = (int)a.W;
+    f32x4 acc[PW][NCO], bacc[NCO];
 #pragma unroll
-    for (int i = 0; i < FW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float bacc = 0.0f;
-    // A thread's share of a tile: NCO quads of dz and NCI quads of x (TP
-    // pixels x COUT / 4 quads = 256 NCO). The next tile's share is loaded
-    // into registers while this one's MFMAs run.
-    bf16x4 vdz[NCO], vx[NCI];
-    auto load = [&](uint64_t t0) {
-        // The tile's first pixel (the same for every thread); pixel t0 + j
-        // lies j columns on, wrapping into the next rows (and images).
-        const uint64_t b0 = t0 / HW, r0 = t0 % HW;
-        const uint32_t y0 = (uint32_t)(r0 / W), x0 = (uint32_t)(r0 % W);
+    for (int f = 0; f < NCO; ++f) {
+        bacc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int k = 0; k < NCO; ++k) {
-            const uint32_t u = threadIdx.x + 256u * k, j = u / (COUT / 4), q = u % (COUT / 4);
-            const uint64_t p = t0 + j;
-            vdz[k] = p < hi ? *(const bf16x4*)(dz + p * COUT + 4 * q) : bf16x4{0, 0, 0, 0};
+        for (int i = 0; i < PW; ++i) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    uint4 vx[XU], vz[ZU];
+    auto load = [&](uint32_t t) {
+        const uint32_t tx = t % tiles_x, r = t / tiles_x, ty = r % tiles_y, b = r / tiles_y;
+        const int x0 = (int)tx * WG_COLS, y0 = (int)ty * WG_ROWS;
+#pragma unroll
+        for (int k = 0; k < XU; ++k) {
+            const uint32_t u = threadIdx.x + 256u * k, pix = u / (CIN / 8), c = 8 * (u % (CIN / 8));
+            const int gy = y0 + (int)(pix / WG_HW) - 1, gx = x0 + (int)(pix % WG_HW) - 1;
+            vx[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (u < WG_HP * (CIN / 8) && gy >= 0 && gy < H && gx >= 0 && gx < W)
+                vx[k] = conv_input(a, b, gy, gx, ci0 + c);
         }
 #pragma unroll
-        for (int k = 0; k < NCI; ++k) {
-            const uint32_t u = threadIdx.x + 256u * k, j = u / (CIN / 4), q = u % (CIN / 4);
-            const uint64_t p = t0 + j;
-            bf16x4 v = bf16x4{0, 0, 0, 0};
-            if (p < hi) {
-                uint64_t b = b0;
-                uint32_t cy = y0, cx = x0 + j;
-                while (cx >= W) {
-                    cx -= W;
-                    if (++cy == H) cy = 0, ++b;
-                }
-                const int yy = (int)cy + dy, xx = (int)cx + dx;
-                if (yy >= 0 && yy < (int)H && xx >= 0 && xx < (int)W)
-                    v = *(const bf16x4*)(x + (b * HW + (uint64_t)yy * W + xx) * CIN + 4 * q);
-            }
-            vx[k] = v;
+        for (int k = 0; k < ZU; ++k) {
+            const uint32_t u = threadIdx.x + 256u * k, pix = u / (COUT / 8), c = 8 * (u % (COUT / 8));
+            const int gy = y0 + (int)(pix / WG_COLS), gx = x0 + (int)(pix % WG_COLS);
+            vz[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (u < WG_PIX * (COUT / 8) && gy < H && gx < W)
+                vz[k] = *(const uint4*)(dz + (((uint64_t)b * a.H + gy) * a.W + gx) * COUT + c);
         }
     };
-    if (lo < hi) load(lo);
-    for (uint64_t t0 = lo; t0 < hi; t0 += TP) {
+    const uint32_t g = lane >> 4;
+    // The lane's place in a run of 32 pixels (pixels_of): its pixel, its bytes.
+    const int run = 8 * (int)g + (int)((lane & 15u) >> 2), part8 = 8 * (int)(lane & 3u);
+    const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);  // eight bf16 1.0
+    uint32_t t = blockIdx.x;
+    if (t < tiles) load(t);
+    for (; t < tiles; t += gridDim.x) {
+        __syncthreads();  // the previous tile's reads are done
 #pragma unroll
-        for (int k = 0; k < NCO; ++k) {
-            const uint32_t u = threadIdx.x + 256u * k, j = u / (COUT / 4), q = u % (COUT / 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sdz[(4 * q + e) * LD + j] = (uint16_t)vdz[k][e];
+        for (int k = 0; k < XU; ++k) {
+            const uint32_t u = threadIdx.x + 256u * k;
+            if (u < WG_HP * (CIN / 8)) *(uint4*)(sx + (u / (CIN / 8)) * PX + 16 * (u % (CIN / 8))) = vx[k];
         }
 #pragma unroll
-        for (int k = 0; k < NCI; ++k) {
-            const uint32_t u = threadIdx.x + 256u * k, j = u / (CIN / 4), q = u % (CIN / 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sx[(4 * q + e) * LD + j] = (uint16_t)vx[k][e];
+        for (int k = 0; k < ZU; ++k) {
+            const uint32_t u = threadIdx.x + 256u * k;
+            if (u < WG_PIX * (COUT / 8)) *(uint4*)(sz + (u / (COUT / 8)) * PZ + 16 * (u % (COUT / 8))) = vz[k];
         }
         __syncthreads();
-        if (t0 + TP < hi) load(t0 + TP);
+        if (t + gridDim.x < tiles) load(t + gridDim.x);
+#pragma unroll 1
+        for (int row = 0; row < WG_ROWS; ++row) {
+            uint4 az[NCO];
 #pragma unroll
-        for (int i = 0; i < FW; ++i) {
-            const int fr = (int)wave + 4 * i;
-            if (fr < NFR) {
-                const int fco = fr / NCI, fci = fr % NCI;
-                const uint16_t* ra = sdz + (16 * fco + (lane & 15u)) * LD + 4 * (lane >> 4);
-                const uint16_t* rb = sx + (16 * fci + (lane & 15u)) * LD + 4 * (lane >> 4);
+            for (int f = 0; f < NCO; ++f) az[f] = pixels_of(sz + (row * WG_COLS + run) * PZ + 32 * f + part8, PZ);
 #pragma unroll
-                for (int kk = 0; kk < TP / 16; ++kk)
-                    acc[i] = mfma16(*(const bf16x4*)(ra + 16 * kk), *(const bf16x4*)(rb + 16 * kk), acc[i]);
+            for (int i = 0; i < PW; ++i) {
+                const int tap = (int)wave + 4 * i;
+                if (tap < 9) {
+                    const uint4 bx = pixels_of(sx + ((row + tap / 3) * WG_HW + tap % 3 + run) * PX + part8, PX);
+#pragma unroll
+                    for (int f = 0; f < NCO; ++f) acc[i][f] = mfma32(az[f], bx, acc[i][f]);
+                }
             }
-        }
-        if (tap == 4u && threadIdx.x < (uint32_t)COUT)
-            for (int j = 0; j < TP; ++j) bacc += from_bf16(sdz[threadIdx.x * LD + j]);
-        __syncthreads();
-    }
-    float* dst = part + ((uint64_t)blockIdx.x * 9 + tap) * (COUT * CIN);
+            if (ci0 == 0u && wave == 3u)
 #pragma unroll
-    for (int i = 0; i < FW; ++i) {
-        const int fr = (int)wave + 4 * i;
-        if (fr < NFR) {
-            const int fco = fr / NCI, fci = fr % NCI;
+                for (int f = 0; f < NCO; ++f) bacc[f] = mfma32(az[f], ones, bacc[f]);
+        }
+    }
+    float* dst = part + (uint64_t)blockIdx.x * 9 * COUT * a.cin;
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const int tap = (int)wave + 4 * i;
+        if (tap >= 9) continue;
+#pragma unroll
+        for (int f = 0; f < NCO; ++f)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                dst[(16 * fco + 4 * (lane >> 4) + j) * CIN + 16 * fci + (lane & 15u)] = acc[i][j];
-        }
+                dst[((uint64_t)tap * COUT + 16 * f + 4 * g + j) * a.cin + ci0 + (lane & 15u)] = acc[i][f][j];
     }
-    if (tap == 4u && threadIdx.x < (uint32_t)COUT) bpart[(uint64_t)blockIdx.x * COUT + threadIdx.x] = bacc;
+    if (ci0 == 0u && wave == 3u && (lane & 15u) == 0u)
+#pragma unroll
+        for (int f = 0; f < NCO; ++f)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bpart[(uint64_t)blockIdx.x * COUT + 16 * f + 4 * g + j] = bacc[f][j];
 }
 
-// Sum the chunk partials in chunk order: grad_w[9][cout][cin], then grad_b[cout].
+// Sum the blocks' partials: grad_w[9][cout][cin], then grad_b[cout]. A block
+// sums 64 of them, a wave every fourth partial (eight loads on their way at a
+// time), then the four waves' sums in order.
 __global__ __launch_bounds__(256) void k_wreduce(const float* __restrict__ part, const float* __restrict__ bpart,
-                                                 uint32_t nchunk, uint32_t nw, uint32_t cout, float* __restrict__ gw,
+                                                 uint32_t nparts, uint32_t nw, uint32_t cout, float* __restrict__ gw,
                                                  float* __restrict__ gb) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < nw) {
-        float s = 0.0f;
-        for (uint32_t c = 0; c < nchunk; ++c) s += part[(uint64_t)c * nw + i];
-        gw[i] = s;
-    } else if (i < nw + cout) {
-        const uint32_t co = i - nw;
-        float s = 0.0f;
-        for (uint32_t c = 0; c < nchunk; ++c) s += bpart[(uint64_t)c * cout + co];
-        gb[co] = s;
+    __shared__ float s_sum[256];
+    const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63u), wave = threadIdx.x >> 6;
+    const bool is_w = i < nw, in = i < nw + cout;
+    const float* src = is_w ? part + i : bpart + (i - nw);
+    const uint64_t pitch = is_w ? nw : cout;
+    float s = 0.0f;
+    if (in) {
+        uint32_t c = wave;
+        for (; c + 28 < nparts; c += 32) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = src[(c + 4 * e) * pitch];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += v[e];
+        }
+        for (; c < nparts; c += 4) s += src[c * pitch];
+    }
+    s_sum[threadIdx.x] = s;
+    __syncthreads();
+    if (wave == 0u && in) {
+        const float v = ((s_sum[threadIdx.x] + s_sum[threadIdx.x + 64]) + s_sum[threadIdx.x + 128]) + s_sum[threadIdx.x + 192];
+        if (is_w) gw[i] = v;
+        else gb[i - nw] = v;
     }
 }
 
-// ---- pooling, upsampling, concatenation -----------------------------------------
-// Average of each 2x2 block: [B][2h][2w][C] -> [B][h][w][C]; one thread per 4 channels.
-__global__ __launch_bounds__(256) void k_pool(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, uint32_t B,
-                                              uint32_t h, uint32_t w, uint32_t C) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const uint32_t Q = C / 4;
-    if (i >= (uint64_t)B * h * w * Q) return;
-    const uint32_t q = (uint32_t)(i % Q);
-    const uint64_t pix = i / Q;
-    const uint32_t x = (uint32_t)(pix % w);
-    const uint64_t r = pix / w;
-    const uint32_t y = (uint32_t)(r % h), b = (uint32_t)(r / h);
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int dy = 0; dy < 2; ++dy)
-        for (int dx = 0; dx < 2; ++dx) {
-            bf16x4 v = *(const bf16x4*)(in + ((((uint64_t)b * 2 * h + 2 * y + dy) * 2 * w) + 2 * x + dx) * C + 4 * q);
-            for (int e = 0; e < 4; ++e) s[e] += from_bf16s(v[e]);
-        }
-    *(uint2*)(out + pix * C + 4 * q) = make_uint2(to_bf16(s[0] * 0.25f) | (uint32_t)to_bf16(s[1] * 0.25f) << 16,
-                                                  to_bf16(s[2] * 0.25f) | (uint32_t)to_bf16(s[3] * 0.25f) << 16);
-}
-
-// out[B][H][W][C1 + C2] = (coarse[y/2][x/2][C1], skip[y][x][C2]); one thread per 4 channels.
-__global__ __launch_bounds__(256) void k_upcat(const uint16_t* __restrict__ coarse, const uint16_t* __restrict__ skip,
-                                               uint16_t* __restrict__ out, uint32_t B, uint32_t H, uint32_t W,
-                                               uint32_t C1, uint32_t C2) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const uint32_t C = C1 + C2, Q = C / 4;
-    if (i >= (uint64_t)B * H * W * Q) return;
-    const uint32_t q = (uint32_t)(i % Q), c = 4 * q;
-    const uint64_t pix = i / Q;
-    const uint32_t x = (uint32_t)(pix % W);
-    const uint64_t r = pix / W;
-    const uint32_t y = (uint32_t)(r % H), b = (uint32_t)(r / H);
-    uint2 v;
-    if (c < C1)
-        v = *(const uint2*)(coarse + (((uint64_t)b * (H / 2) + y / 2) * (W / 2) + x / 2) * C1 + c);
-    else
-        v = *(const uint2*)(skip + pix * C2 + (c - C1));
-    *(uint2*)(out + pix * C + c) = v;
-}
-
+// ---- backward of pooling, upsampling and concatenation ----------------------------
 // Backward of k_upcat. Coarse part: dZ[b][y][x][c] = sum of the 2x2 children's
 // gradient, zeroed where the coarse activation is not positive (its ReLU).
 __global__ __launch_bounds__(256) void k_upcat_bwd_coarse(const float* __restrict__ g, const uint16_t* __restrict__ act,
@@ -652,8 +651,7 @@ struct phr_kpcn {
     bool train = false;
     char* ws = nullptr;
     uint64_t ws_bytes = 0;
-    uint16_t *F = nullptr, *act[NLAYERS] = {}, *Q0 = nullptr, *Q1 = nullptr, *Q2 = nullptr, *U2 = nullptr, *U1 = nullptr,
-             *U0 = nullptr;
+    uint16_t *F = nullptr, *act[NLAYERS] = {};
     float* logits = nullptr;
     uint16_t* dz[NLAYERS] = {};
     float *G = nullptr, *Gs0 = nullptr, *Gs1 = nullptr, *Gs2 = nullptr, *part = nullptr, *bpart = nullptr,
@@ -669,11 +667,15 @@ namespace {
 
 uint64_t level_pixels(const phr_kpcn* k, uint32_t l) { return (uint64_t)k->B * (k->Hp >> l) * (k->Wp >> l); }
 
-// Chunk length (a multiple of the 64-pixel tile) giving about 224 chunks per tap.
-uint64_t wgrad_chunk(uint64_t P) {
-    uint64_t c = (P + 223) / 224;
-    c = (c + 63) / 64 * 64;
-    return c < 1024 ? 1024 : c;
+// Blocks (grid x) of a weight gradient over `tiles` tiles, `groups` (grid y)
+// of them a tile.
+uint32_t wgrad_blocks(uint64_t tiles, uint32_t groups) {
+    const uint64_t fill = std::min<uint64_t>(tiles, (WG_BLOCKS + groups - 1) / groups);
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tiles / WG_TILES, fill), WG_BLOCKS);
+}
+uint64_t wgrad_tiles(const phr_kpcn* k, uint32_t level) {
+    const uint32_t h = k->Hp >> level, w = k->Wp >> level;
+    return (uint64_t)k->B * ((h + WG_ROWS - 1) / WG_ROWS) * ((w + WG_COLS - 1) / WG_COLS);
 }
 
 void free_ws(phr_kpcn* k) {
@@ -681,7 +683,6 @@ void free_ws(phr_kpcn* k) {
     k->ws = nullptr;
     k->ws_bytes = 0;
     k->B = k->H = k->W = 0;
-    k->Q0 = k->Q1 = k->Q2 = k->U2 = k->U1 = k->U0 = nullptr;
     for (int i = 0; i < NLAYERS; ++i) k->dz[i] = nullptr;
     k->G = k->Gs0 = k->Gs1 = k->Gs2 = k->part = k->bpart = nullptr;
 }
@@ -704,13 +705,7 @@ int ensure_ws(phr_kpcn* k, uint32_t B, uint32_t H, uint32_t W, bool train) {
     add((void**)&k->logits, P(0) * LOGITS * 4);
     k->loss_n = grid_of(P(0));
     add((void**)&k->loss_part, k->loss_n * 4);
-    if (train) {  // the pooled and concatenated inputs, whole, for the weight gradients
-        add((void**)&k->Q0, P(1) * 32 * 2);
-        add((void**)&k->Q1, P(2) * 48 * 2);
-        add((void**)&k->Q2, P(3) * 64 * 2);
-        add((void**)&k->U2, P(2) * 160 * 2);
-        add((void**)&k->U1, P(1) * 112 * 2);
-        add((void**)&k->U0, P(0) * 80 * 2);
+    if (train) {
         for (int i = 0; i < NLAYERS; ++i) add((void**)&k->dz[i], P(LAYERS[i].level) * LAYERS[i].cout * 2);
         uint64_t g = 0;
         for (int i = 1; i < NLAYERS; ++i) g = std::max<uint64_t>(g, P(LAYERS[i].level) * LAYERS[i].cin);
@@ -720,9 +715,9 @@ int ensure_ws(phr_kpcn* k, uint32_t B, uint32_t H, uint32_t W, bool train) {
         add((void**)&k->Gs2, P(2) * 64 * 4);
         uint64_t pn = 0, bn = 0;
         for (int i = 0; i < NLAYERS; ++i) {
-            const uint64_t Pl = P(LAYERS[i].level), nch = (Pl + wgrad_chunk(Pl) - 1) / wgrad_chunk(Pl);
-            pn = std::max<uint64_t>(pn, nch * 9 * LAYERS[i].cout * LAYERS[i].cin);
-            bn = std::max<uint64_t>(bn, nch * LAYERS[i].cout);
+            const uint64_t nb = wgrad_blocks(wgrad_tiles(k, LAYERS[i].level), LAYERS[i].cin / 16);
+            pn = std::max<uint64_t>(pn, nb * 9 * LAYERS[i].cout * LAYERS[i].cin);
+            bn = std::max<uint64_t>(bn, nb * LAYERS[i].cout);
         }
         k->part_n = pn, k->bpart_n = bn;
         add((void**)&k->part, pn * 4);
@@ -782,22 +777,31 @@ int launch_conv(const ConvArgs& a, hipStream_t s, int rw = 0) {
     return PHR_OK;
 }
 
-// Forward conv of layer `li` at its level; `pooled` / (`xc`, `c1`) select the
-// fused input forms (ConvArgs).
-int conv_fwd(phr_kpcn* k, int li, const uint16_t* x, uint16_t* y16, float* y32, uint32_t pooled = 0,
-             const uint16_t* xc = nullptr, uint32_t c1 = 0) {
+// Layer `li`'s input as the network reads it (ConvArgs' input forms): pooled
+// for the first conv of levels 1-3, the coarser output upsampled beside the
+// skip for the decoders; with its shape, weights and bias.
+ConvArgs conv_args(const phr_kpcn* k, int li) {
     const LayerDef& L = LAYERS[li];
+    uint16_t* const* A = k->act;
     ConvArgs a{};
-    a.x = x;
     a.w = k->wf + k->off_16[li];
     a.bias = k->master + k->off_b[li];
-    a.mask = nullptr;
-    a.y16 = y16;
-    a.y32 = y32;
     a.B = k->B, a.H = k->Hp >> L.level, a.W = k->Wp >> L.level;
     a.cin = L.cin, a.cout = L.cout, a.relu = L.relu;
-    a.pooled = pooled, a.xc = xc, a.c1 = c1;
-    return launch_conv(a, k->gpu->stream, k->rw[li]);
+    switch (li) {
+        case E0A: a.x = k->F; break;
+        case E0B: a.x = A[E0A]; break;
+        case E1A: a.x = A[E0B], a.pooled = 1; break;
+        case E1B: a.x = A[E1A]; break;
+        case E2A: a.x = A[E1B], a.pooled = 1; break;
+        case E2B: a.x = A[E2A]; break;
+        case E3: a.x = A[E2B], a.pooled = 1; break;
+        case D2: a.x = A[E2B], a.xc = A[E3], a.c1 = 96; break;
+        case D1: a.x = A[E1B], a.xc = A[D2], a.c1 = 64; break;
+        case D0: a.x = A[E0B], a.xc = A[D1], a.c1 = 48; break;
+        default: a.x = A[D0]; break;
+    }
+    return a;
 }
 
 // Input gradient of layer `li`: conv of its output gradient with the flipped,
@@ -817,49 +821,31 @@ int conv_bwd_data(phr_kpcn* k, int li, const uint16_t* dzi, const uint16_t* mask
     return launch_conv(a, k->gpu->stream);
 }
 
-template <int NCO, int NCI>
-void launch_wgrad_t(phr_kpcn* k, const uint16_t* x, const uint16_t* dzi, uint32_t level, uint64_t nch, uint64_t chunk) {
-    hipLaunchKernelGGL((k_wgrad<NCO, NCI>), dim3((uint32_t)nch, 9), dim3(256), 0, k->gpu->stream, x, dzi, k->B,
-                       k->Hp >> level, k->Wp >> level, chunk, k->part, k->bpart);
+template <int NCO>
+void launch_wgrad_t(phr_kpcn* k, const ConvArgs& a, const uint16_t* dzi, uint64_t tiles, uint32_t blocks) {
+    const uint32_t tx = (a.W + WG_COLS - 1) / WG_COLS, ty = (a.H + WG_ROWS - 1) / WG_ROWS;
+    hipLaunchKernelGGL(k_wgrad<NCO>, dim3(blocks, a.cin / 16), dim3(256), 0, k->gpu->stream, a, dzi, tx, ty, (uint32_t)tiles, k->part,
+                       k->bpart);
 }
 
-int wgrad(phr_kpcn* k, int li, const uint16_t* x) {
+// The weight and bias gradient of layer `li` over its input as the forward
+// convolution reads it (conv_args).
+int wgrad(phr_kpcn* k, int li) {
     const LayerDef& L = LAYERS[li];
-    const uint64_t P = level_pixels(k, L.level), chunk = wgrad_chunk(P), nch = (P + chunk - 1) / chunk;
-    switch (li) {
-        case E0A: launch_wgrad_t<2, 1>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case E0B: launch_wgrad_t<2, 2>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case E1A: launch_wgrad_t<3, 2>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case E1B: launch_wgrad_t<3, 3>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case E2A: launch_wgrad_t<4, 3>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case E2B: launch_wgrad_t<4, 4>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case E3: launch_wgrad_t<6, 4>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case D2: launch_wgrad_t<4, 10>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case D1: launch_wgrad_t<3, 7>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case D0: launch_wgrad_t<2, 5>(k, x, k->dz[li], L.level, nch, chunk); break;
-        case OUT: launch_wgrad_t<2, 2>(k, x, k->dz[li], L.level, nch, chunk); break;
+    const ConvArgs a = conv_args(k, li);
+    const uint64_t tiles = wgrad_tiles(k, L.level);
+    const uint32_t blocks = wgrad_blocks(tiles, L.cin / 16);
+    switch (L.cout / 16) {
+        case 2: launch_wgrad_t<2>(k, a, k->dz[li], tiles, blocks); break;
+        case 3: launch_wgrad_t<3>(k, a, k->dz[li], tiles, blocks); break;
+        case 4: launch_wgrad_t<4>(k, a, k->dz[li], tiles, blocks); break;
+        case 6: launch_wgrad_t<6>(k, a, k->dz[li], tiles, blocks); break;
+        default: phr_set_error_msg("kpcn weight gradient: unsupported output channel count"); return PHR_ERR_ARG;
     }
     PHR_HIP(hipGetLastError());
     const uint32_t nw = 9 * L.cout * L.cin;
-    hipLaunchKernelGGL(k_wreduce, dim3(grid_of(nw + L.cout)), dim3(256), 0, k->gpu->stream, k->part, k->bpart,
-                       (uint32_t)nch, nw, L.cout, k->grad + k->off_w[li], k->grad + k->off_b[li]);
-    PHR_HIP(hipGetLastError());
-    return PHR_OK;
-}
-
-int pool(phr_kpcn* k, const uint16_t* in, uint16_t* out, uint32_t level_out, uint32_t C) {
-    const uint32_t h = k->Hp >> level_out, w = k->Wp >> level_out;
-    hipLaunchKernelGGL(k_pool, dim3(grid_of((uint64_t)k->B * h * w * (C / 4))), dim3(256), 0, k->gpu->stream, in, out,
-                       k->B, h, w, C);
-    PHR_HIP(hipGetLastError());
-    return PHR_OK;
-}
-
-int upcat(phr_kpcn* k, const uint16_t* coarse, const uint16_t* skip, uint16_t* out, uint32_t level, uint32_t C1,
-          uint32_t C2) {
-    const uint32_t H = k->Hp >> level, W = k->Wp >> level;
-    hipLaunchKernelGGL(k_upcat, dim3(grid_of((uint64_t)k->B * H * W * ((C1 + C2) / 4))), dim3(256), 0, k->gpu->stream,
-                       coarse, skip, out, k->B, H, W, C1, C2);
+    hipLaunchKernelGGL(k_wreduce, dim3((nw + L.cout + 63) / 64), dim3(256), 0, k->gpu->stream, k->part, k->bpart, blocks, nw, L.cout,
+                       k->grad + k->off_w[li], k->grad + k->off_b[li]);
     PHR_HIP(hipGetLastError());
     return PHR_OK;
 }
@@ -870,44 +856,20 @@ int upcat(phr_kpcn* k, const uint16_t* coarse, const uint16_t* skip, uint16_t* o
         if (rc_ != PHR_OK) return rc_; \
     } while (0)
 
-// Layer li's forward conv with its input as the network reads it: pooled for
-// the first conv of levels 1-3, the coarser output upsampled beside the skip
-// for the decoders.
+// Layer li's forward conv: its activation, or the output layer's logits.
 int conv_layer(phr_kpcn* k, int li) {
-    uint16_t** A = k->act;
-    switch (li) {
-        case E0A: return conv_fwd(k, E0A, k->F, A[E0A], nullptr);
-        case E0B: return conv_fwd(k, E0B, A[E0A], A[E0B], nullptr);
-        case E1A: return conv_fwd(k, E1A, A[E0B], A[E1A], nullptr, 1);
-        case E1B: return conv_fwd(k, E1B, A[E1A], A[E1B], nullptr);
-        case E2A: return conv_fwd(k, E2A, A[E1B], A[E2A], nullptr, 1);
-        case E2B: return conv_fwd(k, E2B, A[E2A], A[E2B], nullptr);
-        case E3: return conv_fwd(k, E3, A[E2B], A[E3], nullptr, 1);
-        case D2: return conv_fwd(k, D2, A[E2B], A[D2], nullptr, 0, A[E3], 96);
-        case D1: return conv_fwd(k, D1, A[E1B], A[D1], nullptr, 0, A[D2], 64);
-        case D0: return conv_fwd(k, D0, A[E0B], A[D0], nullptr, 0, A[D1], 48);
-        default: return conv_fwd(k, OUT, A[D0], nullptr, k->logits);
-    }
+    ConvArgs a = conv_args(k, li);
+    if (li == OUT) a.y32 = k->logits;
+    else a.y16 = k->act[li];
+    return launch_conv(a, k->gpu->stream, k->rw[li]);
 }
 
-// Forward to the logits. The pooled and concatenated inputs are read by the
-// convolutions themselves; training also keeps them whole for the weight
-// gradients.
-int forward(phr_kpcn* k, const float* frames, bool keep) {
-    hipStream_t s = k->gpu->stream;
-    hipLaunchKernelGGL(k_features, dim3(grid_of(level_pixels(k, 0))), dim3(256), 0, s, frames, k->B, k->H, k->W, k->Hp,
+// Forward to the logits.
+int forward(phr_kpcn* k, const float* frames) {
+    hipLaunchKernelGGL(k_features, dim3(grid_of(level_pixels(k, 0))), dim3(256), 0, k->gpu->stream, frames, k->B, k->H, k->W, k->Hp,
                        k->Wp, k->F);
     PHR_HIP(hipGetLastError());
-    uint16_t** A = k->act;
     for (int li = 0; li < NLAYERS; ++li) KP_TRY(conv_layer(k, li));
-    if (keep) {
-        KP_TRY(pool(k, A[E0B], k->Q0, 1, 32));
-        KP_TRY(pool(k, A[E1B], k->Q1, 2, 48));
-        KP_TRY(pool(k, A[E2B], k->Q2, 3, 64));
-        KP_TRY(upcat(k, A[E3], A[E2B], k->U2, 2, 96, 64));
-        KP_TRY(upcat(k, A[D2], A[E1B], k->U1, 1, 64, 48));
-        KP_TRY(upcat(k, A[D1], A[E0B], k->U0, 0, 48, 32));
-    }
     return PHR_OK;
 }
 
@@ -954,33 +916,33 @@ int pool_bwd(phr_kpcn* k, uint32_t level, uint32_t C, const float* gskip, const 
 int backward(phr_kpcn* k) {
     uint16_t** A = k->act;
     uint16_t** Z = k->dz;
-    KP_TRY(wgrad(k, OUT, A[D0]));
+    KP_TRY(wgrad(k, OUT));
     KP_TRY(conv_bwd_data(k, OUT, Z[OUT], A[D0], Z[D0], nullptr));
-    KP_TRY(wgrad(k, D0, k->U0));
+    KP_TRY(wgrad(k, D0));
     KP_TRY(conv_bwd_data(k, D0, Z[D0], nullptr, nullptr, k->G));
     KP_TRY(upcat_bwd(k, 0, 48, 32, A[D1], Z[D1], k->Gs0));
-    KP_TRY(wgrad(k, D1, k->U1));
+    KP_TRY(wgrad(k, D1));
     KP_TRY(conv_bwd_data(k, D1, Z[D1], nullptr, nullptr, k->G));
     KP_TRY(upcat_bwd(k, 1, 64, 48, A[D2], Z[D2], k->Gs1));
-    KP_TRY(wgrad(k, D2, k->U2));
+    KP_TRY(wgrad(k, D2));
     KP_TRY(conv_bwd_data(k, D2, Z[D2], nullptr, nullptr, k->G));
     KP_TRY(upcat_bwd(k, 2, 96, 64, A[E3], Z[E3], k->Gs2));
-    KP_TRY(wgrad(k, E3, k->Q2));
+    KP_TRY(wgrad(k, E3));
     KP_TRY(conv_bwd_data(k, E3, Z[E3], nullptr, nullptr, k->G));
     KP_TRY(pool_bwd(k, 2, 64, k->Gs2, A[E2B], Z[E2B]));
-    KP_TRY(wgrad(k, E2B, A[E2A]));
+    KP_TRY(wgrad(k, E2B));
     KP_TRY(conv_bwd_data(k, E2B, Z[E2B], A[E2A], Z[E2A], nullptr));
-    KP_TRY(wgrad(k, E2A, k->Q1));
+    KP_TRY(wgrad(k, E2A));
     KP_TRY(conv_bwd_data(k, E2A, Z[E2A], nullptr, nullptr, k->G));
     KP_TRY(pool_bwd(k, 1, 48, k->Gs1, A[E1B], Z[E1B]));
-    KP_TRY(wgrad(k, E1B, A[E1A]));
+    KP_TRY(wgrad(k, E1B));
     KP_TRY(conv_bwd_data(k, E1B, Z[E1B], A[E1A], Z[E1A], nullptr));
-    KP_TRY(wgrad(k, E1A, k->Q0));
+    KP_TRY(wgrad(k, E1A));
     KP_TRY(conv_bwd_data(k, E1A, Z[E1A], nullptr, nullptr, k->G));
     KP_TRY(pool_bwd(k, 0, 32, k->Gs0, A[E0B], Z[E0B]));
-    KP_TRY(wgrad(k, E0B, A[E0A]));
+    KP_TRY(wgrad(k, E0B));
     KP_TRY(conv_bwd_data(k, E0B, Z[E0B], A[E0A], Z[E0A], nullptr));
-    KP_TRY(wgrad(k, E0A, k->F));
+    KP_TRY(wgrad(k, E0A));
     return PHR_OK;
 }
 
@@ -1179,7 +1141,7 @@ int phr_kpcn_get_grads(phr_kpcn* k, float* host, uint64_t count) {
 // Device-pointer form of inference, shared with the tracer.
 int phr_kpcn_infer_dev(phr_kpcn* k, const float* frames, uint32_t b, uint32_t w, uint32_t h, float* out) {
     KP_TRY(ensure_ws(k, b, h, w, false));
-    KP_TRY(forward(k, frames, false));
+    KP_TRY(forward(k, frames));
     return apply(k, frames, out, nullptr, false);
 }
 
@@ -1197,7 +1159,7 @@ int phr_kpcn_loss(phr_kpcn* k, phr_array* frames, phr_array* targets, uint32_t b
     KP_TRY(check_shape(frames, b, w, h, targets, "phr_kpcn_loss"));
     if (out) KP_TRY(check_shape(frames, b, w, h, out, "phr_kpcn_loss"));
     KP_TRY(ensure_ws(k, b, h, w, false));
-    KP_TRY(forward(k, (const float*)frames->ptr, false));
+    KP_TRY(forward(k, (const float*)frames->ptr));
     KP_TRY(apply(k, (const float*)frames->ptr, out ? (float*)out->ptr : nullptr, (const float*)targets->ptr, false));
     return read_loss(k, loss);
 }
@@ -1207,7 +1169,7 @@ int phr_kpcn_backward(phr_kpcn* k, phr_array* frames, phr_array* targets, uint32
     PHR_CHECK(k && targets, PHR_ERR_ARG, "phr_kpcn_backward: null");
     KP_TRY(check_shape(frames, b, w, h, targets, "phr_kpcn_backward"));
     KP_TRY(ensure_ws(k, b, h, w, true));
-    KP_TRY(forward(k, (const float*)frames->ptr, true));
+    KP_TRY(forward(k, (const float*)frames->ptr));
     KP_TRY(apply(k, (const float*)frames->ptr, nullptr, (const float*)targets->ptr, true));
     KP_TRY(backward(k));
     if (loss) return read_loss(k, loss);
@@ -1300,7 +1262,7 @@ int phr_kpcn_autotune(phr_kpcn* k, phr_array* frames, uint32_t b, uint32_t w, ui
     PHR_CHECK(k, PHR_ERR_ARG, "phr_kpcn_autotune: null");
     KP_TRY(check_shape(frames, b, w, h, nullptr, "phr_kpcn_autotune"));
     KP_TRY(ensure_ws(k, b, h, w, false));
-    KP_TRY(forward(k, (const float*)frames->ptr, false));  // every layer's input in place
+    KP_TRY(forward(k, (const float*)frames->ptr));  // every layer's input in place
     hipStream_t s = k->gpu->stream;
     hipEvent_t e0, e1;
     PHR_HIP(hipEventCreate(&e0));
@@ -1364,7 +1326,7 @@ int phr_kpcn_train_indexed(phr_kpcn* k, phr_array* frames, const uint32_t* fidx,
                                hipMemcpyDeviceToDevice, k->gpu->stream));
     }
     KP_TRY(ensure_ws(k, b, h, w, true));
-    KP_TRY(forward(k, (const float*)bf, true));
+    KP_TRY(forward(k, (const float*)bf));
     KP_TRY(apply(k, (const float*)bf, nullptr, (const float*)bt, true));
     KP_TRY(backward(k));
     KP_TRY(phr_kpcn_adam(k, lr));

@@ -201,3 +201,23 @@ def test_autotuned_tiles_give_the_same_output(gpu):
     assert set(rows.tolist()) <= {1, 2}
     net.infer(f, 1, 96, 72, b)
     assert np.array_equal(a.read(), b.read())
+
+
+@pytest.mark.parametrize("b,h,w", [(1, 8, 8), (2, 9, 33), (1, 44, 72), (3, 24, 104), (1, 200, 264)])
+def test_gradients_at_the_tiles_edges(gpu, b, h, w):
+    """Every layer's gradient where the 4 x 32 pixel tiles are partly outside
+    (down to one pixel at the coarsest level), where a block takes one tile and
+    where it takes several; the same bound as the whole-frame test: bf16
+    activations against autograd through the same roundings."""
+    fr, tg = R.synthetic_frames(b, h, w, 40 + h)
+    p = _params(8)
+    net = P.Kpcn(gpu, p)
+    net.backward(_upload(gpu, fr), _upload(gpu, tg), b, w, h)
+    g = net.grads()
+    _, want = R.grads(p, P.Kpcn.layers(), fr, tg, bf16=True)
+    off = 0
+    for i, (cin, cout, _l, _r) in enumerate(P.Kpcn.layers().tolist()):
+        for n in (9 * cin * cout, cout):
+            a, e = g[off:off + n], want[off:off + n]
+            off += n
+            assert np.linalg.norm(a - e) <= 5e-2 * np.linalg.norm(e) + 1e-9, (i, n)
