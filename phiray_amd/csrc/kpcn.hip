@@ -172,8 +172,20 @@ constexpr int TILE_W = 32;
 constexpr int CHUNK = 32;            // input channels staged at once
 constexpr int HALO_STRIDE = CHUNK + 8;  // shorts a staged pixel (80 B: 16-B aligned, banks spread)
 
-template <int NF, int RW>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs a, uint32_t tiles_x, uint32_t tiles_y) {
+// Waves a SIMD the registers are fitted to: the loads' latency bounds the
+// kernel, so as many as cost no more than a few spilled registers. Measured at
+// 8 x 512 x 512 (us): 32 -> 80 channels 442 unfitted, 272 at two, 513 at three;
+// 48 -> 112 245 unfitted, 160 at two, 682 at three; 64 -> 160 and 64 -> 96
+// are fastest unfitted.
+constexpr int conv_waves(int nf, int rw, bool one) {
+    if (nf * rw <= 4) return one ? 5 : 4;
+    if (one && nf * rw <= 6) return 4;
+    return nf == 10 || nf == 6 ? 1 : 2;
+}
+// ONE: at most CHUNK input channels, so no chunk is loaded ahead.
+template <int NF, int RW, bool ONE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_waves(NF, RW, ONE)))) void k_conv(
+    ConvArgs a, uint32_t tiles_x, uint32_t tiles_y) {
     constexpr int TH = 4 * RW, MT = 2 * RW;
     constexpr int HWD = TILE_W + 2, HP = HWD * (TH + 2);
     __shared__ __align__(16) uint16_t tile[HP * HALO_STRIDE];
@@ -212,7 +224,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a, uint32_t tiles_x, uint
         }
     };
     load(0);
-    for (uint32_t c0 = 0; c0 < cin; c0 += CHUNK) {
+    for (uint32_t c0 = 0; c0 < (ONE ? 1u : cin); c0 += CHUNK) {
         // A last chunk of 16 channels runs the same instruction with the K
         // slots of lane groups 2 and 3 zero in both operands.
         const uint32_t cc = min((uint32_t)CHUNK, cin - c0), parts = cc / 8;
@@ -225,7 +237,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a, uint32_t tiles_x, uint
             if (u < HP * parts) *(uint4*)(tile + (u >> lp) * HALO_STRIDE + 8 * (u & (parts - 1u))) = v[k];
         }
         __syncthreads();
-        if (c0 + CHUNK < cin) load(c0 + CHUNK);
+        if (!ONE && c0 + CHUNK < cin) load(c0 + CHUNK);
         // A row of three taps at a time: its 3 NF weight fragments are loaded
         // together (one wait on the caches a row, not one a tap).
 #pragma unroll 1
@@ -745,7 +757,8 @@ int ensure_ws(phr_kpcn* k, uint32_t B, uint32_t H, uint32_t W, bool train) {
 template <int NF, int RW>
 void launch_conv_t(const ConvArgs& a, hipStream_t s) {
     const uint32_t tx = (a.W + TILE_W - 1) / TILE_W, ty = (a.H + 4 * RW - 1) / (4 * RW);
-    hipLaunchKernelGGL((k_conv<NF, RW>), dim3(tx * ty * a.B), dim3(256), 0, s, a, tx, ty);
+    if (a.cin <= CHUNK) hipLaunchKernelGGL((k_conv<NF, RW, true>), dim3(tx * ty * a.B), dim3(256), 0, s, a, tx, ty);
+    else hipLaunchKernelGGL((k_conv<NF, RW, false>), dim3(tx * ty * a.B), dim3(256), 0, s, a, tx, ty);
 }
 
 // rw: rows a wave owns (1 or 2; 0 = 2 up to 96 output channels, else 1).
