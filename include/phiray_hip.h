@@ -406,12 +406,13 @@ uint32_t phr_tracer_path_waves(const phr_tracer* t);
  * They serve a camera with lamps or a lit world and no Adaptive Sampling, and
  * 1 and 2 one tree only (3 serves a forest too); other frames take the
  * nested build, and a sliced sample or a recorded frame takes 1 for 2. The
- * autotune tries every build the scene and camera allow. */
+ * autotune tries every build the scene and camera allow. Default: 3 for a
+ * forest, 0 for one tree. */
 int phr_tracer_set_path_regen(phr_tracer* t, uint32_t on);
 uint32_t phr_tracer_path_regen(const phr_tracer* t);
 /* No counterpart in the reference: the split build's shading point. A wave
  * walks until `eighths` (1 to 8) eighths of its working lanes wait to shade
- * (default 6); the autotune picks 4 or 6. The sums do not depend on it. */
+ * (default 6; a forest's 4); the autotune picks 4 or 6. The sums do not depend on it. */
 int phr_tracer_set_split_shade(phr_tracer* t, uint32_t eighths);
 uint32_t phr_tracer_split_shade(const phr_tracer* t);
 /* No counterpart in the reference: the mesh-tree stack entries a thread of

@@ -994,10 +994,11 @@ class Tracer:
     def set_path_regen(self, mode: "bool | int") -> None:
         """Which build the path frames take: the nested one (False, 0), the
         path-regenerating one (True, 1), the wavefront one (2) or the split
-        one (3: a wave walks until three quarters of its lanes have finished their walk,
-        those shade and start their next walk while the others walk on). The
-        last three serve one tree and a camera with lamps or a lit world, no
-        Adaptive Sampling; other frames take the nested build."""
+        one (3: a wave walks until enough of its lanes have finished their walk,
+        those shade and start their next walk while the others walk on; the
+        default of a scene of instances). The last three serve a camera with
+        lamps or a lit world, no Adaptive Sampling, the second and third one
+        tree only; other frames take the nested build."""
         m = int(mode) if not isinstance(mode, bool) else (1 if mode else 0)
         _check(lib().phr_tracer_set_path_regen(self._h, m), "Tracer set_path_regen")
 

@@ -181,6 +181,25 @@ def test_forest_path_matches_the_twin(gpu, scene, spp):
     t.set_path_regen(P.Tracer.PATH_NESTED)
 
 
+@pytest.mark.parametrize("ninsts", [1, 2, 3, None])  # a top tree that is one leaf, of one inner node, of several; all bodies
+@pytest.mark.parametrize("w,h", [(1, 1), (17, 9), (130, 66)])  # fewer pixels than a wave, edges of tiles, more than one wave's
+def test_split_walk_is_the_default_and_matches_the_nested(gpu, ninsts, w, h):
+    print(f"[forest] split walk {ninsts} {w}x{h}", flush=True)
+    v, f, m, me, ins = forest_scene().arrays()
+    t = P.Tracer.from_scene(gpu, v, f, m, me, ins if ninsts is None else ins[:ninsts], leaf=4)
+    assert t.path_regen == P.Tracer.PATH_SPLIT
+    t.set_samples(64)
+    cam = S.path_camera(w, h, eye=(0.0, -7.0, 3.5), target=(0.0, 0.5, 0.8), rr_from=2)
+    got = {}
+    for build in (P.Tracer.PATH_SPLIT, P.Tracer.PATH_NESTED):
+        t.set_path_regen(build)
+        t.sample(S.path_camera(w + 1, h), w + 1, h, 1)  # another view: the next call starts over
+        t.sample(cam, w, h, 3)
+        t.sample(cam, w, h, 2)  # goes on from the sums
+        got[build] = t.px().copy()
+    assert np.array_equal(got[P.Tracer.PATH_SPLIT], got[P.Tracer.PATH_NESTED])  # the same walks in the same order
+
+
 def test_reinstance_matches_the_oracle(gpu, orc):
     print("[forest] reinstance", flush=True)
     arrs = forest_scene().arrays()
