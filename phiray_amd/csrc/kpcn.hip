@@ -94,21 +94,37 @@ __device__ __forceinline__ f32x4 mfma32(uint4 a, uint4 b, f32x4 c) {
                                                    0);
 }
 
+// i / d and i % d, in 32 bits where i fits (k_upcat_bwd_coarse 67 -> 65 us).
+__device__ __forceinline__ uint64_t div_of(uint64_t i, uint32_t d, uint32_t& rem) {
+    if (i >> 32) {
+        rem = (uint32_t)(i % d);
+        return i / d;
+    }
+    const uint32_t q = (uint32_t)i / d;
+    rem = (uint32_t)i - q * d;
+    return q;
+}
+
 // ---- features ---------------------------------------------------------------
+// The network's input, and beside it each pixel's demodulated radiance for the
+// filter, which reads it 25 times instead of dividing 75 (k_apply 165 -> 142 us
+// at 1080p; 298 -> 240 with the gradient at 8 x 512 x 512).
 __global__ __launch_bounds__(256) void k_features(const float* __restrict__ fr, uint32_t B, uint32_t H, uint32_t W,
-                                                  uint32_t Hp, uint32_t Wp, uint16_t* __restrict__ out) {
+                                                  uint32_t Hp, uint32_t Wp, uint16_t* __restrict__ out,
+                                                  float4* __restrict__ demod) {
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= (uint64_t)B * Hp * Wp) return;
-    const uint32_t x = (uint32_t)(i % Wp);
-    const uint64_t r = i / Wp;
-    const uint32_t y = (uint32_t)(r % Hp), b = (uint32_t)(r / Hp);
+    uint32_t x, y;
+    const uint32_t b = (uint32_t)div_of(div_of(i, Wp, x), Hp, y);
     const uint32_t sx = min(x, W - 1), sy = min(y, H - 1);
     const float* f = fr + (((uint64_t)b * H + sy) * W + sx) * FRAME;
     uint16_t v[FEAT];
+    float d[3];
     for (int c = 0; c < 3; ++c) {
-        float d = f[c] / fmaxf(f[3 + c], 0.05f);
-        v[c] = to_bf16(log1pf(fmaxf(d, 0.0f)));
+        d[c] = f[c] / fmaxf(f[3 + c], 0.05f);
+        v[c] = to_bf16(log1pf(fmaxf(d[c], 0.0f)));
     }
+    if (x < W && y < H) demod[((uint64_t)b * H + y) * W + x] = make_float4(d[0], d[1], d[2], 0.0f);
     for (int c = 3; c < 9; ++c) v[c] = to_bf16(f[c]);
     float z = f[9];
     v[9] = to_bf16(z < 0.0f ? -1.0f : z / (1.0f + z));
@@ -460,7 +476,7 @@ __global__ __launch_bounds__(256) void k_wreduce(const float* __restrict__ part,
 }
 
 // ---- backward of pooling, upsampling and concatenation ----------------------------
-// Backward of k_upcat. Coarse part: dZ[b][y][x][c] = sum of the 2x2 children's
+// Backward of upsampling: dZ[b][y][x][c] = sum of the 2x2 children's
 // gradient, zeroed where the coarse activation is not positive (its ReLU).
 __global__ __launch_bounds__(256) void k_upcat_bwd_coarse(const float* __restrict__ g, const uint16_t* __restrict__ act,
                                                           uint16_t* __restrict__ dz, uint32_t B, uint32_t h, uint32_t w,
@@ -468,11 +484,9 @@ __global__ __launch_bounds__(256) void k_upcat_bwd_coarse(const float* __restric
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     const uint32_t Q = C1 / 4;
     if (i >= (uint64_t)B * h * w * Q) return;
-    const uint32_t q = (uint32_t)(i % Q), c = 4 * q;
-    const uint64_t pix = i / Q;
-    const uint32_t x = (uint32_t)(pix % w);
-    const uint64_t r = pix / w;
-    const uint32_t y = (uint32_t)(r % h), b = (uint32_t)(r / h);
+    uint32_t q, x, y;
+    const uint64_t pix = div_of(i, Q, q);
+    const uint32_t c = 4 * q, b = (uint32_t)div_of(div_of(pix, w, x), h, y);
     float s[4] = {0.f, 0.f, 0.f, 0.f};
     for (int dy = 0; dy < 2; ++dy)
         for (int dx = 0; dx < 2; ++dx) {
@@ -486,31 +500,21 @@ __global__ __launch_bounds__(256) void k_upcat_bwd_coarse(const float* __restric
         make_uint2(to_bf16(s[0]) | (uint32_t)to_bf16(s[1]) << 16, to_bf16(s[2]) | (uint32_t)to_bf16(s[3]) << 16);
 }
 
-// Skip part of k_upcat's backward: gskip[p][c] = g[p][C1 + c].
-__global__ __launch_bounds__(256) void k_upcat_bwd_skip(const float* __restrict__ g, float* __restrict__ gs, uint64_t P,
-                                                        uint32_t C1, uint32_t C2) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const uint32_t Q = C2 / 4;
-    if (i >= P * Q) return;
-    const uint32_t c = 4 * (uint32_t)(i % Q);
-    const uint64_t pix = i / Q;
-    *(float4*)(gs + pix * C2 + c) = *(const float4*)(g + pix * (C1 + C2) + C1 + c);
-}
-
-// Backward of k_pool joined with the skip gradient:
-// dZ[p][c] = (gskip[p][c] + gq[parent][c] / 4) where act > 0, else 0.
-__global__ __launch_bounds__(256) void k_pool_bwd(const float* __restrict__ gq, const float* __restrict__ gs,
+// Backward of pooling joined with the skip gradient, which is channels C1 on of
+// the decoder's input gradient g [P][C1 + C]:
+// dZ[p][c] = (g[p][C1 + c] + gq[parent][c] / 4) where act > 0, else 0. Bound by
+// its bytes; reading g in place saved copying the skips' gradients out (three
+// launches, 156 us a step at 8 x 512 x 512).
+__global__ __launch_bounds__(256) void k_pool_bwd(const float* __restrict__ gq, const float* __restrict__ g,
                                                   const uint16_t* __restrict__ act, uint16_t* __restrict__ dz, uint32_t B,
-                                                  uint32_t H, uint32_t W, uint32_t C) {
+                                                  uint32_t H, uint32_t W, uint32_t C1, uint32_t C) {
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     const uint32_t Q = C / 4;
     if (i >= (uint64_t)B * H * W * Q) return;
-    const uint32_t c = 4 * (uint32_t)(i % Q);
-    const uint64_t pix = i / Q;
-    const uint32_t x = (uint32_t)(pix % W);
-    const uint64_t r = pix / W;
-    const uint32_t y = (uint32_t)(r % H), b = (uint32_t)(r / H);
-    float4 a = *(const float4*)(gs + pix * C + c);
+    uint32_t q, x, y;
+    const uint64_t pix = div_of(i, Q, q);
+    const uint32_t c = 4 * q, b = (uint32_t)div_of(div_of(pix, W, x), H, y);
+    float4 a = *(const float4*)(g + pix * (C1 + C) + C1 + c);
     float4 up = *(const float4*)(gq + (((uint64_t)b * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c);
     float s[4] = {a.x + up.x * 0.25f, a.y + up.y * 0.25f, a.z + up.z * 0.25f, a.w + up.w * 0.25f};
     bf16x4 m = *(const bf16x4*)(act + pix * C + c);
@@ -521,18 +525,17 @@ __global__ __launch_bounds__(256) void k_pool_bwd(const float* __restrict__ gq, 
 }
 
 // ---- filter application, loss and its gradient ------------------------------------
-__device__ __forceinline__ void demod_at(const float* __restrict__ fr, uint64_t base, uint32_t H, uint32_t W, int y, int x,
-                                         float d[3]) {
+__device__ __forceinline__ float4 demod_at(const float4* __restrict__ dm, uint64_t base, uint32_t H, uint32_t W, int y, int x) {
     y = min(max(y, 0), (int)H - 1);
     x = min(max(x, 0), (int)W - 1);
-    const float* f = fr + (base + (uint64_t)y * W + x) * FRAME;
-    for (int c = 0; c < 3; ++c) d[c] = f[c] / fmaxf(f[3 + c], 0.05f);
+    return dm[base + (uint64_t)y * W + x];
 }
 
 // One thread per padded pixel. Writes the filtered radiance where the pixel is
 // in the image; with a target, the per-block loss sum and the logits' gradient
 // (zero on the padding and the unused logit channels).
-__global__ __launch_bounds__(256) void k_apply(const float* __restrict__ lg, const float* __restrict__ fr, uint32_t B,
+__global__ __launch_bounds__(256) void k_apply(const float* __restrict__ lg, const float* __restrict__ fr,
+                                               const float4* __restrict__ dm, uint32_t B,
                                                uint32_t H, uint32_t W, uint32_t Hp, uint32_t Wp, float* __restrict__ out,
                                                const float* __restrict__ tgt, uint16_t* __restrict__ dlg,
                                                float* __restrict__ loss_part, float inv_count) {
@@ -540,9 +543,8 @@ __global__ __launch_bounds__(256) void k_apply(const float* __restrict__ lg, con
     const uint64_t np = (uint64_t)B * Hp * Wp;
     float l = 0.0f;
     if (i < np) {
-        const uint32_t x = (uint32_t)(i % Wp);
-        const uint64_t r = i / Wp;
-        const uint32_t y = (uint32_t)(r % Hp), b = (uint32_t)(r / Hp);
+        uint32_t x, y;
+        const uint32_t b = (uint32_t)div_of(div_of(i, Wp, x), Hp, y);
         const bool in = x < W && y < H;
         float g[LOGITS];
         for (int k = 0; k < (int)LOGITS; ++k) g[k] = 0.0f;
@@ -567,9 +569,8 @@ __global__ __launch_bounds__(256) void k_apply(const float* __restrict__ lg, con
             const uint64_t base = (uint64_t)b * H * W;
             float acc[3] = {0.f, 0.f, 0.f};
             for (int k = 0; k < (int)TAPS; ++k) {
-                float d[3];
-                demod_at(fr, base, H, W, (int)y + k / 5 - 2, (int)x + k % 5 - 2, d);
-                for (int c = 0; c < 3; ++c) acc[c] += w[k] * d[c];
+                const float4 d = demod_at(dm, base, H, W, (int)y + k / 5 - 2, (int)x + k % 5 - 2);
+                acc[0] += w[k] * d.x, acc[1] += w[k] * d.y, acc[2] += w[k] * d.z;
             }
             const uint64_t o = base + (uint64_t)y * W + x;
             const float* f = fr + o * FRAME;
@@ -592,9 +593,8 @@ __global__ __launch_bounds__(256) void k_apply(const float* __restrict__ lg, con
                 }
                 float gbar = 0.0f;
                 for (int k = 0; k < (int)TAPS; ++k) {
-                    float d[3];
-                    demod_at(fr, base, H, W, (int)y + k / 5 - 2, (int)x + k % 5 - 2, d);
-                    g[k] = ds[0] * d[0] + ds[1] * d[1] + ds[2] * d[2];
+                    const float4 d = demod_at(dm, base, H, W, (int)y + k / 5 - 2, (int)x + k % 5 - 2);
+                    g[k] = ds[0] * d.x + ds[1] * d.y + ds[2] * d.z;
                     gbar += w[k] * g[k];
                 }
                 for (int k = 0; k < (int)TAPS; ++k) g[k] = w[k] * (g[k] - gbar);
@@ -664,9 +664,10 @@ struct phr_kpcn {
     char* ws = nullptr;
     uint64_t ws_bytes = 0;
     uint16_t *F = nullptr, *act[NLAYERS] = {};
+    float4* demod = nullptr;  // [B][H][W] demodulated radiance
     float* logits = nullptr;
     uint16_t* dz[NLAYERS] = {};
-    float *G = nullptr, *Gs0 = nullptr, *Gs1 = nullptr, *Gs2 = nullptr, *part = nullptr, *bpart = nullptr,
+    float *G = nullptr, *Gd[3] = {}, *part = nullptr, *bpart = nullptr,
           *loss_part = nullptr;
     uint64_t part_n = 0, bpart_n = 0, loss_n = 0;
     std::vector<float> loss_host;
@@ -696,7 +697,7 @@ void free_ws(phr_kpcn* k) {
     k->ws_bytes = 0;
     k->B = k->H = k->W = 0;
     for (int i = 0; i < NLAYERS; ++i) k->dz[i] = nullptr;
-    k->G = k->Gs0 = k->Gs1 = k->Gs2 = k->part = k->bpart = nullptr;
+    k->G = k->Gd[0] = k->Gd[1] = k->Gd[2] = k->part = k->bpart = nullptr;
 }
 
 int ensure_ws(phr_kpcn* k, uint32_t B, uint32_t H, uint32_t W, bool train) {
@@ -713,18 +714,19 @@ int ensure_ws(phr_kpcn* k, uint32_t B, uint32_t H, uint32_t W, bool train) {
     auto add = [&](void** slot, uint64_t bytes) { want.push_back({slot, (bytes + 255) / 256 * 256}); };
     auto P = [&](uint32_t l) { return level_pixels(k, l); };
     add((void**)&k->F, P(0) * FEAT * 2);
+    add((void**)&k->demod, (uint64_t)B * H * W * 16);
     for (int i = 0; i < NLAYERS - 1; ++i) add((void**)&k->act[i], P(LAYERS[i].level) * LAYERS[i].cout * 2);
     add((void**)&k->logits, P(0) * LOGITS * 4);
     k->loss_n = grid_of(P(0));
     add((void**)&k->loss_part, k->loss_n * 4);
     if (train) {
         for (int i = 0; i < NLAYERS; ++i) add((void**)&k->dz[i], P(LAYERS[i].level) * LAYERS[i].cout * 2);
+        // The gradients of the pooled inputs (G, one at a time) and of the
+        // decoders' inputs (Gd, by level, whose skip part waits for G).
         uint64_t g = 0;
-        for (int i = 1; i < NLAYERS; ++i) g = std::max<uint64_t>(g, P(LAYERS[i].level) * LAYERS[i].cin);
+        for (int i : {E1A, E2A, E3}) g = std::max<uint64_t>(g, P(LAYERS[i].level) * LAYERS[i].cin);
         add((void**)&k->G, g * 4);
-        add((void**)&k->Gs0, P(0) * 32 * 4);
-        add((void**)&k->Gs1, P(1) * 48 * 4);
-        add((void**)&k->Gs2, P(2) * 64 * 4);
+        for (int i : {D0, D1, D2}) add((void**)&k->Gd[LAYERS[i].level], P(LAYERS[i].level) * LAYERS[i].cin * 4);
         uint64_t pn = 0, bn = 0;
         for (int i = 0; i < NLAYERS; ++i) {
             const uint64_t nb = wgrad_blocks(wgrad_tiles(k, LAYERS[i].level), LAYERS[i].cin / 16);
@@ -880,7 +882,7 @@ int conv_layer(phr_kpcn* k, int li) {
 // Forward to the logits.
 int forward(phr_kpcn* k, const float* frames) {
     hipLaunchKernelGGL(k_features, dim3(grid_of(level_pixels(k, 0))), dim3(256), 0, k->gpu->stream, frames, k->B, k->H, k->W, k->Hp,
-                       k->Wp, k->F);
+                       k->Wp, k->F, k->demod);
     PHR_HIP(hipGetLastError());
     for (int li = 0; li < NLAYERS; ++li) KP_TRY(conv_layer(k, li));
     return PHR_OK;
@@ -889,7 +891,7 @@ int forward(phr_kpcn* k, const float* frames) {
 int apply(phr_kpcn* k, const float* frames, float* out, const float* tgt, bool grad) {
     const uint64_t np = level_pixels(k, 0);
     const float inv_count = 1.0f / (3.0f * (float)k->B * (float)k->H * (float)k->W);
-    hipLaunchKernelGGL(k_apply, dim3(grid_of(np)), dim3(256), 0, k->gpu->stream, k->logits, frames, k->B, k->H, k->W,
+    hipLaunchKernelGGL(k_apply, dim3(grid_of(np)), dim3(256), 0, k->gpu->stream, k->logits, frames, k->demod, k->B, k->H, k->W,
                        k->Hp, k->Wp, out, tgt, grad ? k->dz[OUT] : nullptr, tgt ? k->loss_part : nullptr, inv_count);
     PHR_HIP(hipGetLastError());
     return PHR_OK;
@@ -904,23 +906,18 @@ int read_loss(phr_kpcn* k, float* loss) {
     return PHR_OK;
 }
 
-int upcat_bwd(phr_kpcn* k, uint32_t level, uint32_t C1, uint32_t C2, const uint16_t* act_coarse, uint16_t* dz_coarse,
-              float* gskip) {
+int upcat_bwd(phr_kpcn* k, uint32_t level, uint32_t C1, uint32_t C2, const uint16_t* act_coarse, uint16_t* dz_coarse) {
     const uint32_t h = k->Hp >> (level + 1), w = k->Wp >> (level + 1);
     hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(grid_of((uint64_t)k->B * h * w * (C1 / 4))), dim3(256), 0,
-                       k->gpu->stream, k->G, act_coarse, dz_coarse, k->B, h, w, C1, C1 + C2);
-    PHR_HIP(hipGetLastError());
-    const uint64_t P = level_pixels(k, level);
-    hipLaunchKernelGGL(k_upcat_bwd_skip, dim3(grid_of(P * (C2 / 4))), dim3(256), 0, k->gpu->stream, k->G, gskip, P, C1,
-                       C2);
+                       k->gpu->stream, k->Gd[level], act_coarse, dz_coarse, k->B, h, w, C1, C1 + C2);
     PHR_HIP(hipGetLastError());
     return PHR_OK;
 }
 
-int pool_bwd(phr_kpcn* k, uint32_t level, uint32_t C, const float* gskip, const uint16_t* act, uint16_t* dzo) {
+int pool_bwd(phr_kpcn* k, uint32_t level, uint32_t C1, uint32_t C, const uint16_t* act, uint16_t* dzo) {
     const uint32_t H = k->Hp >> level, W = k->Wp >> level;
     hipLaunchKernelGGL(k_pool_bwd, dim3(grid_of((uint64_t)k->B * H * W * (C / 4))), dim3(256), 0, k->gpu->stream, k->G,
-                       gskip, act, dzo, k->B, H, W, C);
+                       k->Gd[level], act, dzo, k->B, H, W, C1, C);
     PHR_HIP(hipGetLastError());
     return PHR_OK;
 }
@@ -932,27 +929,27 @@ int backward(phr_kpcn* k) {
     KP_TRY(wgrad(k, OUT));
     KP_TRY(conv_bwd_data(k, OUT, Z[OUT], A[D0], Z[D0], nullptr));
     KP_TRY(wgrad(k, D0));
-    KP_TRY(conv_bwd_data(k, D0, Z[D0], nullptr, nullptr, k->G));
-    KP_TRY(upcat_bwd(k, 0, 48, 32, A[D1], Z[D1], k->Gs0));
+    KP_TRY(conv_bwd_data(k, D0, Z[D0], nullptr, nullptr, k->Gd[0]));
+    KP_TRY(upcat_bwd(k, 0, 48, 32, A[D1], Z[D1]));
     KP_TRY(wgrad(k, D1));
-    KP_TRY(conv_bwd_data(k, D1, Z[D1], nullptr, nullptr, k->G));
-    KP_TRY(upcat_bwd(k, 1, 64, 48, A[D2], Z[D2], k->Gs1));
+    KP_TRY(conv_bwd_data(k, D1, Z[D1], nullptr, nullptr, k->Gd[1]));
+    KP_TRY(upcat_bwd(k, 1, 64, 48, A[D2], Z[D2]));
     KP_TRY(wgrad(k, D2));
-    KP_TRY(conv_bwd_data(k, D2, Z[D2], nullptr, nullptr, k->G));
-    KP_TRY(upcat_bwd(k, 2, 96, 64, A[E3], Z[E3], k->Gs2));
+    KP_TRY(conv_bwd_data(k, D2, Z[D2], nullptr, nullptr, k->Gd[2]));
+    KP_TRY(upcat_bwd(k, 2, 96, 64, A[E3], Z[E3]));
     KP_TRY(wgrad(k, E3));
     KP_TRY(conv_bwd_data(k, E3, Z[E3], nullptr, nullptr, k->G));
-    KP_TRY(pool_bwd(k, 2, 64, k->Gs2, A[E2B], Z[E2B]));
+    KP_TRY(pool_bwd(k, 2, 96, 64, A[E2B], Z[E2B]));
     KP_TRY(wgrad(k, E2B));
     KP_TRY(conv_bwd_data(k, E2B, Z[E2B], A[E2A], Z[E2A], nullptr));
     KP_TRY(wgrad(k, E2A));
     KP_TRY(conv_bwd_data(k, E2A, Z[E2A], nullptr, nullptr, k->G));
-    KP_TRY(pool_bwd(k, 1, 48, k->Gs1, A[E1B], Z[E1B]));
+    KP_TRY(pool_bwd(k, 1, 64, 48, A[E1B], Z[E1B]));
     KP_TRY(wgrad(k, E1B));
     KP_TRY(conv_bwd_data(k, E1B, Z[E1B], A[E1A], Z[E1A], nullptr));
     KP_TRY(wgrad(k, E1A));
     KP_TRY(conv_bwd_data(k, E1A, Z[E1A], nullptr, nullptr, k->G));
-    KP_TRY(pool_bwd(k, 0, 32, k->Gs0, A[E0B], Z[E0B]));
+    KP_TRY(pool_bwd(k, 0, 48, 32, A[E0B], Z[E0B]));
     KP_TRY(wgrad(k, E0B));
     KP_TRY(conv_bwd_data(k, E0B, Z[E0B], A[E0A], Z[E0A], nullptr));
     KP_TRY(wgrad(k, E0A));
