@@ -3904,6 +3904,9 @@ int phr_tracer_warm(phr_gpu* g, uint32_t cap, const char** names, double* ms, ui
         {"k_path_batch_sw<3>", (const void*)k_path_batch_sw<3>}, {"k_path_batch_sw<4>", (const void*)k_path_batch_sw<4>},
         {"k_path_batch_sw<5>", (const void*)k_path_batch_sw<5>}, {"k_path_sw_forest<2>", (const void*)k_path_sw_forest<2>},
         {"k_path_sw_forest<3>", (const void*)k_path_sw_forest<3>},
+        // the settings with the short stack or four waves: one kernel serves the three
+        {"k_path_sw_forest<3, short stack>", (const void*)k_path_sw_forest<3>},
+        {"k_path_sw_forest<4>", (const void*)k_path_sw_forest<3>},
     };
     uint32_t n = 0;
     for (const K& k : ks) {
