@@ -35,7 +35,7 @@
 //    output channels; the input tile and its halo are staged in LDS, read
 //    straight from the finer level (2x2 average) or from the coarser output
 //    beside the skip (upsampled concatenation), so the pooled and concatenated
-//    tensors exist only for training. The same kernel computes the input
+//    tensors never exist. The same kernel computes the input
 //    gradient, with the weights flipped and transposed.
 //  * wgrad: dW[tap][co][ci] = sum_p dZ[p][co] X[p + off(tap)][ci]. The
 //    reduction over pixels is the MFMA K dimension: the pixel tiles are staged

@@ -37,7 +37,7 @@ constexpr uint32_t PHR_INST = 1u << 30;  // a top-tree leaf's range is instance 
 
 struct SceneDev {
     const float4* nodes;
-    const float4* wide;    // one tree's wide records (WIDE_ROWS float4 a node index); a forest walks `nodes`
+    const float4* wide;    // one tree's wide records (WIDE_ROWS float4 an inner node); a forest walks `nodes`
     const float4* recs;    // binary records (4 float4 a node index) of the ordered any-hit walk
     const float4* kids;    // their second level (8 float4 a node index), after the first
     const float4* tris;    // 3 float4 per slot: (a.xyz, b.x) (b.yz, c.xy) (c.z, -, -, -)
@@ -3107,8 +3107,8 @@ struct phr_tracer {
     phr_array* prims = nullptr;     // Aabb per input face
     phr_array* faces = nullptr;     // uint4 per slot
     phr_array* tris = nullptr;      // 3 float4 per slot
-    phr_array* wide = nullptr;      // one tree's wide walk records: 128 B a node index
-    phr_array* recs = nullptr;      // its binary records for ordered any-hit rays: 192 B a node index
+    phr_array* wide = nullptr;      // one tree's wide walk records: 128 B an inner node
+    phr_array* recs = nullptr;      // its binary records for ordered any-hit rays: 192 B an inner node
     phr_array* lights = nullptr;    // [count, ids, insts, cdf]
     phr_array* px = nullptr;        // PX_LEN * w * h + 1 words
     unsigned long long* rays = nullptr;  // the walk counters, COUNT_SLOTS sets
@@ -4263,8 +4263,8 @@ int phr_tracer_rays(phr_tracer* t, uint64_t* closest, uint64_t* shadow) {
     return PHR_OK;
 }
 
-// All walk counters: path kernel [closest rays, shadow rays, inner steps,
-// triangle tests], raycasts [inner steps, triangle tests].
+// All walk counters: path kernel [closest rays, shadow rays, node visits,
+// triangle tests], raycasts [node visits, triangle tests].
 int phr_tracer_counters(phr_tracer* t, uint64_t* out6) {
     PHR_CHECK(t && out6, PHR_ERR_ARG, "phr_tracer_counters: null");
     return read_counts(t->gpu, t->rays, out6, 6);
@@ -5433,7 +5433,7 @@ int phr_batch_px(phr_batch* b, uint32_t k, uint64_t from, uint64_t count, uint32
     return PHR_OK;
 }
 
-// Rays traced since the batch was made: closest, shadow, inner steps, triangle tests.
+// Rays traced since the batch was made: closest, shadow, node visits, triangle tests.
 int phr_batch_counters(phr_batch* b, uint64_t* out4) {
     PHR_CHECK(b && out4, PHR_ERR_ARG, "phr_batch_counters: null");
     return read_counts(b->gpu, b->rays, out4, 4);
