@@ -704,15 +704,14 @@ def main() -> int:
                             "algorithmic_bytes": nbytes,
                             "kernel": {"nested": "k_path", "regen": "k_path_rg", "split": "k_path_sw",
                                        "wavefront": "k_wf_walk + k_wf_shade (one frame's turns)"}[build],
-                            "per_ray_bytes": "32 ray + 8 hit + 32 root + 64 x inner steps + 48 x triangle tests",
+                            "per_ray_bytes": "32 ray + 8 hit + 32 root + 112 x node visits + 48 x triangle tests",
                             "launch_ms": kernel_s * 1e3}
         if traffic:
             # What the DRAM counters saw: most node and triangle reads hit
             # L2 and the MALL, so the kernel waits on latency, not bandwidth.
             line["roofline"]["dram_achieved"] = traffic / kernel_s / 1e9
             line["roofline"]["dram_frac"] = traffic / kernel_s / 1e9 / HBM_PEAK_GBS
-            line["roofline"]["limiter"] = ("VALU issue of divergent waves (lanes a VALU instruction: 15.1 of 64 split, 11.0 nested; "
-                                           "VALU busy 0.76 / 0.73) and L2/MALL latency: frac counts the walk's logical bytes, "
+            line["roofline"]["limiter"] = ("VALU issue of divergent waves and L2/MALL latency: frac counts the walk's logical bytes, "
                                            "dram_frac the counted DRAM bytes")
         line["s_per_frame"] = per
         line["path_waves_per_simd"] = tracer.path_waves
