@@ -140,12 +140,15 @@ __device__ __forceinline__ float box_t(float4 lo, float4 hi, V3 o, V3 inv, float
 // enters at the very t of the hit in hand is still entered, for a tie.
 constexpr uint32_t WIDE_ROWS = 8;  // lo.x hi.x lo.y hi.y lo.z hi.z words, one row unused: 128 B, one cache line
 
+// A wide visit needs three free entries of the walk's LDS column.
+template <uint32_t N>
+__device__ __forceinline__ bool wide_room(uint32_t sp) { return sp + 3u <= N; }
+
 typedef float vec4 __attribute__((ext_vector_type(4)));
 // The visit of inner node `cur`: the nearest child met is entered (cur), the
-// others are pushed. False when none is met. The caller keeps three free
-// entries on the stack.
-__device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float best_t, uint32_t& cur, uint32_t* stk, uint32_t stride,
-                                       uint32_t& sp) {
+// others are pushed. False when none is met. The stack has room.
+template <uint32_t STRIDE>
+__device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float best_t, uint32_t& cur, uint32_t* stk, uint32_t& sp) {
     // A ray's near x, y and z rows: lo where it goes up the axis, else hi.
     const uint32_t nx = (__float_as_uint(inv.x) >> 27) & 16u, ny = (__float_as_uint(inv.y) >> 27) & 16u,
                    nz = (__float_as_uint(inv.z) >> 27) & 16u;
@@ -173,18 +176,35 @@ __device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float be
     nearer_first(k2, w2, k3, w3);
     nearer_first(k0, w0, k2, w2);
     // Stored whether met or not; the count moves on only past a met one.
-    stk[sp * stride] = __float_as_uint(w3);
+    stk[sp * STRIDE] = __float_as_uint(w3);
     sp += k3 < PHR_INF ? 1u : 0u;
-    stk[sp * stride] = __float_as_uint(w2);
+    stk[sp * STRIDE] = __float_as_uint(w2);
     sp += k2 < PHR_INF ? 1u : 0u;
-    stk[sp * stride] = __float_as_uint(w1);
+    stk[sp * STRIDE] = __float_as_uint(w1);
     sp += k1 < PHR_INF ? 1u : 0u;
     cur = __float_as_uint(w0);
     return k0 < PHR_INF;
 }
-// The most entries a stack of `entries` may hold before a visit, which stores
-// at up to two past them.
-constexpr uint32_t wide_room(uint32_t entries) { return entries - 3u; }
+// The largest t below a positive one.
+__device__ __forceinline__ float below(float t) { return __uint_as_float(__float_as_uint(t) - 1u); }
+// A visit a level at a time, from the nodes: of cur's two children those
+// entered up to `limit` are met, the nearer (a tie to the left) is entered, the
+// other pushed.
+template <class STACK>
+__device__ __forceinline__ bool visit1(const SceneDev& s, V3 o, V3 inv, float limit, uint32_t& cur, const STACK& stk, uint32_t& sp) {
+    const uint32_t l = __float_as_uint(s.nodes[2 * (size_t)cur].w), r = __float_as_uint(s.nodes[2 * (size_t)cur + 1].w);
+    const float4 llo = s.nodes[2 * (size_t)l], lhi = s.nodes[2 * (size_t)l + 1];
+    const float4 rlo = s.nodes[2 * (size_t)r], rhi = s.nodes[2 * (size_t)r + 1];
+    float tl = box_t(llo, lhi, o, inv, PHR_INF), tr = box_t(rlo, rhi, o, inv, PHR_INF);
+    tl = tl <= limit ? tl : PHR_INF;
+    tr = tr <= limit ? tr : PHR_INF;
+    const uint32_t wl = (__float_as_uint(llo.w) & PHR_LEAF) ? __float_as_uint(llo.w) : l;
+    const uint32_t wr = (__float_as_uint(rlo.w) & PHR_LEAF) ? __float_as_uint(rlo.w) : r;
+    const bool left = tl <= tr;
+    if ((left ? tr : tl) < PHR_INF) stk.push(sp, left ? wr : wl);
+    cur = left ? wl : wr;
+    return (left ? tl : tr) < PHR_INF;
+}
 
 // The first slot of the tree under node x: its leftmost leaf's.
 __device__ __forceinline__ uint32_t first_slot(const SceneDev& s, uint32_t x) {
@@ -223,49 +243,6 @@ __device__ __forceinline__ bool blocks(const SceneDev& s, uint32_t id) {  // bvh
     return !(m[6] > 0.5f || m[3] < 0.5f);
 }
 
-// The rest of a walk whose stack has no room left (13 entries at most on the
-// benchmark scenes): the whole tree again by its nodes and without a stack,
-// leaf after leaf in slot order, each found from the root (a box the ray
-// misses skips its leaves), with the hit found so far.
-__device__ __forceinline__ uint32_t end_slot(const SceneDev& s, uint32_t x) {
-    while (!(__float_as_uint(s.nodes[2 * (size_t)x].w) & PHR_LEAF)) x = __float_as_uint(s.nodes[2 * (size_t)x + 1].w);
-    return __float_as_uint(s.nodes[2 * (size_t)x + 1].w);
-}
-__device__ __forceinline__ void walk_nodes(const SceneDev& s, V3 o, V3 inv, const RaySpace& rs, bool any, PhrHit& best, uint32_t& tests) {
-    const uint32_t last = end_slot(s, s.root);
-    for (uint32_t slot = first_slot(s, s.root); slot < last;) {
-        for (uint32_t x = s.root;;) {
-            const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
-            // One step past a hit: an equal t further on may come first.
-            const float far = best.tri != PHR_NONE && !any ? __uint_as_float(__float_as_uint(best.t) + 1u) : best.t;
-            if (box_t(lo, hi, o, inv, far) >= PHR_INF) {
-                slot = end_slot(s, x);
-                break;
-            }
-            const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
-            if (!(l & PHR_LEAF)) {
-                x = slot < first_slot(s, r) ? l : r;
-                continue;
-            }
-            for (uint32_t id = l & ~PHR_LEAF; id < r; ++id) {
-                ++tests;
-                float u, v;
-                const float t = tri_t(s.tris[3 * (size_t)id], s.tris[3 * (size_t)id + 1], s.tris[3 * (size_t)id + 2], o, rs, u, v);
-                if (any) {
-                    if (t < best.t && blocks(s, id)) {
-                        best.tri = id;
-                        return;
-                    }
-                } else if (takes(s, o, inv, t, id, best.t, best.tri)) {
-                    best = PhrHit{t, id, u, v, 0u};
-                }
-            }
-            slot = r;
-            break;
-        }
-    }
-}
-
 // Where a walk starts: the root's index, or its leaf word where the root is
 // a leaf, whose end (no record holds it) is then `end` (else PHR_NONE).
 __device__ __forceinline__ uint32_t wide_root(const SceneDev& s, uint32_t& end) {
@@ -274,13 +251,52 @@ __device__ __forceinline__ uint32_t wide_root(const SceneDev& s, uint32_t& end) 
     return (w & PHR_LEAF) ? w : s.root;
 }
 
+// A stack of PHR_STACK LDS entries: what a walk a level at a time needs, which
+// pushes one of each level.
+template <uint32_t STRIDE>
+struct LevelStack {
+    uint32_t* lds;
+    __device__ __forceinline__ void push(uint32_t& sp, uint32_t word) const { lds[sp++ * STRIDE] = word; }
+};
+// The walk a level at a time, in the binary walk's order: where a wide walk's
+// stack is full. (No ray of 3,000 through 50,000 triangles as long as the
+// scene fills 32 entries; it takes boxes nested in one another.)
+template <bool ANY, uint32_t STRIDE>
+__device__ __forceinline__ PhrHit walk_binary(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* lds, uint32_t& steps, uint32_t& tests) {
+    PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
+    const V3 inv = safe_inv(d);
+    const RaySpace rs = ray_space(d);
+    const LevelStack<STRIDE> stk{lds};
+    uint32_t sp = 0, cur = s.root;  // an inner node, or the wide walk had not begun
+    for (;;) {
+        if (cur & PHR_LEAF) {
+            uint32_t id = cur & ~PHR_LEAF, end = PHR_NONE;
+            do {
+                ++tests;
+                const float4 t0 = s.tris[3 * (size_t)id], t1 = s.tris[3 * (size_t)id + 1], t2 = s.tris[3 * (size_t)id + 2];
+                if (end == PHR_NONE) end = __float_as_uint(t2.y);
+                float u, v;
+                const float t = tri_t(t0, t1, t2, o, rs, u, v);
+                if (t < best.t && (!ANY || blocks(s, id))) {
+                    best = PhrHit{t, id, u, v, 0u};
+                    if constexpr (ANY) return best;
+                }
+            } while (++id < end);
+        } else {
+            ++steps;
+            if (visit1(s, o, inv, below(best.t), cur, stk, sp)) continue;
+        }
+        if (sp == 0) return best;
+        cur = lds[--sp * STRIDE];
+    }
+}
+
 // The walk to the closest hit, or (ANY) to whether something blocks the ray
 // before tmax (then the hit's triangle is some blocking one). `steps` and
 // `tests` count visits and triangle tests, the units the walk's memory
 // traffic is priced in.
-template <bool ANY>
-__device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* stk, uint32_t stride, uint32_t& steps,
-                                       uint32_t& tests) {
+template <bool ANY, uint32_t STRIDE>
+__device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* lds, uint32_t& steps, uint32_t& tests) {
     PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
     const V3 inv = safe_inv(d);
     const RaySpace rs = ray_space(d);
@@ -313,15 +329,14 @@ __device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax
                 t1 = n1;
                 t2 = n2;
             }
-        } else if (sp > wide_room(PHR_STACK)) {
-            walk_nodes(s, o, inv, rs, ANY, best, tests);
-            break;
+        } else if (!wide_room<PHR_STACK>(sp)) {
+            return walk_binary<ANY, STRIDE>(s, o, d, tmax, lds, steps, tests);
         } else {
             ++steps;
-            if (visit4(s, o, inv, best.t, cur, stk, stride, sp)) continue;
+            if (visit4<STRIDE>(s, o, inv, best.t, cur, lds, sp)) continue;
         }
         if (sp == 0) break;
-        cur = stk[--sp * stride];
+        cur = lds[--sp * STRIDE];
     }
     return best;
 }
@@ -454,6 +469,30 @@ __device__ __forceinline__ PhrHit walk_first(const SceneDev& s, V3 o, V3 d, floa
 // or a leaf's triangles. A leaf reached is put by and the walk goes on from
 // the stack, until a second leaf is reached or nothing else is left.
 // `any`: a shadow ray's walk, which ends at the first triangle that blocks it.
+// The split build's stack: N LDS entries (a pixel's sums have the rest of the
+// column) and then scratch. With no room for a wide visit it visits a level at a
+// time. The N entries then come from at least N / 3 of the path's 31 inner
+// nodes and one more a level follows. (50,000 thin triangles as long as the
+// scene have 25 nodes pending, compact ones 13 to 16.)
+constexpr uint32_t DEEP_WORDS = 24;
+template <uint32_t N, uint32_t STRIDE>
+struct DeepStack {
+    static_assert(DEEP_WORDS + (N + 2) / 3 >= PHR_STACK - 1, "a tree's pending nodes fit");
+    uint32_t* lds;
+    volatile uint32_t* deep;  // DEEP_WORDS of scratch; volatile keeps them out of registers
+    __device__ __forceinline__ void push(uint32_t& sp, uint32_t word) const {
+        if (sp < N) lds[sp * STRIDE] = word;
+        else deep[sp - N] = word;
+        ++sp;
+    }
+    // DEEP: the top may lie in scratch (not so after a wide visit).
+    template <bool DEEP>
+    __device__ __forceinline__ uint32_t pop(uint32_t& sp) const {
+        --sp;
+        if (DEEP && sp >= N) return deep[sp - N];
+        return lds[sp * STRIDE];
+    }
+};
 struct Walker {
     V3 o, inv;
     RaySpace rs;
@@ -461,16 +500,18 @@ struct Walker {
     uint32_t tri, cur, leaf, sp;  // cur, leaf: PHR_NONE when there is none
     bool on, any;
 };
-__device__ __forceinline__ void walker_pop(Walker& w, const uint32_t* stk, uint32_t stride) {
+template <bool DEEP, class STACK>
+__device__ __forceinline__ void walker_pop(Walker& w, const STACK& stk) {
     w.cur = PHR_NONE;
-    if (w.sp != 0u) w.cur = stk[--w.sp * stride];
+    if (w.sp != 0u) w.cur = stk.template pop<DEEP>(w.sp);
 }
 // A leaf in hand is put by if none is yet; a walk with nothing left ends.
-__device__ __forceinline__ void walker_settle(Walker& w, const uint32_t* stk, uint32_t stride) {
+template <bool DEEP, class STACK>
+__device__ __forceinline__ void walker_settle(Walker& w, const STACK& stk) {
     if (w.leaf == PHR_NONE && (w.cur & PHR_LEAF)) {
         w.leaf = w.cur;
         w.on = w.cur != PHR_NONE;
-        if (w.on) walker_pop(w, stk, stride);
+        if (w.on) walker_pop<DEEP>(w, stk);
     }
 }
 __device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, uint32_t root, V3 o, V3 d, float tmax, bool any) {
@@ -487,25 +528,20 @@ __device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, uint3
     w.cur = leaf ? PHR_NONE : root;
     w.leaf = leaf ? root : PHR_NONE;
 }
-__device__ __forceinline__ void walker_visit(Walker& w, const SceneDev& s, uint32_t* stk, uint32_t stride, uint32_t entries,
-                                             uint32_t& steps, uint32_t& tests) {
-    if (w.sp > wide_room(entries)) {
-        PhrHit best{w.t, w.tri, w.u, w.v, 0u};
-        walk_nodes(s, w.o, w.inv, w.rs, w.any, best, tests);
-        w.t = best.t;
-        w.tri = best.tri;
-        w.u = best.u;
-        w.v = best.v;
-        w.on = false;
-        return;
-    }
+template <uint32_t N, uint32_t STRIDE>
+__device__ __forceinline__ void walker_visit(Walker& w, const SceneDev& s, const DeepStack<N, STRIDE>& stk, uint32_t& steps) {
     ++steps;
-    if (!visit4(s, w.o, w.inv, w.t, w.cur, stk, stride, w.sp)) walker_pop(w, stk, stride);
-    walker_settle(w, stk, stride);
+    if (wide_room<N>(w.sp)) {
+        if (!visit4<STRIDE>(s, w.o, w.inv, w.t, w.cur, stk.lds, w.sp)) walker_pop<false>(w, stk);
+        walker_settle<false>(w, stk);
+    } else {
+        if (!visit1(s, w.o, w.inv, w.t, w.cur, stk, w.sp)) walker_pop<true>(w, stk);
+        walker_settle<true>(w, stk);
+    }
 }
 // The triangles of the leaf put by; `only`: the root's end where it is a leaf.
-__device__ __forceinline__ void walker_leaf(Walker& w, const SceneDev& s, uint32_t only, const uint32_t* stk, uint32_t stride,
-                                            uint32_t& tests) {
+template <class STACK>
+__device__ __forceinline__ void walker_leaf(Walker& w, const SceneDev& s, uint32_t only, const STACK& stk, uint32_t& tests) {
     uint32_t id = w.leaf & ~PHR_LEAF;
     float4 t0 = s.tris[3 * (size_t)id], t1 = s.tris[3 * (size_t)id + 1], t2 = s.tris[3 * (size_t)id + 2];
     const uint32_t end = only != PHR_NONE ? only : __float_as_uint(t2.y);
@@ -540,7 +576,7 @@ __device__ __forceinline__ void walker_leaf(Walker& w, const SceneDev& s, uint32
         t1 = n1;
         t2 = n2;
     }
-    walker_settle(w, stk, stride);
+    walker_settle<true>(w, stk);
 }
 
 // The walk records of a tree's nodes (one entry per node index; only inner
@@ -975,7 +1011,7 @@ __global__ __launch_bounds__(RAYCAST_THREADS) void k_raycast(SceneDev sc, const 
         uint32_t* stk = s_stack + threadIdx.x;
         if constexpr (F) hits[i] = walk_forest<ANY>(sc, o, d, a.w, s_tstack + threadIdx.x, stk, RAYCAST_THREADS, steps, tests);
         else if constexpr (ANY) hits[i] = walk_first(sc, o, d, a.w, stk, RAYCAST_THREADS, steps, tests);
-        else hits[i] = walk<false>(sc, o, d, a.w, stk, RAYCAST_THREADS, steps, tests);
+        else hits[i] = walk<false, RAYCAST_THREADS>(sc, o, d, a.w, stk, steps, tests);
     }
     if (counters) {
         unsigned long long cs = steps, ct = tests;
@@ -1048,11 +1084,11 @@ __device__ __forceinline__ PhrHit trace(Ctx& c, V3 o, V3 d, float tmax, bool fir
     if (first) {
         c.shadow++;
         if constexpr (F) return walk_forest<true>(c.s, o, d, tmax, c.tstk, c.stk, TRACE_THREADS, c.steps, c.tests);
-        return walk<true>(c.s, o, d, tmax, c.stk, TRACE_THREADS, c.steps, c.tests);
+        return walk<true, TRACE_THREADS>(c.s, o, d, tmax, c.stk, c.steps, c.tests);
     }
     c.closest++;
     if constexpr (F) return walk_forest<false>(c.s, o, d, tmax, c.tstk, c.stk, TRACE_THREADS, c.steps, c.tests);
-    return walk<false>(c.s, o, d, tmax, c.stk, TRACE_THREADS, c.steps, c.tests);
+    return walk<false, TRACE_THREADS>(c.s, o, d, tmax, c.stk, c.steps, c.tests);
 }
 template <bool F>
 __device__ __forceinline__ float visible(Ctx& c, V3 org, V3 l, float dist) {
@@ -2038,13 +2074,15 @@ struct SplitWalk {
     // enough; once LEAF8 eighths of the walks have a leaf put by and nothing
     // to visit, every lane with a leaf put by tests its triangles.
     template <uint32_t STK>
-    __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t*, uint32_t& steps, uint32_t& tests) {
+    __device__ __forceinline__ void step(const SceneDev& s, uint32_t* lds, volatile uint32_t* deep, uint16_t*, uint32_t& steps,
+                                         uint32_t& tests) {
+        const DeepStack<STK, SPLIT_THREADS> stk{lds, deep};
         const uint32_t on = (uint32_t)__popcll(__ballot(w.on));
         const uint32_t stuck = (uint32_t)__popcll(__ballot(w.on && (w.cur & PHR_LEAF)));
         if (8u * stuck >= LEAF8 * on) {
-            if (w.on && w.leaf != PHR_NONE) walker_leaf(w, s, only, stk, SPLIT_THREADS, tests);
+            if (w.on && w.leaf != PHR_NONE) walker_leaf(w, s, only, stk, tests);
         } else if (w.on && !(w.cur & PHR_LEAF)) {
-            walker_visit(w, s, stk, SPLIT_THREADS, STK, steps, tests);
+            walker_visit(w, s, stk, steps);
         }
     }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, 0u}; }
@@ -2061,7 +2099,8 @@ struct SplitWalk<true> {
     // ms; by kind 24.2, with the visits in a loop of their own 21.9; visits
     // down to half of the walks 22.3, to a quarter 22.8).
     template <uint32_t STK>
-    __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, uint16_t* tstk, uint32_t& steps, uint32_t& tests) {
+    __device__ __forceinline__ void step(const SceneDev& s, uint32_t* stk, volatile uint32_t*, uint16_t* tstk, uint32_t& steps,
+                                         uint32_t& tests) {
         const int on = __popcll(__ballot(w.on));
         int nv = __popcll(__ballot(w.on && !(w.li & PHR_LEAF)));
         while (2 * nv >= on - nv) {
@@ -2095,6 +2134,7 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
     const uint32_t lane = threadIdx.x;
     uint32_t* stk = s_stack + lane;
     uint16_t* tstk = F ? s_tstack + lane : nullptr;
+    volatile uint32_t deep[F ? 1u : DEEP_WORDS];
     PixelSums<F> sum;
     if constexpr (!F) sum.c = s_sum + lane;
     uint32_t closest = 0, shadow = 0, steps = 0, tests = 0;
@@ -2187,7 +2227,7 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
         for (;;) {  // walk until shade8 / 8 of the lanes at work wait to shade, or all do
             const uint32_t working = (uint32_t)__popcll(lv), waiting = working - (uint32_t)__popcll(__ballot(w.on));
             if (waiting == working || 8u * waiting >= shade8 * working) break;
-            sw.template step<STK>(sc, stk, tstk, steps, tests);
+            sw.template step<STK>(sc, stk, deep, tstk, steps, tests);
         }
         if (!live || w.on) continue;
         bool next = false;
@@ -2463,7 +2503,7 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                                                         uint32_t tiles_x, uint32_t* __restrict__ px,
                                                         unsigned long long* __restrict__ rays) {
     __shared__ uint32_t s_stack[PHR_STACK * WF_THREADS];
-    uint32_t* stk = s_stack + threadIdx.x;
+    const LevelStack<WF_THREADS> stk{s_stack + threadIdx.x};
     uint32_t* ctr = w.ctr;
     if (!ANY && blockIdx.x == 0 && threadIdx.x == 0) {  // for this turn's shade and shadow walk
         ctr[1u - parity] = 0u;
@@ -2479,7 +2519,7 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
     RaySpace rs{};
     uint32_t cur = 0, sp = 0, slot = 0;
     uint32_t steps = 0, tests = 0, nrays = 0;
-    bool live = false, drained = count == 0u;
+    bool live = false, drained = count == 0u, binary = false;
     uint32_t cbase = 0, cend = 0;  // the wave's chunk of the queue
     uint32_t only;
     const uint32_t root = wide_root(sc, only);
@@ -2533,6 +2573,7 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                 sp = 0;
                 cur = root;
                 live = true;
+                binary = false;
             }
         }
         if (__ballot(live) == 0ull) {
@@ -2561,18 +2602,21 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                     best = PhrHit{t, id, u, v, 0u};
                 }
             } while (++id < end);
-        } else if (sp > wide_room(PHR_STACK)) {
-            walk_nodes(sc, o, inv, rs, ANY, best, tests);
-            more = false;
         } else {
             ++steps;
-            popped = !visit4(sc, o, inv, best.t, cur, stk, WF_THREADS, sp);
+            if (!binary && !wide_room<PHR_STACK>(sp)) {  // the stack is full: again, a level at a time (walk_binary)
+                binary = true;
+                sp = 0;
+                cur = root;
+                if constexpr (!ANY) best = PhrHit{PHR_INF, PHR_NONE, 0.f, 0.f, 0u};
+            }
+            popped = !(binary ? visit1(sc, o, inv, below(best.t), cur, stk, sp) : visit4<WF_THREADS>(sc, o, inv, best.t, cur, stk.lds, sp));
         }
         if (more && popped) {
             if (sp == 0) {
                 more = false;
             } else {
-                cur = stk[--sp * WF_THREADS];
+                cur = stk.lds[--sp * WF_THREADS];
             }
         }
         if (!more) {

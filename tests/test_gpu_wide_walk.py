@@ -7,8 +7,8 @@ hits must equal the oracle's binary walk bit for bit.
 * Scenes of one to nine triangles: a root that is a leaf, records with one to
   four children.
 * Rays along the axes and through the planes of flat boxes, and from inside.
-* A chain of nested boxes, every one of them met, whose pending nodes pass the
-  stack's room: the walk ends by the binary one.
+* A chain of nested boxes, every one of them met, and thin triangles as long
+  as the scene: more pending nodes than the stack's LDS entries.
 """
 import numpy as np
 import pytest
@@ -77,10 +77,10 @@ def test_axis_rays_flat_boxes_and_inside(gpu, orc):
     same(gpu, orc, walls, rays_of(np.concatenate([o, o]), np.concatenate([d, slant]), tmax=0.5), "walls, short rays")
 
 
-def test_more_pending_nodes_than_the_stack_holds(gpu, orc):
-    # Centres at 2^-k of the scene along one axis after the other: the tree is
-    # a chain some 28 levels deep, eight triangles off each level, and every
-    # box spans the scene's middle, where the rays start.
+def chain():
+    """Centres at 2^-k of the scene along one axis after the other: the tree is
+    a chain some 28 levels deep, eight triangles off each level, and every box
+    spans the scene's middle, where the rays start: 39 nodes are pending."""
     corners = []
     for k in range(27):
         c = np.array([0.5 ** (k // 3 + (k % 3 > a)) for a in range(3)]) * 4.0 - 2.0
@@ -88,7 +88,84 @@ def test_more_pending_nodes_than_the_stack_holds(gpu, orc):
         for j in range(8):
             e = half * (1.0 - 0.001 * j)
             corners.append([c + e * [1, 1, 1], c + e * [-1, -1, 0.5], c + e * [-1, 0.25 * (j - 4), -1]])
+    return np.array(corners)
+
+
+def test_more_pending_nodes_than_the_stack_holds(gpu, orc):
     rng = np.random.default_rng(5)
     d = rng.normal(size=(2000, 3))
     o = rng.uniform(-0.5, 0.5, (2000, 3))
-    same(gpu, orc, np.array(corners), rays_of(o, d / np.linalg.norm(d, axis=1)[:, None]), "chain")
+    same(gpu, orc, chain(), rays_of(o, d / np.linalg.norm(d, axis=1)[:, None]), "chain")
+
+
+def lit(corners):
+    """The triangles with a lamp among them, and a view from their middle."""
+    tris = S.tris_from_corners(np.asarray(corners, dtype=np.float32), color=(0.7, 0.6, 0.5, 1.0))
+    tris["emit"][::8] = 2.0
+    cam = S.path_camera(40, 24, eye=(0.11, -0.23, 0.17), target=(0.4, 0.6, 0.3), fov_deg=90.0, rr_from=3)
+    cam["env"] = (0.4, 0.5, 0.6, 0.0)
+    return tris, cam
+
+
+@pytest.fixture(scope="module")
+def chain_frame(orc):
+    tris, cam = lit(chain())
+    px = np.zeros(P.PX_LEN * 40 * 24 + 1, dtype=np.uint32)
+    sc = orc.Scene(tris, 4, P.NODE)
+    for f in range(2):
+        sc.sample(cam, 40, 24, px, f, nthreads=8)
+    return tris, cam, px
+
+
+def same_planes(got, want):
+    a, b = P.planes(got, 40, 24), P.planes(want, 40, 24)
+    for k in ("radiance", "albedo", "normal", "depth", "count", "missed"):
+        assert np.allclose(a[k], b[k], rtol=1e-5, atol=0), k  # the tracer's bound against the oracle
+
+
+@pytest.mark.parametrize("build", [0, 1, 2, 3], ids=["nested", "regen", "wavefront", "split"])
+def test_full_stacks_in_path_frames(gpu, chain_frame, build):
+    """The chain as a path frame, closest and shadow rays, at every register
+    fit (the split build's stacks hold 27 entries, 19 at five waves)."""
+    tris, cam, px = chain_frame
+    tr = P.Tracer.new(gpu, tris, 4)
+    tr.set_path_regen(build)
+    for waves in (2, 3, 4, 5):
+        tr.set_path_waves(waves)
+        tr.sample(cam, 40, 24, 2)
+        same_planes(tr.px(), px)
+        tr.sample(S.path_camera(41, 24), 41, 24, 1)  # another view: the next call starts over
+
+
+@pytest.mark.parametrize("build", [0, 3], ids=["nested", "split"])
+def test_full_stacks_in_a_batch(gpu, chain_frame, build):
+    tris, cam, px = chain_frame
+    b = P.Batch(gpu, np.concatenate([tris, tris]), np.array([0, len(tris), 2 * len(tris)], dtype=np.uint32))
+    b.set_path_build(build)
+    for waves in (2, 3, 4, 5):
+        b.set_path(waves, 0)
+        b.render(cam, 40, 24, 2)
+        for k in range(2):
+            same_planes(b.px(k), px)
+
+
+def test_a_full_stack_costs_no_second_walk(gpu):
+    """4,000 thin triangles as long as the scene: a third of the rays have more
+    nodes pending than the split build's 19 entries at five waves. They test
+    the triangles that rays with 27 entries test, and hardly a node more."""
+    rng = np.random.default_rng(4)
+    c = rng.uniform(0, 1, (4000, 1, 3))
+    u, v = rng.normal(size=(2, 4000, 1, 3))
+    u /= 2 * np.linalg.norm(u, axis=2, keepdims=True)
+    v *= 0.002 / np.linalg.norm(v, axis=2, keepdims=True)
+    tris, cam = lit(np.concatenate([c - u, c + u, c + v], 1))
+    tr = P.Tracer.new(gpu, tris, 4)
+    tr.set_path_regen(P.Tracer.PATH_SPLIT)
+    tests = {}
+    for waves in (2, 5):
+        before = tr.counters()[3]
+        tr.set_path_waves(waves)
+        tr.sample(cam, 40, 24, 1)
+        tests[waves] = int(tr.counters()[3] - before)
+        tr.sample(S.path_camera(41, 24, eye=(0.0, -60.0, 0.0), target=(0.0, -70.0, 0.0)), 41, 24, 1)
+    assert tests[5] < 1.05 * tests[2], tests
