@@ -59,10 +59,11 @@ namespace {
 // ---- walk -------------------------------------------------------------------
 struct RaySpace { uint32_t kz; bool flip; float sx, sy, sz; };
 
-__device__ __forceinline__ void ray_axes(float vx, float vy, float vz, uint32_t kz, bool flip, float& ox, float& oy, float& oz) {
-    float px = kz == 0 ? vy : (kz == 1 ? vz : vx);
-    float py = kz == 0 ? vz : (kz == 1 ? vx : vy);
-    float pz = kz == 0 ? vx : (kz == 1 ? vy : vz);
+template <class T>
+__device__ __forceinline__ void ray_axes(T vx, T vy, T vz, uint32_t kz, bool flip, T& ox, T& oy, T& oz) {
+    T px = kz == 0 ? vy : (kz == 1 ? vz : vx);
+    T py = kz == 0 ? vz : (kz == 1 ? vx : vy);
+    T pz = kz == 0 ? vx : (kz == 1 ? vy : vz);
     ox = flip ? py : px;
     oy = flip ? px : py;
     oz = pz;
@@ -79,28 +80,33 @@ __device__ __forceinline__ RaySpace ray_space(V3 d) {
     return RaySpace{kz, flip, x * sz, y * sz, sz};
 }
 
-// Returns t (PHR_INF on a miss) and the weights of b and c.
-__device__ __forceinline__ float tri_t(float4 t0, float4 t1, float4 t2, V3 o, const RaySpace& r, float& u, float& v) {
-    float ax, ay, az, bx, by, bz, cx, cy, cz;
-    ray_axes(t0.x - o.x, t0.y - o.y, t0.z - o.z, r.kz, r.flip, ax, ay, az);
-    ray_axes(t0.w - o.x, t1.x - o.y, t1.y - o.z, r.kz, r.flip, bx, by, bz);
-    ray_axes(t1.z - o.x, t1.w - o.y, t2.x - o.z, r.kz, r.flip, cx, cy, cz);
-    float sax = ax - r.sx * az, say = ay - r.sy * az;
-    float sbx = bx - r.sx * bz, sby = by - r.sy * bz;
-    float scx = cx - r.sx * cz, scy = cy - r.sy * cz;
+// The triangle test on corners given from the ray's origin in its axes:
+// returns t (PHR_INF on a miss) and the weights of b and c.
+__device__ __forceinline__ float tri_rel(V3 a, V3 b, V3 c, const RaySpace& r, float& u, float& v) {
+    float sax = a.x - r.sx * a.z, say = a.y - r.sy * a.z;
+    float sbx = b.x - r.sx * b.z, sby = b.y - r.sy * b.z;
+    float scx = c.x - r.sx * c.z, scy = c.y - r.sy * c.z;
     float ea = scx * sby - scy * sbx;
     float eb = sax * scy - say * scx;
     float ec = sbx * say - sby * sax;
     if ((ea < 0.f || eb < 0.f || ec < 0.f) && (ea > 0.f || eb > 0.f || ec > 0.f)) return PHR_INF;
     float det = ea + eb + ec;
     if (det == 0.f) return PHR_INF;
-    float tt = ea * (r.sz * az) + eb * (r.sz * bz) + ec * (r.sz * cz);
+    float tt = ea * (r.sz * a.z) + eb * (r.sz * b.z) + ec * (r.sz * c.z);
     float sg = det < 0.f ? -1.0f : 1.0f;
     if (tt * sg <= 0.f) return PHR_INF;
     float inv = 1.0f / det;
     u = eb * inv;
     v = ec * inv;
     return tt * inv;
+}
+// The same on a triangle cache row, from the origin.
+__device__ __forceinline__ float tri_t(float4 t0, float4 t1, float4 t2, V3 o, const RaySpace& r, float& u, float& v) {
+    V3 a, b, c;
+    ray_axes(t0.x - o.x, t0.y - o.y, t0.z - o.z, r.kz, r.flip, a.x, a.y, a.z);
+    ray_axes(t0.w - o.x, t1.x - o.y, t1.y - o.z, r.kz, r.flip, b.x, b.y, b.z);
+    ray_axes(t1.z - o.x, t1.w - o.y, t2.x - o.z, r.kz, r.flip, c.x, c.y, c.z);
+    return tri_rel(a, b, c, r, u, v);
 }
 
 __device__ __forceinline__ V3 safe_inv(V3 d) {  // bvh.wgsl:111-114
@@ -120,24 +126,100 @@ __device__ __forceinline__ float box_t(float4 lo, float4 hi, V3 o, V3 inv, float
 }
 
 // ---- the wide walk ---------------------------------------------------------
-// A closest hit is the least t over the triangles the ray meets, and of equal
-// t's the first in the binary walk's order; a shadow ray only asks whether
-// anything blocks it. Neither depends on the order the walk takes, so one
-// tree is walked four boxes at a time: each inner node x has a record of up
+// One tree is walked four boxes at a time: each inner node x has a record of up
 // to four descendants (x's children, the widest inner one opened, then the
 // widest of those), as rows of one coordinate of all four, and a child word
 // each: an inner child's node index, a leaf's first | LEAF (its end sits in
 // row 2 .y of its first triangle's cache row), PHR_NONE for no child (its box
-// is NaN and never met). On the 1.31M-triangle spheres scene a ray takes 11.7
+// is NaN and never met). On the 1.31M-triangle spheres scene a ray takes 12
 // such visits where the binary records took 14.5 two-level ones, and a visit
 // is shorter: near and far planes are picked by address from the ray's signs
 // (no min / max a plane) and only the nearest child is sorted out (the others
 // pushed as they lie: 1% more visits than a full sort).
 //
-// Every box's test is box_t's, product for product, so a leaf is met exactly
-// where the binary walk would meet it (a box inside another is met only where
-// the other is, since rounding keeps the order of the planes); a box the ray
-// enters at the very t of the hit in hand is still entered, for a tie.
+// The hit is the binary walk's, bit for bit, whatever order the boxes are met
+// in. The binary walk enters a box up to the t of the hit in hand, and a
+// triangle's t can round below the t at which its box is entered, so in that
+// walk it can depend on the order whether a triangle is tested. It does not
+// where no two triangles lie close together on the ray, and the wide walk makes
+// sure of that:
+//   * It culls by the slab of the ray's dominant axis alone, against the hit's
+//     t times WIDE_MARGIN. A triangle's t is a mean, with weights of one sign,
+//     of its corners' t along that axis, so (underflow aside) it lies at most 7
+//     roundings below the slab: no triangle within the margin goes untested.
+//     The whole box would save 1 to 2% of a ray's visits (4 to 11% among thin
+//     triangles a tenth to a third of the scene long), but t has no such bound
+//     against the other two axes' entries where a triangle is seen edge-on.
+//   * A hit is in doubt if another triangle, or the ray's end, lies within the
+//     margin, or if its own box is entered beyond it. If not, every other
+//     triangle is beyond the entry of the hit's leaf, so the binary walk tests
+//     it, and it is the nearest.
+//   * A shadow ray's blocker must have its own box entered before the ray's
+//     end: then the binary walk tests it too.
+// A ray in doubt is walked again in the binary order. Of 50,000 rays of path
+// frames none was; of rays aimed at the edges of a flat grid 1 in 100, of rays
+// at two layers in one plane a quarter. (Without all this the 1080p 64-spp
+// spheres frame takes 3% less, and of 24 such frames, previews and batches one
+// had a pixel that was not the binary walk's.)
+constexpr float WIDE_MARGIN = 1.000004f;  // 67 roundings
+constexpr float WIDE_ENTRY = 1.000001f;   // 16: more than the 7 above, less than the margin
+// The ray in its own axes (ray_axes), its shear, and the byte offsets of its
+// near rows in a record, 8 bits an axis: lo where it goes up the axis, else hi.
+// The last axis' offset holds kz; flip is the bit above.
+struct WideRay {
+    V3 o, inv;
+    float sx, sy, sz;
+    uint32_t rows;
+    __device__ __forceinline__ uint32_t kz() const { return (rows >> 21) & 3u; }
+    __device__ __forceinline__ bool flip() const { return (rows >> 24) != 0u; }
+    __device__ __forceinline__ RaySpace space() const { return RaySpace{kz(), flip(), sx, sy, sz}; }
+    __device__ __forceinline__ V3 axes(float x, float y, float z) const {
+        V3 v;
+        ray_axes(x, y, z, kz(), flip(), v.x, v.y, v.z);
+        return v;
+    }
+};
+__device__ __forceinline__ WideRay wide_ray(V3 o, V3 d) {
+    const RaySpace rs = ray_space(d);
+    const V3 inv = safe_inv(d);
+    WideRay r;
+    uint32_t x, y, z;
+    ray_axes(0u, 32u, 64u, rs.kz, rs.flip, x, y, z);
+    r.rows = x | y << 8 | z << 16 | (rs.flip ? 1u << 24 : 0u);
+    r.o = r.axes(o.x, o.y, o.z);
+    r.inv = r.axes(inv.x, inv.y, inv.z);
+    r.rows |= ((__float_as_uint(r.inv.x) >> 27) & 16u) | ((__float_as_uint(r.inv.y) >> 19) & (16u << 8)) |
+              ((__float_as_uint(r.inv.z) >> 11) & (16u << 16));
+    r.sx = rs.sx;
+    r.sy = rs.sy;
+    r.sz = rs.sz;
+    return r;
+}
+struct RelTri {
+    V3 a, b, c;  // the corners from the ray's origin, in its axes
+};
+__device__ __forceinline__ RelTri rel_tri(float4 t0, float4 t1, float4 t2, const WideRay& r) {
+    return RelTri{r.axes(t0.x, t0.y, t0.z) - r.o, r.axes(t0.w, t1.x, t1.y) - r.o, r.axes(t1.z, t1.w, t2.x) - r.o};
+}
+// Where the ray enters the triangle's own box, at or beyond its leaf's.
+__device__ __forceinline__ float own_entry(const RelTri& q, const WideRay& r) {
+    auto near = [](float a, float b, float c, float inv) {
+        return (__float_as_int(inv) < 0 ? fmaxf(fmaxf(a, b), c) : fminf(fminf(a, b), c)) * inv;
+    };
+    return fmaxf(fmaxf(fmaxf(near(q.a.x, q.b.x, q.c.x, r.inv.x), near(q.a.y, q.b.y, q.c.y, r.inv.y)), near(q.a.z, q.b.z, q.c.z, r.inv.z)),
+                 0.f);
+}
+// Whether a triangle at t and the nearest so far (or the ray's end, where there
+// is none) lie within the margin.
+__device__ __forceinline__ bool too_close(float t, float best_t, bool found) {
+    return (found || t < best_t) && t * WIDE_MARGIN >= best_t && t <= best_t * WIDE_MARGIN;
+}
+// Whether the hit a walk ended with (a blocker of a shadow ray of length t where
+// `any`) may be one the binary walk does not test.
+__device__ __forceinline__ bool entered_late(const SceneDev& s, const WideRay& r, uint32_t id, float t, bool any) {
+    const float e = own_entry(rel_tri(s.tris[3 * (size_t)id], s.tris[3 * (size_t)id + 1], s.tris[3 * (size_t)id + 2], r), r);
+    return any ? !(e < t) : !(e * WIDE_ENTRY <= t * WIDE_MARGIN);
+}
 constexpr uint32_t WIDE_ROWS = 8;  // lo.x hi.x lo.y hi.y lo.z hi.z words, one row unused: 128 B, one cache line
 
 // A wide visit needs three free entries of the walk's LDS column.
@@ -148,18 +230,18 @@ typedef float vec4 __attribute__((ext_vector_type(4)));
 // The visit of inner node `cur`: the nearest child met is entered (cur), the
 // others are pushed. False when none is met. The stack has room.
 template <uint32_t STRIDE>
-__device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float best_t, uint32_t& cur, uint32_t* stk, uint32_t& sp) {
-    // A ray's near x, y and z rows: lo where it goes up the axis, else hi.
-    const uint32_t nx = (__float_as_uint(inv.x) >> 27) & 16u, ny = (__float_as_uint(inv.y) >> 27) & 16u,
-                   nz = (__float_as_uint(inv.z) >> 27) & 16u;
+__device__ __forceinline__ bool visit4(const SceneDev& s, const WideRay& ray, float best_t, uint32_t& cur, uint32_t* stk, uint32_t& sp) {
+    const uint32_t nx = ray.rows & 0xffu, ny = (ray.rows >> 8) & 0xffu, nz = (ray.rows >> 16) & 0xffu;
+    const V3 o = ray.o, inv = ray.inv;
+    const float limit = best_t * WIDE_MARGIN;
     const char* r = (const char*)s.wide + (uint64_t)cur * (16u * WIDE_ROWS);
-    auto row = [&](uint32_t off, uint32_t at) { return *(const vec4*)(r + off + at); };
-    const vec4 ax = row(nx, 0u), bx = row(nx ^ 16u, 0u), ay = row(ny, 32u), by = row(ny ^ 16u, 32u), az = row(nz, 64u),
-               bz = row(nz ^ 16u, 64u), wd = row(96u, 0u);
+    auto row = [&](uint32_t at) { return *(const vec4*)(r + at); };
+    const vec4 ax = row(nx), bx = row(nx ^ 16u), ay = row(ny), by = row(ny ^ 16u), az = row(nz), bz = row(nz ^ 16u), wd = row(96u);
     auto child = [&](float x0, float x1, float y0, float y1, float z0, float z1) {  // where the ray enters, PHR_INF on a miss
-        const float tn = fmaxf(fmaxf(fmaxf((x0 - o.x) * inv.x, (y0 - o.y) * inv.y), (z0 - o.z) * inv.z), 0.f);
+        const float tz = (z0 - o.z) * inv.z;
+        const float tn = fmaxf(fmaxf(fmaxf((x0 - o.x) * inv.x, (y0 - o.y) * inv.y), tz), 0.f);
         const float tf = fminf(fminf((x1 - o.x) * inv.x, (y1 - o.y) * inv.y), (z1 - o.z) * inv.z);
-        return (tn <= tf && tn <= best_t) ? tn : PHR_INF;
+        return (tn <= tf && tz <= limit) ? tn : PHR_INF;
     };
     float k0 = child(ax.x, bx.x, ay.x, by.x, az.x, bz.x), k1 = child(ax.y, bx.y, ay.y, by.y, az.y, bz.y);
     float k2 = child(ax.z, bx.z, ay.z, by.z, az.z, bz.z), k3 = child(ax.w, bx.w, ay.w, by.w, az.w, bz.w);
@@ -187,57 +269,31 @@ __device__ __forceinline__ bool visit4(const SceneDev& s, V3 o, V3 inv, float be
 }
 // The largest t below a positive one.
 __device__ __forceinline__ float below(float t) { return __uint_as_float(__float_as_uint(t) - 1u); }
-// A visit a level at a time, from the nodes: of cur's two children those
-// entered up to `limit` are met, the nearer (a tie to the left) is entered, the
-// other pushed.
+// A visit a level at a time, from the nodes: of cur's two children that are
+// met the nearer (a tie to the left) is entered, the other pushed. `binary`: met
+// as the binary walk meets them, else as visit4 does.
 template <class STACK>
-__device__ __forceinline__ bool visit1(const SceneDev& s, V3 o, V3 inv, float limit, uint32_t& cur, const STACK& stk, uint32_t& sp) {
+__device__ __forceinline__ bool visit1(const SceneDev& s, const WideRay& ray, float best_t, bool binary, uint32_t& cur, const STACK& stk,
+                                       uint32_t& sp) {
     const uint32_t l = __float_as_uint(s.nodes[2 * (size_t)cur].w), r = __float_as_uint(s.nodes[2 * (size_t)cur + 1].w);
+    const float limit = binary ? below(best_t) : best_t * WIDE_MARGIN;
     const float4 llo = s.nodes[2 * (size_t)l], lhi = s.nodes[2 * (size_t)l + 1];
     const float4 rlo = s.nodes[2 * (size_t)r], rhi = s.nodes[2 * (size_t)r + 1];
-    float tl = box_t(llo, lhi, o, inv, PHR_INF), tr = box_t(rlo, rhi, o, inv, PHR_INF);
-    tl = tl <= limit ? tl : PHR_INF;
-    tr = tr <= limit ? tr : PHR_INF;
-    const uint32_t wl = (__float_as_uint(llo.w) & PHR_LEAF) ? __float_as_uint(llo.w) : l;
-    const uint32_t wr = (__float_as_uint(rlo.w) & PHR_LEAF) ? __float_as_uint(rlo.w) : r;
+    auto enter = [&](float4 lo, float4 hi) {
+        const V3 a = ray.axes(lo.x, lo.y, lo.z), b = ray.axes(hi.x, hi.y, hi.z);
+        const float e = box_t(make_float4(a.x, a.y, a.z, 0.f), make_float4(b.x, b.y, b.z, 0.f), ray.o, ray.inv, PHR_INF);
+        const float tz = ((__float_as_int(ray.inv.z) < 0 ? b.z : a.z) - ray.o.z) * ray.inv.z;
+        return (binary ? e : tz) <= limit ? e : PHR_INF;
+    };
+    auto word = [](float4 lo, uint32_t y) { return (__float_as_uint(lo.w) & PHR_LEAF) ? __float_as_uint(lo.w) : y; };
+    const uint32_t wl = word(llo, l), wr = word(rlo, r);
+    const float tl = enter(llo, lhi), tr = enter(rlo, rhi);
     const bool left = tl <= tr;
     if ((left ? tr : tl) < PHR_INF) stk.push(sp, left ? wr : wl);
     cur = left ? wl : wr;
     return (left ? tl : tr) < PHR_INF;
 }
 
-// The first slot of the tree under node x: its leftmost leaf's.
-__device__ __forceinline__ uint32_t first_slot(const SceneDev& s, uint32_t x) {
-    uint32_t w = __float_as_uint(s.nodes[2 * (size_t)x].w);
-    while (!(w & PHR_LEAF)) w = __float_as_uint(s.nodes[2 * (size_t)w].w);
-    return w & ~PHR_LEAF;
-}
-// Of two triangles (slots a and b) the ray meets at the same t, whether a
-// comes first in the binary walk: at the node where their ways part, the
-// nearer child does (a tie to the left); within a leaf, the lower slot.
-__device__ __forceinline__ bool first_of(const SceneDev& s, V3 o, V3 inv, uint32_t a, uint32_t b) {
-    uint32_t x = s.root;
-    for (;;) {
-        const float4 lo = s.nodes[2 * (size_t)x], hi = s.nodes[2 * (size_t)x + 1];
-        const uint32_t l = __float_as_uint(lo.w), r = __float_as_uint(hi.w);
-        if (l & PHR_LEAF) return a < b;
-        const uint32_t split = first_slot(s, r);
-        const bool a_left = a < split, b_left = b < split;
-        if (a_left == b_left) {
-            x = a_left ? l : r;
-            continue;
-        }
-        const float tl = box_t(s.nodes[2 * (size_t)l], s.nodes[2 * (size_t)l + 1], o, inv, PHR_INF);
-        const float tr = box_t(s.nodes[2 * (size_t)r], s.nodes[2 * (size_t)r + 1], o, inv, PHR_INF);
-        return (tl <= tr) == a_left;
-    }
-}
-// Whether a triangle met at t replaces the hit (best_t, best): the nearer one
-// does, and of two at one t the binary walk's first.
-__device__ __forceinline__ bool takes(const SceneDev& s, V3 o, V3 inv, float t, uint32_t id, float best_t, uint32_t best) {
-    if (t < best_t) return true;
-    return t == best_t && best != PHR_NONE && id != best && first_of(s, o, inv, id, best);
-}
 __device__ __forceinline__ bool blocks(const SceneDev& s, uint32_t id) {  // bvh.wgsl:158-160: glass and cut-outs pass
     const float* m = s.mats + MAT_WORDS * (size_t)s.faces[id].w;
     return !(m[6] > 0.5f || m[3] < 0.5f);
@@ -258,25 +314,25 @@ struct LevelStack {
     uint32_t* lds;
     __device__ __forceinline__ void push(uint32_t& sp, uint32_t word) const { lds[sp++ * STRIDE] = word; }
 };
-// The walk a level at a time, in the binary walk's order: where a wide walk's
-// stack is full. (No ray of 3,000 through 50,000 triangles as long as the
-// scene fills 32 entries; it takes boxes nested in one another.)
+// The binary walk, for a ray whose wide walk is in doubt or has its stack full
+// (none of 3,000 rays through 50,000 triangles as long as the scene fills 32
+// entries; it takes boxes nested in one another).
 template <bool ANY, uint32_t STRIDE>
-__device__ __forceinline__ PhrHit walk_binary(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* lds, uint32_t& steps, uint32_t& tests) {
+__device__ __forceinline__ PhrHit walk_binary(const SceneDev& s, const WideRay& r, float tmax, uint32_t only, uint32_t* lds, uint32_t& steps,
+                                              uint32_t& tests) {
     PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
-    const V3 inv = safe_inv(d);
-    const RaySpace rs = ray_space(d);
     const LevelStack<STRIDE> stk{lds};
-    uint32_t sp = 0, cur = s.root;  // an inner node, or the wide walk had not begun
+    uint32_t sp = 0, cur = only != PHR_NONE ? __float_as_uint(s.nodes[2 * (size_t)s.root].w) : s.root;
     for (;;) {
         if (cur & PHR_LEAF) {
-            uint32_t id = cur & ~PHR_LEAF, end = PHR_NONE;
+            uint32_t id = cur & ~PHR_LEAF, end = only;
             do {
                 ++tests;
                 const float4 t0 = s.tris[3 * (size_t)id], t1 = s.tris[3 * (size_t)id + 1], t2 = s.tris[3 * (size_t)id + 2];
                 if (end == PHR_NONE) end = __float_as_uint(t2.y);
+                const RelTri q = rel_tri(t0, t1, t2, r);
                 float u, v;
-                const float t = tri_t(t0, t1, t2, o, rs, u, v);
+                const float t = tri_rel(q.a, q.b, q.c, r.space(), u, v);
                 if (t < best.t && (!ANY || blocks(s, id))) {
                     best = PhrHit{t, id, u, v, 0u};
                     if constexpr (ANY) return best;
@@ -284,7 +340,7 @@ __device__ __forceinline__ PhrHit walk_binary(const SceneDev& s, V3 o, V3 d, flo
             } while (++id < end);
         } else {
             ++steps;
-            if (visit1(s, o, inv, below(best.t), cur, stk, sp)) continue;
+            if (visit1(s, r, best.t, true, cur, stk, sp)) continue;
         }
         if (sp == 0) return best;
         cur = lds[--sp * STRIDE];
@@ -298,9 +354,9 @@ __device__ __forceinline__ PhrHit walk_binary(const SceneDev& s, V3 o, V3 d, flo
 template <bool ANY, uint32_t STRIDE>
 __device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax, uint32_t* lds, uint32_t& steps, uint32_t& tests) {
     PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
-    const V3 inv = safe_inv(d);
-    const RaySpace rs = ray_space(d);
+    const WideRay r = wide_ray(o, d);
     uint32_t sp = 0, only, cur = wide_root(s, only);
+    bool doubt = false;
     for (;;) {
         if (cur & PHR_LEAF) {
             uint32_t id = cur & ~PHR_LEAF;
@@ -316,29 +372,28 @@ __device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax
                     n1 = s.tris[3 * (size_t)(id + 1u) + 1];
                     n2 = s.tris[3 * (size_t)(id + 1u) + 2];
                 }
+                const RelTri q = rel_tri(t0, t1, t2, r);
                 float u, v;
-                const float t = tri_t(t0, t1, t2, o, rs, u, v);
-                if constexpr (ANY) {
-                    if (t < best.t && blocks(s, id)) return PhrHit{t, id, u, v, 0u};
-                } else {
-                    if (takes(s, o, inv, t, id, best.t, best.tri)) best = PhrHit{t, id, u, v, 0u};
-                }
-                if (!more) break;
+                const float t = tri_rel(q.a, q.b, q.c, r.space(), u, v);
+                if (!ANY && too_close(t, best.t, best.tri != PHR_NONE)) doubt = true;
+                if (t < best.t && (!ANY || blocks(s, id))) best = PhrHit{t, id, u, v, 0u};
+                if (!more || (ANY && best.tri != PHR_NONE)) break;
                 ++id;
                 t0 = n0;
                 t1 = n1;
                 t2 = n2;
             }
         } else if (!wide_room<PHR_STACK>(sp)) {
-            return walk_binary<ANY, STRIDE>(s, o, d, tmax, lds, steps, tests);
+            doubt = true;
         } else {
             ++steps;
-            if (visit4<STRIDE>(s, o, inv, best.t, cur, lds, sp)) continue;
+            if (visit4<STRIDE>(s, r, best.t, cur, lds, sp)) continue;
         }
-        if (sp == 0) break;
+        if (doubt || sp == 0 || (ANY && best.tri != PHR_NONE)) break;
         cur = lds[--sp * STRIDE];
     }
-    return best;
+    if (best.tri != PHR_NONE && entered_late(s, r, best.tri, ANY ? tmax : best.t, ANY)) doubt = true;
+    return doubt ? walk_binary<ANY, STRIDE>(s, r, tmax, only, lds, steps, tests) : best;
 }
 
 // ---- the ordered any-hit walk -------------------------------------------------
@@ -468,7 +523,10 @@ __device__ __forceinline__ PhrHit walk_first(const SceneDev& s, V3 o, V3 d, floa
 // stack (sp entries of the thread's column). A unit is an inner node's visit
 // or a leaf's triangles. A leaf reached is put by and the walk goes on from
 // the stack, until a second leaf is reached or nothing else is left.
-// `any`: a shadow ray's walk, which ends at the first triangle that blocks it.
+// `any`: a shadow ray's walk, which ends at the first triangle that blocks it;
+// the others begin with t at PHR_INF. `doubt`, `binary`: a walk in doubt is begun
+// again in the binary walk's order, where a leaf put by is tested before the
+// walk goes on.
 // The split build's stack: N LDS entries (a pixel's sums have the rest of the
 // column) and then scratch. With no room for a wide visit it visits a level at a
 // time. The N entries then come from at least N / 3 of the path's 31 inner
@@ -494,11 +552,10 @@ struct DeepStack {
     }
 };
 struct Walker {
-    V3 o, inv;
-    RaySpace rs;
+    WideRay r;
     float t, u, v;  // closest: the nearest hit so far; shadow: t is the ray's length
     uint32_t tri, cur, leaf, sp;  // cur, leaf: PHR_NONE when there is none
-    bool on, any;
+    bool on, any, doubt, binary;
 };
 template <bool DEEP, class STACK>
 __device__ __forceinline__ void walker_pop(Walker& w, const STACK& stk) {
@@ -511,31 +568,43 @@ __device__ __forceinline__ void walker_settle(Walker& w, const STACK& stk) {
     if (w.leaf == PHR_NONE && (w.cur & PHR_LEAF)) {
         w.leaf = w.cur;
         w.on = w.cur != PHR_NONE;
-        if (w.on) walker_pop<DEEP>(w, stk);
+        if (w.on && !w.binary) walker_pop<DEEP>(w, stk);
+        else w.cur = PHR_NONE;
     }
 }
-__device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, uint32_t root, V3 o, V3 d, float tmax, bool any) {
-    w.o = o;
-    w.inv = safe_inv(d);
-    w.rs = ray_space(d);
-    w.t = tmax;
-    w.u = w.v = 0.f;
+__device__ __forceinline__ void walker_root(Walker& w, uint32_t root) {
     w.tri = PHR_NONE;
     w.sp = 0;
-    w.any = any;
-    w.on = true;
     const bool leaf = (root & PHR_LEAF) != 0u;
     w.cur = leaf ? PHR_NONE : root;
     w.leaf = leaf ? root : PHR_NONE;
 }
+__device__ __forceinline__ void walker_begin(Walker& w, uint32_t root, V3 o, V3 d, float tmax, bool any) {
+    w.r = wide_ray(o, d);
+    w.t = tmax;
+    w.u = w.v = 0.f;
+    w.any = any;
+    w.on = true;
+    w.doubt = w.binary = false;
+    walker_root(w, root);
+}
+// A walk that ended: begun again if its answer is in doubt.
+__device__ __forceinline__ bool walker_again(Walker& w, const SceneDev& s, uint32_t root) {
+    if (w.binary || (!w.doubt && (w.tri == PHR_NONE || !entered_late(s, w.r, w.tri, w.t, w.any)))) return false;
+    if (!w.any) w.t = PHR_INF;
+    w.u = w.v = 0.f;
+    w.on = w.binary = true;
+    walker_root(w, root);
+    return true;
+}
 template <uint32_t N, uint32_t STRIDE>
 __device__ __forceinline__ void walker_visit(Walker& w, const SceneDev& s, const DeepStack<N, STRIDE>& stk, uint32_t& steps) {
     ++steps;
-    if (wide_room<N>(w.sp)) {
-        if (!visit4<STRIDE>(s, w.o, w.inv, w.t, w.cur, stk.lds, w.sp)) walker_pop<false>(w, stk);
+    if (!w.binary && wide_room<N>(w.sp)) {
+        if (!visit4<STRIDE>(s, w.r, w.t, w.cur, stk.lds, w.sp)) walker_pop<false>(w, stk);
         walker_settle<false>(w, stk);
     } else {
-        if (!visit1(s, w.o, w.inv, w.t, w.cur, stk, w.sp)) walker_pop<true>(w, stk);
+        if (!visit1(s, w.r, w.t, w.binary, w.cur, stk, w.sp)) walker_pop<true>(w, stk);
         walker_settle<true>(w, stk);
     }
 }
@@ -556,19 +625,23 @@ __device__ __forceinline__ void walker_leaf(Walker& w, const SceneDev& s, uint32
             n1 = s.tris[3 * (size_t)(id + 1u) + 1];
             n2 = s.tris[3 * (size_t)(id + 1u) + 2];
         }
+        const RelTri q = rel_tri(t0, t1, t2, w.r);
         float u, v;
-        const float t = tri_t(t0, t1, t2, w.o, w.rs, u, v);
+        const float t = tri_rel(q.a, q.b, q.c, w.r.space(), u, v);
         if (w.any) {
             if (t < w.t && blocks(s, id)) {
                 w.tri = id;
                 w.on = false;
                 return;
             }
-        } else if (takes(s, w.o, w.inv, t, id, w.t, w.tri)) {
-            w.t = t;
-            w.tri = id;
-            w.u = u;
-            w.v = v;
+        } else {
+            if (too_close(t, w.t, w.tri != PHR_NONE)) w.doubt = true;
+            if (t < w.t) {
+                w.t = t;
+                w.tri = id;
+                w.u = u;
+                w.v = v;
+            }
         }
         if (!more) break;
         ++id;
@@ -576,6 +649,7 @@ __device__ __forceinline__ void walker_leaf(Walker& w, const SceneDev& s, uint32
         t1 = n1;
         t2 = n2;
     }
+    if (w.binary) walker_pop<true>(w, stk);
     walker_settle<true>(w, stk);
 }
 
@@ -2069,7 +2143,7 @@ struct SplitWalk {
     Walker w;
     uint32_t root, only;
     __device__ __forceinline__ void scene(const SceneDev& s) { root = wide_root(s, only); }
-    __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, s, root, o, d, tmax, any); }
+    __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, root, o, d, tmax, any); }
     // The wave's next unit: the lanes at an inner node visit it while they are
     // enough; once LEAF8 eighths of the walks have a leaf put by and nothing
     // to visit, every lane with a leaf put by tests its triangles.
@@ -2085,6 +2159,7 @@ struct SplitWalk {
             walker_visit(w, s, stk, steps);
         }
     }
+    __device__ __forceinline__ bool again(const SceneDev& s) { return walker_again(w, s, root); }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, 0u}; }
 };
 template <>
@@ -2115,6 +2190,7 @@ struct SplitWalk<true> {
             if (leaf && !tri) forest_between(w, s, tstk, stk, SPLIT_THREADS);
         }
     }
+    __device__ __forceinline__ bool again(const SceneDev&) { return false; }
     __device__ __forceinline__ PhrHit hit() const { return PhrHit{w.t, w.tri, w.u, w.v, w.hinst}; }
 };
 
@@ -2229,7 +2305,7 @@ __device__ __forceinline__ void path_split(const SceneDev& sc, const PhrCamera* 
             if (waiting == working || 8u * waiting >= shade8 * working) break;
             sw.template step<STK>(sc, stk, deep, tstk, steps, tests);
         }
-        if (!live || w.on) continue;
+        if (!live || w.on || sw.again(sc)) continue;
         bool next = false;
         if (w.any) {  // the turn's shadow ray has its answer
             const bool blocked = w.tri != PHR_NONE;
@@ -2515,11 +2591,10 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
     const uint32_t* queue = ANY ? w.sq : (parity ? w.q1 : w.q0);
     const uint32_t lane = threadIdx.x & 63u;
     PhrHit best{PHR_INF, PHR_NONE, 0.f, 0.f, 0u};
-    V3 o = v3(0, 0, 0), inv = o;
-    RaySpace rs{};
+    WideRay r{};
     uint32_t cur = 0, sp = 0, slot = 0;
     uint32_t steps = 0, tests = 0, nrays = 0;
-    bool live = false, drained = count == 0u, binary = false;
+    bool live = false, drained = count == 0u, doubt = false, binary = false;
     uint32_t cbase = 0, cend = 0;  // the wave's chunk of the queue
     uint32_t only;
     const uint32_t root = wide_root(sc, only);
@@ -2548,12 +2623,12 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
         }
         if (nidle >= 32u && cbase < cend) {  // refill the idle lanes from the chunk
             const uint32_t take = min(nidle, cend - cbase);
-            const uint32_t r = lanes_below(idle);
-            const uint32_t my = cbase + r;
+            const uint32_t rank = lanes_below(idle);
+            const uint32_t my = cbase + rank;
             cbase += take;
-            if (!live && r < take) {
+            if (!live && rank < take) {
                 slot = queue[my];
-                V3 d;
+                V3 o, d;
                 float tmax;
                 if constexpr (ANY) {
                     const float4 a = w.sh[4 * (size_t)slot], b = w.sh[4 * (size_t)slot + 1];
@@ -2568,12 +2643,11 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                 }
                 ++nrays;
                 best = PhrHit{tmax, PHR_NONE, 0.f, 0.f, 0u};
-                inv = safe_inv(d);
-                rs = ray_space(d);
+                r = wide_ray(o, d);
                 sp = 0;
                 cur = root;
                 live = true;
-                binary = false;
+                doubt = binary = false;
             }
         }
         if (__ballot(live) == 0ull) {
@@ -2590,27 +2664,24 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                 ++tests;
                 const float4 t0 = sc.tris[3 * (size_t)id], t1 = sc.tris[3 * (size_t)id + 1], t2 = sc.tris[3 * (size_t)id + 2];
                 if (end == PHR_NONE) end = __float_as_uint(t2.y);
+                const RelTri q = rel_tri(t0, t1, t2, r);
                 float u, v;
-                const float t = tri_t(t0, t1, t2, o, rs, u, v);
-                if constexpr (ANY) {
-                    if (t < best.t && blocks(sc, id)) {
-                        best = PhrHit{t, id, u, v, 0u};
+                const float t = tri_rel(q.a, q.b, q.c, r.space(), u, v);
+                if (!ANY && too_close(t, best.t, best.tri != PHR_NONE)) doubt = true;
+                if (t < best.t && (!ANY || blocks(sc, id))) {
+                    best = PhrHit{ANY ? best.t : t, id, u, v, 0u};
+                    if constexpr (ANY) {
                         more = false;
                         break;
                     }
-                } else if (takes(sc, o, inv, t, id, best.t, best.tri)) {
-                    best = PhrHit{t, id, u, v, 0u};
                 }
             } while (++id < end);
+        } else if (!binary && !wide_room<PHR_STACK>(sp)) {
+            doubt = true;
+            more = false;
         } else {
             ++steps;
-            if (!binary && !wide_room<PHR_STACK>(sp)) {  // the stack is full: again, a level at a time (walk_binary)
-                binary = true;
-                sp = 0;
-                cur = root;
-                if constexpr (!ANY) best = PhrHit{PHR_INF, PHR_NONE, 0.f, 0.f, 0u};
-            }
-            popped = !(binary ? visit1(sc, o, inv, below(best.t), cur, stk, sp) : visit4<WF_THREADS>(sc, o, inv, best.t, cur, stk.lds, sp));
+            popped = !(binary ? visit1(sc, r, best.t, true, cur, stk, sp) : visit4<WF_THREADS>(sc, r, best.t, cur, stk.lds, sp));
         }
         if (more && popped) {
             if (sp == 0) {
@@ -2618,6 +2689,12 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
             } else {
                 cur = stk.lds[--sp * WF_THREADS];
             }
+        }
+        if (!more && !binary && (doubt || (best.tri != PHR_NONE && entered_late(sc, r, best.tri, best.t, ANY)))) {
+            binary = more = true;  // again in the binary walk's order (walk_binary)
+            sp = 0;
+            cur = root;
+            best = PhrHit{ANY ? best.t : PHR_INF, PHR_NONE, 0.f, 0.f, 0u};
         }
         if (!more) {
             finish();

@@ -4,6 +4,8 @@ hits must equal the oracle's binary walk bit for bit.
 * Rays through the shared edges and corners of a regular grid, whose
   coordinates are exact in binary: several triangles in different leaves are
   met at the very same t, and the binary walk's first must be kept.
+* Slanted rays at edges and at two layers in one plane, at coordinates that are
+  not exact: triangles met within a few roundings of each other.
 * Scenes of one to nine triangles: a root that is a leaf, records with one to
   four children.
 * Rays along the axes and through the planes of flat boxes, and from inside.
@@ -37,9 +39,9 @@ def same(gpu, orc, corners, rays, what):
     return want
 
 
-def grid(n, tilt=0.0):
+def grid(n, tilt=0.0, z=0.0):
     x, y = np.meshgrid(np.arange(n + 1), np.arange(n + 1), indexing="ij")
-    p = np.stack([x / 8.0, y / 8.0, tilt * (x + 2 * y) / 8.0], -1)
+    p = np.stack([x / 8.0, y / 8.0, tilt * (x + 2 * y) / 8.0 + z], -1)
     a, b, c, d = p[:-1, :-1], p[1:, :-1], p[1:, 1:], p[:-1, 1:]
     return np.concatenate([np.stack([a, b, c], -2).reshape(-1, 3, 3), np.stack([a, c, d], -2).reshape(-1, 3, 3)])
 
@@ -54,6 +56,73 @@ def test_rays_through_shared_edges(gpu, orc, tilt):
     up = rays_of(np.concatenate([o, o * [1, 1, -1]]), np.concatenate([d, -d]))
     want = same(gpu, orc, grid(n, tilt), up, f"grid tilt {tilt}")
     assert (want[:, 1] != P.NONE).mean() > 0.9
+
+
+def towards(corners, count, seed, spread):
+    """Rays at points on the triangles' edges, from all round them."""
+    rng = np.random.default_rng(seed)
+    e, k, f = rng.integers(0, len(corners), count), rng.integers(0, 3, count), rng.uniform(0, 1, (count, 1))
+    to = corners[e, k] * f + corners[e, (k + 1) % 3] * (1 - f)
+    o = to + rng.uniform(-1, 1, (count, 3)) * spread
+    d = to - o
+    return o, d / np.linalg.norm(d, axis=1)[:, None], np.linalg.norm(d, axis=1)
+
+
+def layers():
+    """Two floors in one plane, at coordinates that are not exact in binary."""
+    return np.concatenate([grid(24, z=0.1), grid(23, z=0.1) + np.array([0.03, 0.07, 0.0])]).astype(np.float32)
+
+
+# Near an edge or in the overlap two triangles are met within a few roundings of
+# each other, and t can round below the t of the triangle's own box: which of
+# them the binary walk tests depends on its order.
+@pytest.mark.parametrize("scene", ["grid", "layers", "spheres"])
+def test_slanted_rays_at_edges_and_layers(gpu, orc, scene):
+    if scene == "spheres":
+        t = S.spheres_scene(8, 3, 1)
+        corners = np.stack([t["a"], t["b"], t["c"]], 1)
+    else:
+        corners = grid(24, z=0.1).astype(np.float32) if scene == "grid" else layers()
+    o, d, ln = towards(corners.astype(np.float64), 200_000, 6, np.array([4.0, 4.0, 4.0]))
+    same(gpu, orc, corners, rays_of(o, d), scene)
+    rays = rays_of(o, d)
+    rays["tmax"] = ln  # a ray's end on the surface
+    same(gpu, orc, corners, rays, f"{scene}, rays that end on it")
+
+
+def test_frames_of_layers_are_the_same_in_every_build(gpu, orc):
+    """Two floors in one plane: every build, register fit and repeat gives the
+    same sums, bit for bit, and they are the oracle's."""
+    tris, _ = lit(layers())
+    w, h = 64, 48
+    cam = S.path_camera(w, h, eye=(1.4, -1.9, 1.7), target=(1.5, 1.5, 0.1), rr_from=3)
+    cam["env"] = (0.4, 0.5, 0.6, 0.0)
+    px = np.zeros(P.PX_LEN * w * h + 1, dtype=np.uint32)
+    sc = orc.Scene(tris, 4, P.NODE)
+    for f in range(4):
+        sc.sample(cam, w, h, px, f, nthreads=8)
+    want = P.planes(px, w, h)
+    tr = P.Tracer.new(gpu, tris, 4)
+    first = None
+    for build, waves in [(0, 2), (0, 4), (1, 4), (2, 4), (3, 4), (3, 4), (3, 5), (3, 2)]:
+        tr.set_path_regen(build)
+        tr.set_path_waves(waves)
+        tr.sample(cam, w, h, 4)
+        got = tr.px()
+        tr.sample(S.path_camera(w + 1, h), w + 1, h, 1)  # another view: the next call starts over
+        if first is None:
+            first = got
+            a = P.planes(got, w, h)
+            for k in ("radiance", "albedo", "normal", "depth", "count", "missed"):
+                assert np.allclose(a[k], want[k], rtol=1e-5, atol=0), k  # the tracer's bound against the oracle
+        assert np.array_equal(got, first), (build, waves)
+    b = P.Batch(gpu, np.concatenate([tris, tris]), np.array([0, len(tris), 2 * len(tris)], dtype=np.uint32))
+    for build in (0, 3):
+        b.set_path_build(build)
+        b.render(cam, w, h, 4)
+        for k in range(2):
+            got = P.planes(b.px(k), w, h)
+            assert np.array_equal(got["radiance"], P.planes(first, w, h)["radiance"]), (build, k)
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 7, 8, 9])
