@@ -307,6 +307,13 @@ __device__ __forceinline__ uint32_t wide_root(const SceneDev& s, uint32_t& end) 
     return (w & PHR_LEAF) ? w : s.root;
 }
 
+// Whether the ray meets the root's box before tmax. No record holds it: the
+// records' boxes lie in it, but where the root is a leaf it is the leaf's own,
+// and a ray at a triangle's edge can meet the triangle and not its box.
+__device__ __forceinline__ bool meets_root(const SceneDev& s, V3 o, V3 d, float tmax) {
+    return box_t(s.nodes[2 * (size_t)s.root], s.nodes[2 * (size_t)s.root + 1], o, safe_inv(d), tmax) < PHR_INF;
+}
+
 // A stack of PHR_STACK LDS entries: what a walk a level at a time needs, which
 // pushes one of each level.
 template <uint32_t STRIDE>
@@ -356,6 +363,7 @@ __device__ __forceinline__ PhrHit walk(const SceneDev& s, V3 o, V3 d, float tmax
     PhrHit best{tmax, PHR_NONE, 0.f, 0.f, 0u};
     const WideRay r = wide_ray(o, d);
     uint32_t sp = 0, only, cur = wide_root(s, only);
+    if (only != PHR_NONE && !meets_root(s, o, d, tmax)) return best;
     bool doubt = false;
     for (;;) {
         if (cur & PHR_LEAF) {
@@ -579,12 +587,12 @@ __device__ __forceinline__ void walker_root(Walker& w, uint32_t root) {
     w.cur = leaf ? PHR_NONE : root;
     w.leaf = leaf ? root : PHR_NONE;
 }
-__device__ __forceinline__ void walker_begin(Walker& w, uint32_t root, V3 o, V3 d, float tmax, bool any) {
+__device__ __forceinline__ void walker_begin(Walker& w, const SceneDev& s, uint32_t root, V3 o, V3 d, float tmax, bool any) {
     w.r = wide_ray(o, d);
     w.t = tmax;
     w.u = w.v = 0.f;
     w.any = any;
-    w.on = true;
+    w.on = !(root & PHR_LEAF) || meets_root(s, o, d, tmax);
     w.doubt = w.binary = false;
     walker_root(w, root);
 }
@@ -2143,7 +2151,7 @@ struct SplitWalk {
     Walker w;
     uint32_t root, only;
     __device__ __forceinline__ void scene(const SceneDev& s) { root = wide_root(s, only); }
-    __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, root, o, d, tmax, any); }
+    __device__ __forceinline__ void begin(const SceneDev& s, V3 o, V3 d, float tmax, bool any) { walker_begin(w, s, root, o, d, tmax, any); }
     // The wave's next unit: the lanes at an inner node visit it while they are
     // enough; once LEAF8 eighths of the walks have a leaf put by and nothing
     // to visit, every lane with a leaf put by tests its triangles.
@@ -2646,8 +2654,9 @@ __global__ __launch_bounds__(WF_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
                 r = wide_ray(o, d);
                 sp = 0;
                 cur = root;
-                live = true;
+                live = only == PHR_NONE || meets_root(sc, o, d, tmax);
                 doubt = binary = false;
+                if (!live) finish();
             }
         }
         if (__ballot(live) == 0ull) {

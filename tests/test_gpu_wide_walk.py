@@ -135,6 +135,38 @@ def test_small_scenes(gpu, orc, n):
     same(gpu, orc, corners, rays_of(o, (tgt - o) / np.linalg.norm(tgt - o, axis=1)[:, None]), f"{n} triangles")
 
 
+@pytest.mark.parametrize("n", [1, 2, 4])
+@pytest.mark.parametrize("build", [0, 1, 2, 3], ids=["nested", "regen", "wavefront", "split"])
+def test_a_leaf_for_a_root(gpu, orc, n, build):
+    """One leaf is the whole tree: its box is tested, as the binary walk tests
+    it. Some rays at a triangle's corner meet the triangle and not the box; the
+    view is of a corner, many pixels to a rounding of its coordinates (with one
+    triangle nine pixels have such a ray)."""
+    rng = np.random.default_rng(n)
+    corners = rng.uniform(0.5, 1, (n, 3, 3)).astype(np.float32)
+    if build == 0:
+        to = corners.reshape(-1, 3)[rng.integers(0, 3 * n, 20_000)].astype(np.float64)
+        o = to + rng.uniform(-3, 3, to.shape)
+        d = (to - o) / np.linalg.norm(to - o, axis=1)[:, None]
+        same(gpu, orc, corners, rays_of(o, d), f"{n} triangles")
+    tris, _ = lit(corners)
+    corner = corners[0, 0].astype(np.float64)
+    cam = S.path_camera(40, 24, eye=tuple(corner + [3.0, 0.4, 0.2]), target=tuple(corner), fov_deg=1e-5, rr_from=3)
+    cam["env"] = (0.4, 0.5, 0.6, 0.0)
+    sc = orc.Scene(tris, 4, P.NODE)
+    px = np.zeros(P.PX_LEN * 40 * 24 + 1, dtype=np.uint32)
+    rays = [0, 0]
+    for f in range(8):
+        r = sc.sample(cam, 40, 24, px, f, nthreads=8)
+        rays = [rays[0] + r[0], rays[1] + r[1]]
+    tr = P.Tracer.new(gpu, tris, 4)
+    tr.set_path_regen(build)
+    tr.set_path_waves(4)
+    tr.sample(cam, 40, 24, 8)
+    same_planes(tr.px(), px)
+    assert list(tr.rays()) == rays
+
+
 def test_axis_rays_flat_boxes_and_inside(gpu, orc):
     g = grid(12)
     walls = np.concatenate([g, g[:, :, [2, 0, 1]], g[:, :, [1, 2, 0]]])
