@@ -406,8 +406,9 @@ uint32_t phr_tracer_path_waves(const phr_tracer* t);
  * They serve a camera with lamps or a lit world and no Adaptive Sampling, and
  * 1 and 2 one tree only (3 serves a forest too); other frames take the
  * nested build, and a sliced sample or a recorded frame takes 1 for 2. The
- * autotune tries every build the scene and camera allow. Default: 3 for a
- * forest, 0 for one tree. */
+ * autotune tries every build the scene and camera allow. Default: 0 for one
+ * tree; 3 for a forest, whose frames then take the nested build where the
+ * forest has too few instances for it to pay. */
 int phr_tracer_set_path_regen(phr_tracer* t, uint32_t on);
 uint32_t phr_tracer_path_regen(const phr_tracer* t);
 /* No counterpart in the reference: the split build's shading point. A wave

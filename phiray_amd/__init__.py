@@ -996,7 +996,8 @@ class Tracer:
         path-regenerating one (True, 1), the wavefront one (2) or the split
         one (3: a wave walks until enough of its lanes have finished their walk,
         those shade and start their next walk while the others walk on; the
-        default of a scene of instances). The last three serve a camera with
+        default of a scene of instances, unless they are too few for it to
+        pay). The last three serve a camera with
         lamps or a lit world, no Adaptive Sampling, the second and third one
         tree only; other frames take the nested build."""
         m = int(mode) if not isinstance(mode, bool) else (1 if mode else 0)

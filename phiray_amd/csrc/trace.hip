@@ -3247,6 +3247,7 @@ struct phr_tracer {
     std::vector<uint32_t> order;          // slot -> input face
     uint32_t w = 0, h = 0, frame = 0, samples = 32;
     uint32_t path_waves = 2;  // which k_path variant runs (2 to 5 waves a SIMD)
+    bool build_chosen = false;  // path_regen was set by the caller or the autotune
     uint32_t path_regen = 0;  // 1: the path-regenerating build, 2: the wavefront build, 3: the split build, where the camera allows it
     uint32_t split_shade = 6;  // the split build shades once this many eighths of a wave's working lanes wait
     uint32_t mesh_depth = PHR_STACK;  // a forest: its deepest mesh tree (the 4-wave build needs <= 24)
@@ -3355,6 +3356,29 @@ struct WordsHash {  // FNV-1a over the words
 uint32_t path_build_waves(const phr_tracer* t) {
     if (t->forest && t->path_waves >= 4) return t->mesh_depth <= FOREST_SHORT_STACK ? 4u : 3u;
     return t->path_waves;
+}
+
+// The build a path frame takes. A forest's split build is its default (the
+// caller has set none) where it pays. Nested time over split time, 64 x 64 to
+// 1280 x 720 at 1 to 4 spp (a body is an instance; two more are the ground and
+// the lamp):
+//   bodies   2 waves     3 waves     4 waves
+//   16       0.85-1.20   0.85-1.05   0.81-1.05
+//   20       0.90-1.24   0.85-1.10   1.02-1.16, above 640 x 360 0.87-1.07
+//   24       1.06-1.27   1.01-1.20   1.04-1.21, at 1280 x 720 0.91-0.93
+//   32       1.00-1.33   0.95-1.23   1.00-1.24, above 960 x 540 0.90-0.98
+//   40-64    1.07-1.49   1.07-1.34   1.00-1.30
+// With few instances a wave's lanes have little to part over, and the nested
+// build's fourth wave a SIMD counts where the image has more pixels than four
+// waves a SIMD have lanes.
+uint32_t frame_build(const phr_tracer* t, const PhrCamera& cam, uint32_t w, uint32_t h) {
+    if (!regen_allowed(cam)) return 0u;
+    if (t->forest && !t->build_chosen) {
+        const uint64_t lanes = 64ull * 4 * 4 * (uint32_t)std::max(t->gpu->cu_count, 1);
+        const bool small = (uint64_t)w * h <= lanes, three = t->ninsts >= 24u && path_build_waves(t) <= 3u;
+        if (t->ninsts < 20u || (t->ninsts < 36u && !small && !three)) return 0u;
+    }
+    return t->path_regen;
 }
 
 // Whether the forest's 3-wave build takes the short mesh-tree stack.
@@ -4195,7 +4219,7 @@ int phr_tracer_sample_in(phr_tracer* t, const void* cam_v, uint32_t w, uint32_t 
     slices = std::min(std::max<uint32_t>(slices, 1u), tiles);
     bool abandoned = false;
     // One launch of `count` samples from f0, in `slices` pieces of the tiles.
-    const uint32_t regen = regen_allowed(cam) ? t->path_regen : 0u;
+    const uint32_t regen = frame_build(t, cam, w, h);
     auto path = [&](uint32_t f0, uint32_t count, uint32_t listed) -> int {
         for (uint32_t k = 0; k < slices && !abandoned; ++k) {
             const uint32_t a = (uint32_t)((uint64_t)tiles * k / slices), b = (uint32_t)((uint64_t)tiles * (k + 1) / slices);
@@ -4276,6 +4300,7 @@ uint32_t phr_tracer_path_waves(const phr_tracer* t) { return t ? t->path_waves :
 int phr_tracer_set_path_regen(phr_tracer* t, uint32_t on) {
     PHR_CHECK(t && on <= 3u, PHR_ERR_ARG, "phr_tracer_set_path_regen: null, or not 0, 1, 2 or 3");
     t->path_regen = on;
+    t->build_chosen = true;
     return PHR_OK;
 }
 uint32_t phr_tracer_path_regen(const phr_tracer* t) { return t ? t->path_regen : 0; }
@@ -4313,6 +4338,7 @@ int phr_tracer_autotune(phr_tracer* t, const void* cam, uint32_t w, uint32_t h, 
                         uint32_t* chosen, double* best_s) {
     PHR_CHECK(t && cam, PHR_ERR_ARG, "phr_tracer_autotune: null");
     reps = std::max<uint32_t>(reps, 1);
+    t->build_chosen = true;
     uint32_t best_w = 2, best_r = 0;
     double best = 1e30;
     PhrCamera probe;
@@ -4534,7 +4560,7 @@ int phr_tracer_record_frame(phr_tracer* t, const void* cam_v, uint32_t w, uint32
     uint32_t* pxp = (uint32_t*)t->px->ptr;
     PHR_HIP(hipStreamSynchronize(s));
     PHR_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-    launch_path(t->gpu, path_build_waves(t), t->forest, regen_allowed(cam) ? t->path_regen : 0u, dim3(tiles), s, sc, cp, tiles_x, 0u, spp, pxp,
+    launch_path(t->gpu, path_build_waves(t), t->forest, frame_build(t, cam, w, h), dim3(tiles), s, sc, cp, tiles_x, 0u, spp, pxp,
                 t->rays, 0u, 0u, path_short_stack(t), t->split_shade);
     int rc = PHR_OK;
     if (denoise == 1) rc = phr_denoise_enqueue(t->gpu, pxp, t->w, t->h, 0, t->dn_scratch, t->last.view);
@@ -4939,9 +4965,9 @@ int phr_tracer_from_scene(phr_gpu* g, const phr_scene_desc* d, uint32_t leaf, ph
     phr_tracer* t = new phr_tracer();
     t->gpu = g;
     t->forest = true;
-    // The split build unless the caller chooses another: the same sums, over
-    // 1,024 bodies at 720p 4-spp 32.6 ms nested, 21.9 split (64 bodies 6.5 and
-    // 5.6). It shades at 4 eighths (at 5 22.3, at 3 22.6).
+    // The split build where it pays (frame_build) unless the caller chooses one:
+    // the same sums, over 1,024 bodies at 720p 4-spp 32.6 ms nested, 21.9 split.
+    // It shades at 4 eighths (at 5 22.3, at 3 22.6).
     t->path_regen = 3;
     t->split_shade = 4;
     t->n = d->nfaces;

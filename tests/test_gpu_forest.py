@@ -200,6 +200,25 @@ def test_split_walk_is_the_default_and_matches_the_nested(gpu, ninsts, w, h):
     assert np.array_equal(got[P.Tracer.PATH_SPLIT], got[P.Tracer.PATH_NESTED])  # the same walks in the same order
 
 
+# Instances on both sides of the default build's lines (20, 24, 36), and images
+# on both sides of 262,144 pixels; four waves a SIMD and two.
+@pytest.mark.parametrize("ninsts", [19, 20, 23, 24, 35, 36])
+@pytest.mark.parametrize("w,h,waves", [(48, 33, 4), (1031, 257, 4), (1031, 257, 2)])
+def test_default_build_by_instances_and_pixels(gpu, ninsts, w, h, waves):
+    v, f, m, me, ins = S.bodies_scene(34)[0].arrays()
+    ins = np.concatenate([ins[-2:], ins[:-2]])[:ninsts]  # the ground and the lamp stay
+    t = P.Tracer.from_scene(gpu, v, f, m, me, ins, leaf=4)
+    t.set_samples(64)
+    t.set_path_waves(waves)
+    cam = S.path_camera(w, h, eye=(0.0, -16.0, 9.0), target=(0.0, 0.0, 1.5), rr_from=2)
+    t.sample(cam, w, h, 2)
+    got = t.px()
+    t.set_path_regen(P.Tracer.PATH_NESTED)
+    t.sample(S.path_camera(w + 1, h), w + 1, h, 1)  # another view: the next call starts over
+    t.sample(cam, w, h, 2)
+    assert np.array_equal(got, t.px())
+
+
 def test_reinstance_matches_the_oracle(gpu, orc):
     print("[forest] reinstance", flush=True)
     arrs = forest_scene().arrays()
