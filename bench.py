@@ -226,7 +226,7 @@ def forest_rates(gpu: P.Gpu, substeps: int = 8, w: int = 1280, h: int = 720, spp
             "substep_ms": wall_s / substeps * 1e3, "substep_gpu_span_ms": g_s / substeps * 1e3,
             "frame": f"{w}x{h}, {spp} spp", "frame_ms": t_frame * 1e3, "mrays_s": rays / t_frame / 1e6,
             "rays_per_frame": rays, "path_waves_per_simd": waves, "path_build": PATH_BUILDS[chosen],
-            "frame_ms_by_build": by_build, "mesh_stack_entries": tr.path_stack}
+            "frame_ms_by_build": by_build, "mesh_stack_entries": 32 if chosen == 3 else tr.path_stack}
 
 
 def xpbd_rates(gpu: P.Gpu, frames: int = 120, substeps: int = 8, w: int = 1280, h: int = 720, spp: int = 4) -> dict:

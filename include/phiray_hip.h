@@ -391,7 +391,9 @@ uint32_t phr_tracer_instance_count(const phr_tracer* t);
  * PHR_ERR_UNSUPPORTED when the last camera had it off. */
 int phr_tracer_open_pixels(phr_tracer* t, uint32_t* count);
 /* The path kernel variant (no counterpart in phiray): register allocation
- * fitted to 2 (default), 3, 4 or 5 waves a SIMD. */
+ * fitted to 2 (default), 3, 4 or 5 waves a SIMD. A forest's nested build has
+ * fits for 2 to 4, its split build for 2 and 3; a higher setting takes the
+ * highest. */
 int phr_tracer_set_path_waves(phr_tracer* t, uint32_t waves);
 uint32_t phr_tracer_path_waves(const phr_tracer* t);
 /* The path-regenerating builds (no counterpart in phiray): 1 lets a lane whose
@@ -417,8 +419,9 @@ uint32_t phr_tracer_path_regen(const phr_tracer* t);
 int phr_tracer_set_split_shade(phr_tracer* t, uint32_t eighths);
 uint32_t phr_tracer_split_shade(const phr_tracer* t);
 /* No counterpart in the reference: the mesh-tree stack entries a thread of
- * the path launches holds (24 or 32; the autotune picks the 24-entry stack
- * at 3 waves too when every mesh tree of a forest is at most 24 deep). */
+ * the nested path launches holds (24 or 32; the autotune picks the 24-entry
+ * stack at 3 waves too when every mesh tree of a forest is at most 24 deep).
+ * The split build's threads hold 32 at any setting. */
 int phr_tracer_set_path_stack(phr_tracer* t, uint32_t entries);
 uint32_t phr_tracer_path_stack(const phr_tracer* t);
 /* Autotune (no counterpart in phiray): time each variant on `spp` samples of

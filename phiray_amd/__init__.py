@@ -1019,7 +1019,8 @@ class Tracer:
 
     @property
     def path_stack(self) -> int:
-        """Mesh-tree stack entries a thread of the path launches holds."""
+        """Mesh-tree stack entries a thread of the nested path launches holds
+        (the split build's hold 32)."""
         return int(lib().phr_tracer_path_stack(self._h))
 
     def set_path_stack(self, entries: int) -> None:

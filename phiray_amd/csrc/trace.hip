@@ -2946,10 +2946,11 @@ bool regen_allowed(const PhrCamera& cam) {
     return cam.adapt[3] == 0.0f && (cam.count != 0u || lit);
 }
 
-// regen: 0 the nested build; 3 the split build (k_path_sw, shading at shade8
-// eighths of a wave); else the regenerating build (k_path_rg); the last two
-// for one tree, no list and no Adaptive Sampling or studio rig (the caller
-// checks the camera).
+// regen: 0 the nested build; 3 the split build (k_path_sw, k_path_sw_forest,
+// shading at shade8 eighths of a wave); else, for one tree, the regenerating
+// build (k_path_rg); the last two without a list, Adaptive Sampling or studio
+// rig (the caller checks the camera). A forest's split build is fitted to two
+// or three waves: three serve any higher setting.
 // short_stack: the forest's nested 3-wave build with FOREST_SHORT_STACK
 // mesh-tree entries (the caller checked the mesh trees' depth).
 void launch_path(phr_gpu* g, uint32_t waves, bool forest, uint32_t regen, dim3 grid, hipStream_t s, const SceneDev& sc,
@@ -4058,9 +4059,7 @@ int phr_tracer_warm(phr_gpu* g, uint32_t cap, const char** names, double* ms, ui
         {"k_path_batch_sw<3>", (const void*)k_path_batch_sw<3>}, {"k_path_batch_sw<4>", (const void*)k_path_batch_sw<4>},
         {"k_path_batch_sw<5>", (const void*)k_path_batch_sw<5>}, {"k_path_sw_forest<2>", (const void*)k_path_sw_forest<2>},
         {"k_path_sw_forest<3>", (const void*)k_path_sw_forest<3>},
-        // the settings with the short stack or four waves: one kernel serves the three
-        {"k_path_sw_forest<3, short stack>", (const void*)k_path_sw_forest<3>},
-        {"k_path_sw_forest<4>", (const void*)k_path_sw_forest<3>},
+        {"k_wf_walk", (const void*)k_wf_walk<false>}, {"k_wf_shade", (const void*)k_wf_shade},
     };
     uint32_t n = 0;
     for (const K& k : ks) {
@@ -4292,11 +4291,11 @@ int phr_tracer_set_path_waves(phr_tracer* t, uint32_t waves) {
 }
 uint32_t phr_tracer_path_waves(const phr_tracer* t) { return t ? t->path_waves : 0; }
 
-// The path-regenerating build (1), the wavefront build (2) or neither (0);
-// they run only for one tree and a camera without Adaptive Sampling or the
-// studio rig, the nested build otherwise. A sliced sample (sample_in with
-// several slices) and a recorded frame take the regenerating build for 2
-// (no counterpart in phiray).
+// The nested build (0), the path-regenerating (1), the wavefront (2) or the
+// split one (3); the last three run for a camera without Adaptive Sampling or
+// the studio rig, 1 and 2 for one tree only, the nested build otherwise. A
+// sliced sample (sample_in with several slices) and a recorded frame take the
+// regenerating build for 2 (no counterpart in phiray).
 int phr_tracer_set_path_regen(phr_tracer* t, uint32_t on) {
     PHR_CHECK(t && on <= 3u, PHR_ERR_ARG, "phr_tracer_set_path_regen: null, or not 0, 1, 2 or 3");
     t->path_regen = on;
@@ -4313,8 +4312,9 @@ int phr_tracer_set_split_shade(phr_tracer* t, uint32_t eighths) {
 }
 uint32_t phr_tracer_split_shade(const phr_tracer* t) { return t ? t->split_shade : 0u; }
 
-// The mesh-tree stack entries the path launches take: the 4-wave forest
+// The mesh-tree stack entries the nested path launches take: the 4-wave forest
 // build's 24, the 3-wave build's 24 or 32 as the autotune chose, 32 otherwise.
+// (The split build's hold 32.)
 int phr_tracer_set_path_stack(phr_tracer* t, uint32_t entries) {
     PHR_CHECK(t, PHR_ERR_ARG, "phr_tracer_set_path_stack: null");
     PHR_CHECK(entries == FOREST_SHORT_STACK || entries == PHR_STACK, PHR_ERR_ARG, "phr_tracer_set_path_stack: 24 or 32 entries");
@@ -4355,14 +4355,16 @@ int phr_tracer_autotune(phr_tracer* t, const void* cam, uint32_t w, uint32_t h, 
         builds[nbuilds++] = 3u;
     }
     const bool fits_short = t->forest && t->mesh_depth <= FOREST_SHORT_STACK;
+    // A forest's split build has fits for two and three waves and one stack.
+    auto most_waves = [&](uint32_t build) { return !t->forest ? PATH_WAVES_MAX : (build == 0u && fits_short ? 4u : 3u); };
     bool best_short = false;
     uint32_t best_shade = t->split_shade;
     for (uint32_t bi = 0; bi < nbuilds; ++bi)
         // The wavefront build's kernels have one register fit: timed once,
         // keeping the waves the others chose for its recorded-frame stand-in.
         for (uint32_t regen = builds[bi], waves = regen == 2u ? best_w : PATH_WAVES_MIN;
-             waves <= (regen == 2u ? best_w : (t->forest ? (fits_short ? 4u : 3u) : PATH_WAVES_MAX)); ++waves)
-            for (uint32_t stk = 0; stk < ((fits_short && waves == 3) ? 2u : 1u); ++stk)
+             waves <= (regen == 2u ? best_w : most_waves(regen)); ++waves)
+            for (uint32_t stk = 0; stk < ((fits_short && waves == 3 && regen == 0u) ? 2u : 1u); ++stk)
                 for (uint32_t shade : {4u, 6u}) {  // the split build's shading point; one pass for the others
                     if (regen != 3u && shade != 4u) continue;
                     t->path_waves = waves;

@@ -219,6 +219,21 @@ def test_default_build_by_instances_and_pixels(gpu, ninsts, w, h, waves):
     assert np.array_equal(got, t.px())
 
 
+def test_the_autotune_times_each_split_kernel_once(gpu):
+    """A forest's split build has fits for two and three waves and one stack:
+    the autotune leaves no setting that names another, and warm lists no kernel
+    that is not there."""
+    names = [n for n, _ in P.Tracer.warm(gpu)]
+    assert [n for n in names if n.startswith("k_path_sw_forest")] == ["k_path_sw_forest<2>", "k_path_sw_forest<3>"]
+    v, f, m, me, ins = S.bodies_scene(64)[0].arrays()
+    t = P.Tracer.from_scene(gpu, v, f, m, me, ins, leaf=4)
+    cam = S.path_camera(320, 180, eye=(0.0, -16.0, 9.0), target=(0.0, 0.0, 1.5), rr_from=2)
+    waves, _ = t.autotune(cam, 320, 180, 1, reps=1)
+    assert t.path_waves == waves
+    if t.path_regen == P.Tracer.PATH_SPLIT:
+        assert waves in (2, 3) and t.path_stack == 32
+
+
 def test_reinstance_matches_the_oracle(gpu, orc):
     print("[forest] reinstance", flush=True)
     arrs = forest_scene().arrays()
