@@ -376,7 +376,10 @@ def learned_vs_plain(gpu: P.Gpu, net: "P.Kpcn", seeds, w: int = 1920, h: int = 1
         log(f"learned vs plain, seed {seed}: plain {plain and plain['spp']} spp {plain and plain['s_per_frame']:.4f} s, "
             f"learned {learned['spp']} spp {learned_s:.4f} s relMSE {learned['relmse']:.4f}"
             f"{' (plain fallback)' if res['plain'] else ''}")
-        per.append(row)
+        # The trials and checks go to the log: eight seeds of them made the line
+        # longer than a reader that keeps 10,000 characters of it takes in.
+        log(json.dumps(row))
+        per.append({**{k: v for k, v in row.items() if k != "trials"}, "learned": {k: v for k, v in learned.items() if k != "checks"}})
     ratios = [r["plain_over_learned"] for r in per if "plain_over_learned" in r]
     return {"workload": f"{len(per)} held-out scenes of 65,536 triangles (seeds {int(seeds[0])}..{int(seeds[-1])}), "
                         f"{w}x{h}, white world, reference {ref_spp} spp, bound relMSE 0.01",
@@ -550,6 +553,15 @@ def cpu_baseline(tris: np.ndarray, cam: np.ndarray, w: int, h: int, budget_s: fl
                       f"CPU LBVH build of the scene took {t_scene:.2f} s",
             "s_per_frame_est": dt / (f * count) * (w * h) * 64,
             "lbvh_65536": cpu_lbvh_raycast(cores)}
+
+
+def short(v):
+    """The same with its numbers to six digits (a shorter line)."""
+    if isinstance(v, dict):
+        return {k: short(x) for k, x in v.items()}
+    if isinstance(v, (list, tuple)):
+        return [short(x) for x in v]
+    return float(f"{v:.6g}") if isinstance(v, float) else v
 
 
 def main() -> int:
@@ -726,7 +738,7 @@ def main() -> int:
         if not args.no_cpu:
             log("CPU twin baseline")
             line["cpu_baseline"] = cpu_baseline(tris, cam, w, h, args.cpu_seconds)
-    line.update(out)
+    line.update(short(out))
     if out.get("lbvh_65536"):
         # The 65,536-triangle set (the CPU-runnable configuration) is the
         # headline LBVH figure; the 1.31M scene's beside it.
