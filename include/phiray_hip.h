@@ -292,8 +292,9 @@ int phr_tracer_sample_in(phr_tracer* t, const void* cam, uint32_t w, uint32_t h,
 int phr_tracer_time(phr_tracer* t, double* submit_s, double* gpu_s);
 /* Rays traced so far: closest-hit and shadow (any-hit). */
 int phr_tracer_rays(phr_tracer* t, uint64_t* closest, uint64_t* shadow);
-/* Walk counters: [closest rays, shadow rays, inner-node steps, triangle tests]
- * of the path kernel, then [steps, tests] of the raycasts. */
+/* Walk counters: [closest rays, shadow rays, node visits, triangle tests] of
+ * the path kernel, then [visits, tests] of the raycasts. A visit tests four
+ * boxes of one tree, two of a forest; an any-hit raycast counts levels. */
 int phr_tracer_counters(phr_tracer* t, uint64_t* out6);
 /* The image buffer (src/trace/read.rs:37-56), raw words. */
 int phr_tracer_px(phr_tracer* t, uint64_t from, uint64_t count, uint32_t* out);
@@ -470,7 +471,7 @@ int phr_batch_record(phr_batch* b, const void* cam, uint32_t w, uint32_t h, uint
 int phr_batch_replay(phr_batch* b, double* gpu_s);
 /* Scene k's image words [from, from + count): its own PX_LEN * w * h + 1. */
 int phr_batch_px(phr_batch* b, uint32_t k, uint64_t from, uint64_t count, uint32_t* out);
-/* Since creation: closest rays, shadow rays, inner-node steps, triangle tests. */
+/* Since creation: closest rays, shadow rays, node visits, triangle tests. */
 int phr_batch_counters(phr_batch* b, uint64_t* out4);
 
 /* ---- the learned denoiser (no counterpart in phiray: it stands beside

@@ -1066,7 +1066,7 @@ class Tracer:
         return int(a.value), int(b.value)
 
     def counters(self) -> np.ndarray:
-        """[closest, shadow, steps, tests] of the path kernel, [steps, tests] of raycasts."""
+        """[closest, shadow, node visits, tests] of the path kernel, [visits, tests] of raycasts."""
         out = np.zeros(6, dtype=np.uint64)
         _check(lib().phr_tracer_counters(self._h, _ptr(out)), "Tracer counters")
         return out

@@ -2418,8 +2418,8 @@ __global__ __launch_bounds__(SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(W
 }
 // The split build over a forest. Three waves a SIMD hold whole mesh-tree stacks
 // (12 KB a wave); fitted to four it spills 117 words and takes 29.4 ms where
-// three take 21.9 (1,024 bodies, 720p 4-spp). It is bound by its VALU work (83%
-// busy): 50.6 node visits a ray at 23 of 64 lanes.
+// three take 21.9 (1,024 bodies, 720p 4-spp). It is bound by its walks' reads and
+// by its VALU work (58% busy, 20 of 64 lanes): 50.8 node visits a ray.
 template <int WPE>
 __global__ __launch_bounds__(SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void k_path_sw_forest(
     SceneDev sc, const PhrCamera* __restrict__ camp, uint32_t tiles_x, uint32_t frame0, uint32_t spp, uint32_t* __restrict__ px,
@@ -3488,9 +3488,11 @@ SceneDev scene_dev(phr_tracer* t) {
     return s;
 }
 
-// Rays a wave. Measured on 2,000 to 200,000 triangles, us by 16 / 32 / 64:
-// 64 x 64 rays 126 / 130 / 138 (65,536 triangles), 256 x 256 rays 155 / 154 /
-// 167 and (200,000) 229 / 219 / 245, 512 x 512 rays 401 / 270 / 192.
+// Rays a wave. Measured, us by 16 / 32 / 64, closest and any-hit: 64 x 64 rays
+// on 65,536 triangles 144 / 143 / 155 and 172 / 173 / 186, on 1,024 bodies 341 /
+// 464 / 468 and 230 / 286 / 294; 256 x 256 rays 170 / 163 / 180 and 208 / 205 /
+// 235, bodies 481 / 438 / 498 and 276 / 283 / 342; 512 x 512 rays 416 / 289 / 200
+// and 576 / 396 / 262, bodies 937 / 752 / 617 and 449 / 376 / 373.
 uint32_t raycast_lanes(uint32_t nrays) { return nrays <= 32768u ? 16u : (nrays <= 131072u ? 32u : RAYCAST_THREADS); }
 void launch_raycast(phr_tracer* t, const PhrRay* rays, uint32_t nrays, int any_hit, PhrHit* hits) {
     SceneDev sc = scene_dev(t);
